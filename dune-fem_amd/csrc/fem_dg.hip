@@ -29,6 +29,7 @@
 
 #include "fem_dg.hpp"
 #include "fem_dg_bj.hpp"
+#include "fem_dg_sync.hpp"
 
 namespace femamd {
 
@@ -87,26 +88,6 @@ __device__ __forceinline__ int lidx(int a, int b, int c)
 {
     using S = DGShape<K>;
     return a * S::S1 + b * K + ((K == 4) ? (c ^ a) : c);
-}
-
-// Orders LDS accesses between the lanes of one wavefront.  LDS instructions of
-// a wavefront execute in issue order, so only the compiler must be kept from
-// moving memory operations across this point; no s_barrier and no wait on
-// outstanding global loads is needed.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// the exchange barrier of a workgroup of WG threads: a wavefront fence for
-// one wavefront, the workgroup barrier for more
-template <int WG>
-__device__ __forceinline__ void lds_sync()
-{
-    if constexpr (WG > 64) __syncthreads();
-    else wave_lds_sync();
 }
 
 // Cross-lane moves inside a 16-lane DPP row (one K = 4 element of the FP32
@@ -317,13 +298,10 @@ struct Ctr {
 
 // KQ: kappa given at the quadrature points (FEM_KAPPA_QP); otherwise one
 // value per element (FEM_KAPPA_CELL) or one constant (FEM_KAPPA_CONST).
-// SM: the damped block-Jacobi sweep of a multigrid level in the same pass,
-// xout = u + omega B^-1 (r - A u), instead of w = A u (sm carries r, the
-// element blocks' eigen data, omega and xout; w and dot are not used)
-template <int K, typename T, bool MF, bool KQ, bool SM = false, bool RX = false>
+template <int K, typename T, bool MF, bool KQ, bool RX = false>
 __global__ void __launch_bounds__(ApplyShape<K>::WG)
     k_dg_apply(const DGArgs<T> a, const T *__restrict__ u, T *__restrict__ w, const int *__restrict__ skip,
-               double *__restrict__ dot, const DGSmooth<T> sm)
+               double *__restrict__ dot)
 {
     using S = DGShape<K>;
     constexpr int K2 = S::K2, K3 = S::K3, EPB = ApplyShape<K>::EPB, WG = ApplyShape<K>::WG;
@@ -349,12 +327,11 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
     // values: loaded once as x-pencils, the y- and z-pencils come from LDS
     // (K = 4 only: the other orders keep the face-trace scratch there)
     constexpr bool KLDS = (K == 4) && KQ;
-    // the pointwise/nonlinear reaction is compiled into the plain applies
-    // with constant or cellwise kappa, and into a separate variant (RX) of
-    // the pointwise-kappa apply that only operators with a reaction use (not
-    // into the BF16-MFMA or fused-smoother variants): the pointwise-kappa
-    // kernel without it keeps its code and registers
-    constexpr bool CV = (!KQ && !MF && !SM) || RX;
+    // the pointwise/nonlinear reaction is compiled into the applies with
+    // constant or cellwise kappa (which come here only with a reaction) and
+    // into a separate variant (RX) of the pointwise-kappa apply: the
+    // pointwise-kappa kernel without it keeps its code and registers
+    constexpr bool CV = (!KQ && !MF) || RX;
     constexpr int SZ = F64MF_ ? (KLDS ? 244 : 164) : D35 ? (K == 3 ? 107 : 361) : S::SZ;
     static_assert(!F64MF_ || SZ >= (KLDS ? 3 : 2) * K * S1, "tensors per element");
     static_assert(F64MF_ || SZ >= 2 * K * S1 + 4 * SXQ, "tensors and face-trace scratch per element");
@@ -816,24 +793,7 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
 #pragma unroll
     for (int q = 0; q < K; ++q) v[q] = A[L(i, j, q)];
     C::BT(tb, mr, v, tmp);
-    if constexpr (SM) {
-        // the element's residual pencil d = r - A u, then the exact element
-        // block inverse through the element's LDS slice (K^3 values, then
-        // its eigen data), every lane of the workgroup taking part
-        static_assert(SZ >= K3 + 3 * K2 + 3 * K, "the element's LDS slice holds the block-inverse scratch");
-        const T *re = sm.r + (size_t)e * K3;
-#pragma unroll
-        for (int c = 0; c < K; ++c) tmp[c] = re[i * K2 + j * K + c] - tmp[c];
-        __syncthreads();   // the slice's last reads above are done
-        T *Ab = smem + el * SZ;
-        bj_element<K>(sm.Q + (size_t)e * 3 * K2, sm.lam + (size_t)e * 3 * K, Ab, Ab + K3, i, j, tmp);
-        if (active) {
-            T *xe = sm.xout + (size_t)e * K3;
-#pragma unroll
-            for (int c = 0; c < K; ++c) xe[i * K2 + j * K + c] = ue[i * K2 + j * K + c] + sm.omega * tmp[c];
-        }
-        return;
-    } else if (active) {
+    if (active) {
         T *we = w + (size_t)e * K3;
 #pragma unroll
         for (int c = 0; c < K; ++c) we[i * K2 + j * K + c] = tmp[c];
@@ -869,60 +829,14 @@ static void launch_apply(const DGArgs<T> &a, const T *u, T *w, const int *skip, 
     const int64_t E = (int64_t)a.n[0] * a.n[1] * a.n[2];
     FEM_CHECK(E * S::K3 < (int64_t)1 << 31, FEM_ERR_UNSUPPORTED, "DG apply: more than 2^31 DoFs");
     const unsigned nb = (unsigned)dg_blocks(K, a.n);
-    bool rx = false;
-    if constexpr (!MF) rx = a.cvol || a.nl_pow;
-    if (a.kappa_mode == FEM_KAPPA_QP && rx) {
+    if (a.kappa_mode == FEM_KAPPA_QP && (a.cvol || a.nl_pow)) {
         if constexpr (!MF)
-            hipLaunchKernelGGL((k_dg_apply<K, T, false, true, false, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w,
-                               skip, dot, DGSmooth<T>{});
+            hipLaunchKernelGGL((k_dg_apply<K, T, false, true, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
     } else if (a.kappa_mode == FEM_KAPPA_QP)
-        hipLaunchKernelGGL((k_dg_apply<K, T, MF, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot,
-                           DGSmooth<T>{});
+        hipLaunchKernelGGL((k_dg_apply<K, T, MF, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
     else
-        hipLaunchKernelGGL((k_dg_apply<K, T, MF, false>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot,
-                           DGSmooth<T>{});
+        hipLaunchKernelGGL((k_dg_apply<K, T, MF, false>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
     FEM_HIP(hipGetLastError());
-}
-
-template <int K, typename T>
-static void launch_smooth(const DGArgs<T> &a, const T *u, const DGSmooth<T> &sm, const int *skip, hipStream_t s)
-{
-    using S = DGShape<K>;
-    using A = ApplyShape<K>;
-    const int64_t E = (int64_t)a.n[0] * a.n[1] * a.n[2];
-    FEM_CHECK(E * S::K3 < (int64_t)1 << 31, FEM_ERR_UNSUPPORTED, "DG apply: more than 2^31 DoFs");
-    FEM_CHECK(a.kappa_mode != FEM_KAPPA_QP, FEM_ERR_UNSUPPORTED, "smoothing sweep: cellwise or constant kappa");
-    FEM_CHECK(sm.r && sm.Q && sm.lam && sm.xout && sm.xout != u, FEM_ERR_ARG,
-              "smoothing sweep: r, eigen data and an output other than the input");
-    const unsigned nb = (unsigned)dg_blocks(K, a.n);
-    hipLaunchKernelGGL((k_dg_apply<K, T, false, false, true>), dim3(nb), dim3(A::WG), 0, s, a, u, (T *)nullptr, skip,
-                       (double *)nullptr, sm);
-    FEM_HIP(hipGetLastError());
-}
-
-template <typename T>
-static void dispatch_smooth(const DGArgs<T> &a, int k, const T *u, const DGSmooth<T> &sm, const int *skip,
-                            hipStream_t s)
-{
-    switch (k) {
-    case 2: launch_smooth<2, T>(a, u, sm, skip, s); break;
-    case 3: launch_smooth<3, T>(a, u, sm, skip, s); break;
-    case 4: launch_smooth<4, T>(a, u, sm, skip, s); break;
-    case 5: launch_smooth<5, T>(a, u, sm, skip, s); break;
-    default: throw Error(FEM_ERR_UNSUPPORTED, "DG apply: order must be 1..4");
-    }
-}
-
-void dg_smooth_f64(const DGArgs<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
-                   hipStream_t s)
-{
-    dispatch_smooth<double>(a, k, u, sm, skip, s);
-}
-
-void dg_smooth_f32(const DGArgs<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
-                   hipStream_t s)
-{
-    dispatch_smooth<float>(a, k, u, sm, skip, s);
 }
 
 template <typename T>
@@ -940,13 +854,15 @@ static void dispatch_apply(const DGArgs<T> &a, int k, const T *u, T *w, const in
 void dg_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                   double *dot)
 {
-    dispatch_apply<double>(a, k, u, w, skip, s, dot);
+    if (dg_is_modal(a)) dg_modal_apply_f64(a, k, u, w, skip, s, dot);
+    else dispatch_apply<double>(a, k, u, w, skip, s, dot);
 }
 
 void dg_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                   double *dot)
 {
-    dispatch_apply<float>(a, k, u, w, skip, s, dot);
+    if (dg_is_modal(a)) dg_modal_apply_f32(a, k, u, w, skip, s, dot);
+    else dispatch_apply<float>(a, k, u, w, skip, s, dot);
 }
 
 int dg_apply_epb(int k)
@@ -1405,7 +1321,7 @@ __global__ void __launch_bounds__(64)
     T v[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) v[c] = x[e * K3 + i * K2 + j * K + c];
-    bj_element<K>(Q + e * 3 * K2, lam + e * 3 * K, smem + el * K3, qsm + el * (3 * K2 + 3 * K), i, j, v);
+    bj_element<K>(Q + e * 3 * K2, lam + e * 3 * K, smem + el * K3, qsm + el * (3 * K2 + 3 * K), i, j, wr, v);
     if (active)
 #pragma unroll
         for (int r = 0; r < K; ++r) y[e * K3 + i * K2 + j * K + r] = v[r];

@@ -26,6 +26,25 @@ __host__ __device__ inline unsigned udiv(unsigned x, UDiv v)
     return (unsigned)(((unsigned long long)x * v.m) >> v.sh);
 }
 
+// traversal of the modal kernel: a workgroup holds a tile of ty x tz elements
+// and walks up to lx elements along x; nty x ntz tiles, ncx walks
+struct ModalTile {
+    int ty = 1, tz = 1, lx = 1, nty = 1, ntz = 1, ncx = 1;
+    int slots = 1;                  // elements of a tile and behind its edges
+    int ks = 3;                     // coefficients kept per slot
+    int64_t blocks = 0;
+    UDiv dv_ty, dv_nty, dv_plane;   // by ty, nty, nty ntz
+};
+ModalTile dg_modal_tile(int k, const int *n);
+// traversal by rows: nxg groups of elements per x-row, four rows per
+// workgroup, slabs of ty workgroups in y (about 16 rows), each through all z
+struct ModalRows {
+    int nxg = 1, ty = 1;
+    int64_t blocks = 0;
+    UDiv dv_slab, dv_zrow, dv_nxg;   // by nxg ty nz, nxg ty, nxg
+};
+ModalRows dg_modal_rows(int k, const int *n);
+
 template <typename T>
 struct DGArgs {
     int n[3];
@@ -58,6 +77,11 @@ struct DGArgs {
     // ty y-rows through all z; `slabs` = 0 selects plain element order
     int slabs, rpb, ty;
     UDiv dv_slab, dv_zrow, dv_rpb;   // by rpb ty nz, rpb ty, rpb
+    // of the modal kernel: 2 |K| / h^2, 2 |F| b, |F| beta / (2 h), |F| / (2 h),
+    // |F| max(b, 0), |F| max(-b, 0) per direction, and c |K|
+    T m_kv[3], m_ad[3], m_pen[3], m_w[3], m_bp[3], m_bm[3], m_c;
+    ModalRows mr;
+    ModalTile mt;   // traversal of the modal kernel (fem_dg_modal.hip)
 };
 
 // the damped block-Jacobi sweep fused into the apply (multigrid smoothing):
@@ -90,6 +114,9 @@ inline void dg_derived(DGArgs<T> &a, int k)
         a.dv_zrow = make_udiv((unsigned)(a.rpb * a.ty));
         a.dv_rpb = make_udiv((unsigned)a.rpb);
     }
+    a.mt = dg_modal_tile(k, a.n);
+    a.mr = dg_modal_rows(k, a.n);
+    a.m_c = a.c * a.h[0] * a.h[1] * a.h[2];
     for (int d = 0; d < 3; ++d) {
         const int t1 = (d == 0) ? 1 : 0, t2 = (d == 2) ? 1 : 2;
         a.pen[d] = a.beta * a.ih[d];
@@ -98,7 +125,31 @@ inline void dg_derived(DGArgs<T> &a, int k)
         a.bh[d] = a.b[d] * a.h[d];
         a.bpos[d] = a.b[d] > T(0) ? a.b[d] : T(0);
         a.bneg[d] = a.b[d] < T(0) ? -a.b[d] : T(0);
+        a.m_kv[d] = T(2) * a.vsc[d];
+        a.m_ad[d] = T(2) * a.farea[d] * a.b[d];
+        a.m_pen[d] = T(0.5) * a.farea[d] * a.pen[d];
+        a.m_w[d] = T(0.5) * a.farea[d] * a.ih[d];
+        a.m_bp[d] = a.farea[d] * a.bpos[d];
+        a.m_bm[d] = a.farea[d] * a.bneg[d];
     }
+}
+
+// the modal kernel (fem_dg_modal.hip): kappa constant per element and no
+// reaction beyond c.  The apply, and the damped block-Jacobi sweep of
+// dg_smooth_*; `dot` as in dg_apply_*, dg_modal_blocks(k, n) entries
+int64_t dg_modal_blocks(int k, const int *n);
+void dg_modal_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
+                        double *dot);
+void dg_modal_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
+                        double *dot);
+void dg_modal_smooth_f64(const DGArgs<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
+                         hipStream_t s);
+void dg_modal_smooth_f32(const DGArgs<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
+                         hipStream_t s);
+template <typename T>
+inline bool dg_is_modal(const DGArgs<T> &a)
+{
+    return a.kappa_mode != FEM_KAPPA_QP && !a.cvol && !a.nl_pow;
 }
 
 // w = A u.  `skip` (device flag, may be null): when *skip != 0 the launch
@@ -109,12 +160,6 @@ void dg_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, co
                   double *dot = nullptr);
 void dg_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                   double *dot = nullptr);
-// the sweep xout = u + omega B^-1 (r - A u) in one pass (cellwise or
-// constant kappa; xout must not alias u, whose neighbours the pass reads)
-void dg_smooth_f64(const DGArgs<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
-                   hipStream_t s);
-void dg_smooth_f32(const DGArgs<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
-                   hipStream_t s);
 // BF16 MFMA contraction variant (FP32 data and accumulation)
 void dg_apply_bf16(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s);
 // workgroups of the DG apply launch for order k-1 on n[0] x n[1] x n[2]

@@ -519,7 +519,7 @@ void Learned::init(Operator *o, CNN *c, int steps, int smoother_kind)
     counter.alloc(sizeof(unsigned));
     FEM_HIP(hipMemset(counter.p, 0, sizeof(unsigned)));
     // the FP64 and FP32 DG applies can write per-workgroup <z1, A z1> partials
-    if (o->desc.precision != FEM_BF16MFMA) dparts.alloc(sizeof(double) * o->dot_blocks());
+    if (o->desc.precision != FEM_BF16MFMA) dparts.alloc(sizeof(double) * o->dot_blocks_max());
 }
 
 template <typename T>

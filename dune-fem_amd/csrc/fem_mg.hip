@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(64)
     T v[K];
 #pragma unroll
     for (int c = 0; c < K; ++c) v[c] = mode ? r[base + c] - t[base + c] : r[base + c];
-    bj_element<K>(Q + e * 3 * K2, lam + e * 3 * K, smem + el * K3, qsm + el * (3 * K2 + 3 * K), i, j, v);
+    bj_element<K>(Q + e * 3 * K2, lam + e * 3 * K, smem + el * K3, qsm + el * (3 * K2 + 3 * K), i, j, wr, v);
     if (active)
 #pragma unroll
         for (int c = 0; c < K; ++c) x[base + c] = mode ? x[base + c] + omega * v[c] : omega * v[c];
@@ -956,8 +956,8 @@ static void mg_sweep(const MGDGLevel &L, const T *r, const T *in, T *out, T *t, 
     sm.lam = L.bj.lam.as<T>();
     sm.omega = omega;
     sm.xout = out;
-    if constexpr (std::is_same<T, double>::value) dg_smooth_f64(o.a64, o.k, in, sm, skip, s);
-    else dg_smooth_f32(o.a32, o.k, in, sm, skip, s);
+    if constexpr (std::is_same<T, double>::value) dg_modal_smooth_f64(o.a64, o.k, in, sm, skip, s);
+    else dg_modal_smooth_f32(o.a32, o.k, in, sm, skip, s);
 }
 
 template <typename T>

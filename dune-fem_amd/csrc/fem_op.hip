@@ -2,6 +2,7 @@
 // dispatch to the DG / CG kernels.
 #include <dlfcn.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "fem_blas.hpp"
@@ -443,7 +444,13 @@ void Operator::constrain(Vec &x, const Vec *add) const
 
 int64_t Operator::dot_blocks() const
 {
-    return is_dg() ? dg_blocks(k, desc.n) : 0;
+    if (!is_dg()) return 0;
+    return dg_is_modal(a64) ? dg_modal_blocks(k, desc.n) : dg_blocks(k, desc.n);
+}
+
+int64_t Operator::dot_blocks_max() const
+{
+    return is_dg() ? std::max(dg_modal_blocks(k, desc.n), dg_blocks(k, desc.n)) : 0;
 }
 
 void Operator::apply_raw(const void *x, void *y, const int *skip, double *dot) const

@@ -107,6 +107,9 @@ struct Operator {
     // dot_blocks() entries
     void apply_raw(const void *x, void *y, const int *skip, double *dot = nullptr) const;
     int64_t dot_blocks() const;
+    // the most dot_blocks() can become with other coefficient data (a
+    // pointwise reaction set or cleared)
+    int64_t dot_blocks_max() const;
     void apply(const Vec &x, Vec &y, const int *skip = nullptr) const;
     void rhs(const double *fq_host, Vec &F) const;
     void diagonal(Vec &d) const;  // FP64 or FP32 output

@@ -1,0 +1,85 @@
+"""The modal apply and sweep (kappa constant per element): parity with the
+oracle where tiles, walks and rows end unevenly.
+
+Bar: as in test_gpu_apply.py, 1e-12 (FP64) and 2e-5 (FP32) of max |w|: both
+sides sum about 10 K^2 terms per value, whose rounding stays below K^2 10 eps =
+6e-14 and 3e-5 / 2 of the largest term at K = 5.
+"""
+import numpy as np
+import pytest
+
+import dunefem_amd as fa
+import pyoracle as ora
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.abs(a - b).max() / np.abs(b).max()
+
+
+def operator(ctx, n, p, b, c, kappa, prec=fa.F64):
+    cell = not np.isscalar(kappa)
+    op = fa.GalerkinOperator(ctx, fa.OP_DG_SIPG_3D, n, p, 10.0 * p * p, b, c, fa.KAPPA_CELL if cell else fa.KAPPA_CONST,
+                             1.0 if cell else kappa, precision=prec)
+    if cell:
+        op.set_kappa_cell(kappa)
+    return op
+
+
+@pytest.mark.parametrize("n,p,b,c,kind", [
+    # one element, and one element thick in each direction
+    ((1, 1, 1), 2, (1, -.5, .25), 0.3, "cell"),
+    ((9, 1, 1), 3, (1, -.5, .25), 0.0, "cell"),
+    ((1, 9, 1), 4, (0, 0, 0), 0.0, "cell"),
+    ((1, 1, 9), 4, (-1, .5, .25), 0.2, "const"),
+    ((1, 7, 6), 1, (1, .5, .25), 0.0, "cell"),
+    # tiles and rows with a remainder in both directions
+    ((6, 17, 5), 1, (1, -.5, .25), 0.0, "cell"),
+    ((5, 9, 13), 2, (0, 0, 0), 0.4, "cell"),
+    ((4, 7, 11), 3, (-1, .5, -.25), 0.0, "cell"),
+    ((3, 5, 7), 4, (1, .5, .25), 0.0, "cell"),
+    # walks of two steps, the last of them shorter
+    ((41, 40, 60), 2, (1, .5, .25), 0.0, "cell"),
+    ((41, 33, 33), 3, (0, 0, 0), 0.0, "cell"),
+    ((41, 21, 33), 4, (1, -.5, .25), 0.1, "cell"),
+])
+def test_modal_apply_matches_oracle(ctx, n, p, b, c, kind):
+    rng = np.random.default_rng(sum(n) + p)
+    kappa = np.exp(rng.normal(size=n[0] * n[1] * n[2])) if kind == "cell" else 1.3
+    oop = ora.DGOperator(n, p, 10.0 * p * p, b, c, kappa=("cell", kappa) if kind == "cell" else kappa)
+    u = rng.normal(size=oop.N)
+    ref = oop.apply(u)
+    for prec, tol in ((fa.F64, 1e-12), (fa.F32, 2e-5)):
+        op = operator(ctx, n, p, b, c, kappa, prec)
+        U, W = op.vector(u), op.vector()
+        W.fill(np.nan)
+        op(U, W)
+        err = rel(W.download(), ref)
+        print("modal", n, p, kind, prec, err, flush=True)
+        assert err < tol
+
+
+@pytest.mark.parametrize("n,p", [((7, 5, 6), 1), ((9, 6, 5), 2), ((5, 7, 4), 3), ((7, 6, 5), 4)])
+def test_sweep_equals_apply_and_block_inverse(ctx, n, p):
+    """One V-cycle smooths with fused sweeps; the block inverse of the oracle's
+    element blocks gives the same Krylov solve, and two V-cycles agree bit for
+    bit (a sweep's workgroups exchange data through LDS)."""
+    rng = np.random.default_rng(5 + p)
+    op = operator(ctx, n, p, (0, 0, 0), 0.0, np.exp(rng.normal(size=n[0] * n[1] * n[2])))
+    mg = fa.Preconditioner(op, fa.PRE_MULTIGRID)
+    R = op.vector(rng.normal(size=op.N))
+    Z = [op.vector(), op.vector()]
+    for z in Z:
+        mg(R, z)
+    assert np.array_equal(Z[0].download(), Z[1].download())
+    F = op.vector(rng.normal(size=op.N))
+    X = [op.vector(), op.vector()]
+    for x, pre in zip(X, (mg, fa.Preconditioner(op, fa.PRE_BLOCK_JACOBI))):
+        inv = fa.InverseOperator(ctx, method=fa.CG, tolerance=1e-11, errormeasure=fa.RELATIVE, maxiterations=5000)
+        inv.bind(op, pre)
+        inv(F, x)
+        assert inv.info()["converged"]
+    # both stop at 1e-11 of |F|; the operator's smallest eigenvalue bounds the
+    # distance of the two solutions by 2e-11 times its condition, about 1e4
+    assert rel(X[0].download(), X[1].download()) < 1e-6
