@@ -28,6 +28,8 @@
 namespace femamd {
 
 constexpr int GRP = 8;   // vectors per register group in the multi-dot
+// partials of a square sum at most (after the multi-dot's in the workspace)
+constexpr int NORM_PARTS = 1024;
 // the CG reductions use RED_DOT_BLOCKS partial slots per quantity (two)
 static_assert(2 * RED_DOT_BLOCKS <= RED_BLOCKS * (GM_MAX + 1), "solver partials buffer");
 
@@ -211,10 +213,35 @@ __global__ void __launch_bounds__(RED_THREADS)
 }
 
 // ---- GMRES kernels --------------------------------------------------------------
+// A reduction leaves one partial per workgroup, and the kernel that needs the
+// result sums the partials itself, each workgroup all of them in the same
+// order: a kernel boundary orders the two, where a finish by the last
+// workgroup to arrive waits for a chain of atomics (at 69 k DoFs, restart 30:
+// multi-dot 37 us and orthogonalisation 15 us with that finish on 512
+// workgroups, 7.6 and 7.4 us so).  The grids grow with the vector, so that few
+// partials are left where the sums are short.
+
+// the sum of n partials, in every thread, for every workgroup alike: thread t
+// takes t, t + 256, ..., then a tree over the workgroup
+__device__ __forceinline__ double sum_parts(const double *__restrict__ part, int n, double *lds)
+{
+    double v = 0;
+    for (int k = threadIdx.x; k < n; k += RED_THREADS) v += part[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = 0;
+#pragma unroll
+    for (int w = 0; w < RED_THREADS / 64; ++w) s += lds[w];
+    return s;
+}
+
+// v0 -= b (v0 = A x on entry), partials of ||v0||^2
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
-    k_gm_start(T *__restrict__ v0, const T *__restrict__ b, int64_t n, KState *st, double *partials,
-               unsigned *counter, int first)
+    k_gm_start(T *__restrict__ v0, const T *__restrict__ b, int64_t n, double *__restrict__ part)
 {
     __shared__ double lds[RED_THREADS / 64];
     double acc = 0;
@@ -223,111 +250,62 @@ __global__ void __launch_bounds__(RED_THREADS)
         v0[i] = v;
         acc += (double)v * (double)v;
     }
-    double bs = block_sum(acc, lds);
-    __shared__ bool amLast;
-    if (threadIdx.x == 0) {
-        publish_partial(&partials[blockIdx.x], bs);
-        amLast = atomicAdd(counter, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!amLast) return;
-    double v = 0;
-    for (unsigned k = threadIdx.x; k < gridDim.x; k += blockDim.x) v += read_partial(&partials[k]);
-    double tot = block_sum(v, lds);
-    if (threadIdx.x == 0) {
-        const double res = sqrt(tot);
-        if (first && st->criteria == FEM_ERRMEASURE_REDUCTION) st->gtol *= res;
-        st->res = res;
-        st->jlast = 0;
-        if (res <= st->gtol * (1 + 1e-15)) {
-            st->converged = 1;
-            st->cycle_done = 1;
-        } else {
-            st->converged = 0;
-            st->cycle_done = st->it >= st->maxit ? 1 : 0;
-            st->g[0] = -res;
-            for (int i = 1; i <= GM_MAX; ++i) st->g[i] = 0.0;
-            st->hinv = 1.0 / res;
-        }
-        reset_counter(counter);
-    }
+    const double bs = block_sum(acc, lds);
+    if (threadIdx.x == 0) part[blockIdx.x] = bs;
 }
 
-template <typename T>
-__global__ void k_gm_scale(T *__restrict__ v, int64_t n, const KState *__restrict__ st)
-{
-    if (st->cycle_done) return;
-    const double a = st->hinv;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        v[i] = (T)((double)v[i] * a);
-}
-
-// H[l][j] = <v_l, w>, l = 0..j  (j+1 dots, w read once per group of GRP)
+// partials of <v_l, w>, l = 0..j: workgroup (s, q) takes slice s of the
+// vectors and the GRP basis vectors from q GRP on, into mpart[l * slices + s]
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
-    k_gm_multidot(const T *__restrict__ V, const T *__restrict__ w, int64_t n, int j, KState *st, double *partials,
-                  unsigned *counter, int m)
+    k_gm_multidot(const T *__restrict__ V, const T *__restrict__ w, int64_t n, int j, const KState *__restrict__ st,
+                  double *__restrict__ mpart)
 {
     if (st->cycle_done) return;
-    __shared__ double lds[RED_THREADS / 64];
-    const int cnt = j + 1;
-    // contiguous slice per block
+    __shared__ double lds[GRP][RED_THREADS / 64];
+    const int g0 = blockIdx.y * GRP, cnt = j + 1 - g0 < GRP ? j + 1 - g0 : GRP;
     const int64_t lo = n * blockIdx.x / gridDim.x, hi = n * (blockIdx.x + 1) / gridDim.x;
-    for (int g0 = 0; g0 < cnt; g0 += GRP) {
-        double acc[GRP];
+    double acc[GRP];
 #pragma unroll
-        for (int l = 0; l < GRP; ++l) acc[l] = 0;
-        // four elements per thread and step, so that 4 (GRP + 1) loads are in
-        // flight per thread (the grid has only two waves per SIMD)
-        int64_t i = lo + threadIdx.x;
-        for (; i + 3 * (int64_t)blockDim.x < hi; i += 4 * (int64_t)blockDim.x) {
-            double wi[4];
+    for (int l = 0; l < GRP; ++l) acc[l] = 0;
+    const T *V0 = V + (int64_t)g0 * n;
+    // four elements per thread and step, so that 4 (GRP + 1) loads are in
+    // flight per thread
+    int64_t i = lo + threadIdx.x;
+    for (; i + 3 * (int64_t)RED_THREADS < hi; i += 4 * (int64_t)RED_THREADS) {
+        double wi[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) wi[u] = (double)w[i + u * blockDim.x];
+        for (int u = 0; u < 4; ++u) wi[u] = (double)w[i + u * RED_THREADS];
 #pragma unroll
-            for (int l = 0; l < GRP; ++l)
-                if (g0 + l < cnt) {
-                    const T *vl = V + (int64_t)(g0 + l) * n + i;
-                    double t = 0;
+        for (int l = 0; l < GRP; ++l)
+            if (l < cnt) {
+                const T *vl = V0 + (int64_t)l * n + i;
+                double t = 0;
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) t = fma((double)vl[u * blockDim.x], wi[u], t);
-                    acc[l] += t;
-                }
-        }
-        for (; i < hi; i += blockDim.x) {
-            const double wi = (double)w[i];
-#pragma unroll
-            for (int l = 0; l < GRP; ++l)
-                if (g0 + l < cnt) acc[l] += (double)V[(int64_t)(g0 + l) * n + i] * wi;
-        }
-#pragma unroll
-        for (int l = 0; l < GRP; ++l) {
-            if (g0 + l < cnt) {
-                double b = block_sum(acc[l], lds);
-                if (threadIdx.x == 0) publish_partial(&partials[(size_t)(g0 + l) * gridDim.x + blockIdx.x], b);
-                __syncthreads();
+                for (int u = 0; u < 4; ++u) t = fma((double)vl[u * RED_THREADS], wi[u], t);
+                acc[l] += t;
             }
-        }
     }
-    __shared__ bool amLast;
-    if (threadIdx.x == 0) {
-        amLast = atomicAdd(counter, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!amLast) return;
-    // one wavefront per dot: lane k sums blocks k, k + 64, ... (independent
-    // reads in flight), then a butterfly over the wavefront; the dots are
-    // spread over the block's wavefronts, so they finish concurrently
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    for (int l = wave; l < cnt; l += nw) {
-        double v = 0;
-        for (unsigned k = lane; k < gridDim.x; k += 64) v += read_partial(&partials[(size_t)l * gridDim.x + k]);
+    for (; i < hi; i += RED_THREADS) {
+        const double wi = (double)w[i];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (lane == 0) st->H[l * m + j] = v;
+        for (int l = 0; l < GRP; ++l)
+            if (l < cnt) acc[l] += (double)V0[(int64_t)l * n + i] * wi;
+    }
+#pragma unroll
+    for (int l = 0; l < GRP; ++l) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) acc[l] += __shfl_xor(acc[l], off, 64);
+        if ((threadIdx.x & 63) == 0) lds[l][threadIdx.x >> 6] = acc[l];
     }
     __syncthreads();
-    if (threadIdx.x == 0) reset_counter(counter);
+    const int l = threadIdx.x;
+    if (l < cnt) {
+        double t = 0;
+#pragma unroll
+        for (int k = 0; k < RED_THREADS / 64; ++k) t += lds[l][k];
+        mpart[(size_t)(g0 + l) * gridDim.x + blockIdx.x] = t;
+    }
 }
 
 __device__ __forceinline__ void rot(double &x, double &y, double c, double s)
@@ -337,72 +315,142 @@ __device__ __forceinline__ void rot(double &x, double &y, double c, double s)
     y = c * b - s * a;
 }
 
-// w -= sum_l H[l][j] v_l ; ||w||^2 -> H[j+1][j], Givens rotation, convergence
+// w -= sum_l h_l v_l with h_l from the multi-dot's partials (kept as column j
+// of H), partials of ||w||^2
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
-    k_gm_orth(const T *__restrict__ V, T *__restrict__ w, int64_t n, int j, KState *st, double *partials,
-              unsigned *counter, int m)
+    k_gm_orth(const T *__restrict__ V, T *__restrict__ w, int64_t n, int j, KState *__restrict__ st,
+              const double *__restrict__ mpart, int slices, double *__restrict__ part, int m)
 {
     if (st->cycle_done) return;
     __shared__ double lds[RED_THREADS / 64];
     __shared__ double h[GM_MAX + 1];
-    for (int l = threadIdx.x; l <= j; l += blockDim.x) h[l] = st->H[l * m + j];
+    {
+        // one wavefront per dot
+        const int lane = threadIdx.x & 63;
+        for (int l = threadIdx.x >> 6; l <= j; l += RED_THREADS / 64) {
+            double v = 0;
+            for (int k = lane; k < slices; k += 64) v += mpart[(size_t)l * slices + k];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            if (lane == 0) {
+                h[l] = v;
+                if (blockIdx.x == 0) st->H[l * m + j] = v;
+            }
+        }
+    }
     __syncthreads();
     double acc = 0;
-    const int64_t lo = n * blockIdx.x / gridDim.x, hi = n * (blockIdx.x + 1) / gridDim.x;
-    for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
+    // a quarter of a slice of the multi-dot, by the workgroup whose number
+    // equals the slice's modulo 8: the same XCD (see there)
+    const int sl = blockIdx.x % slices, sub = 4 * sl + blockIdx.x / slices;
+    const int64_t lo = n * sub / (4 * slices), hi = n * (sub + 1) / (4 * slices);
+    for (int64_t i = lo + threadIdx.x; i < hi; i += RED_THREADS) {
         double v = (double)w[i];
         // unrolled so that several basis-vector loads are in flight
-#pragma unroll 8
+#pragma unroll 16
         for (int l = 0; l <= j; ++l) v -= h[l] * (double)V[(int64_t)l * n + i];
         const T vt = (T)v;
         w[i] = vt;
         acc += (double)vt * (double)vt;
     }
-    double bs = block_sum(acc, lds);
-    __shared__ bool amLast;
-    if (threadIdx.x == 0) {
-        publish_partial(&partials[blockIdx.x], bs);
-        amLast = atomicAdd(counter, 1u) == gridDim.x - 1;
+    const double bs = block_sum(acc, lds);
+    if (threadIdx.x == 0) part[blockIdx.x] = bs;
+}
+
+// v /= ||v|| from the partials of its square sum; the first workgroup also
+// keeps the scalars.  j >= 0: column j of H is finished (subdiagonal, Givens
+// rotations, residual estimate, convergence); j < 0: a cycle begins with the
+// residual v (j = -1 the first of a solve, -2 a later one).  z (may be null):
+// the Jacobi preconditioner's z = dinv v in the same pass
+template <typename T>
+__global__ void __launch_bounds__(RED_THREADS)
+    k_gm_scale(T *__restrict__ v, int64_t n, int j, KState *__restrict__ st, const double *__restrict__ part,
+               int nparts, int m, const T *__restrict__ dinv, T *__restrict__ z)
+{
+    // (a workgroup that sees the first one's flag of this very step skips the
+    // scaling of a vector that nothing reads any more)
+    if (j >= 0 && st->cycle_done) return;
+    __shared__ double lds[RED_THREADS / 64];
+    __shared__ double col[GM_MAX + 1], cs[GM_MAX], sn[GM_MAX];
+    const bool keeper = blockIdx.x == 0;
+    if (keeper && j >= 0)
+        for (int i = threadIdx.x; i <= j; i += RED_THREADS) {
+            col[i] = st->H[i * m + j];
+            if (i < j) {
+                cs[i] = st->cs[i];
+                sn[i] = st->sn[i];
+            }
+        }
+    const double nrm = sqrt(sum_parts(part, nparts, lds));
+    if (nrm > 0) {
+        const double a = 1.0 / nrm;
+        for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+            const T t = (T)((double)v[i] * a);
+            v[i] = t;
+            if (z) z[i] = dinv[i] * t;
+        }
     }
-    __syncthreads();
-    if (!amLast) return;
-    double v = 0;
-    for (unsigned k = threadIdx.x; k < gridDim.x; k += blockDim.x) v += read_partial(&partials[k]);
-    double tot = block_sum(v, lds);
-    if (threadIdx.x == 0) {
-        double *H = st->H;
-        const double hn = sqrt(tot);
-        H[(j + 1) * m + j] = hn;
-        st->hinv = 1.0 / hn;
-        for (int i = 0; i < j; ++i) rot(H[(i + 1) * m + j], H[i * m + j], st->cs[i], st->sn[i]);
-        const double a = H[j * m + j], b = H[(j + 1) * m + j];
-        const double nrm = sqrt(a * a + b * b);
-        st->cs[j] = a / nrm;
-        st->sn[j] = -b / nrm;
-        rot(H[(j + 1) * m + j], H[j * m + j], st->cs[j], st->sn[j]);
-        rot(st->g[j + 1], st->g[j], st->cs[j], st->sn[j]);
-        st->it += 1;
-        st->jlast = j + 1;
-        if (fabs(st->g[j + 1]) < st->gtol) {
+    if (!keeper || threadIdx.x != 0) return;
+    if (j < 0) {
+        if (j == -1 && st->criteria == FEM_ERRMEASURE_REDUCTION) st->gtol *= nrm;
+        st->res = nrm;
+        st->jlast = 0;
+        st->gres = nrm;
+        if (nrm <= st->gtol * (1 + 1e-15)) {
             st->converged = 1;
             st->cycle_done = 1;
-        } else if (st->it >= st->maxit || j + 1 == m) {
-            st->cycle_done = 1;
+        } else {
+            st->converged = 0;
+            st->cycle_done = st->it >= st->maxit ? 1 : 0;
+            st->g[0] = -nrm;
         }
-        reset_counter(counter);
+        return;
+    }
+    double x = col[0];   // H[i][j] while the rotations pass down the column
+    for (int i = 0; i < j; ++i) {
+        double below = col[i + 1];
+        rot(below, x, cs[i], sn[i]);
+        st->H[i * m + j] = x;
+        x = below;
+    }
+    const double a = x, b = nrm;
+    const double r = sqrt(a * a + b * b);
+    const double c = a / r, s = -b / r;
+    st->cs[j] = c;
+    st->sn[j] = s;
+    double low = b, top = a;
+    rot(low, top, c, s);
+    st->H[j * m + j] = top;
+    double gl = 0.0, gt = st->g[j];
+    rot(gl, gt, c, s);
+    st->g[j] = gt;
+    st->g[j + 1] = gl;
+    st->gres = fabs(gl);
+    st->it += 1;
+    st->jlast = j + 1;
+    if (fabs(gl) < st->gtol) {
+        st->converged = 1;
+        st->cycle_done = 1;
+    } else if (st->it >= st->maxit || j + 1 == m) {
+        st->cycle_done = 1;
     }
 }
 
-__global__ void k_gm_backsolve(KState *st, int m)
+// H y = g, back substitution by one wavefront, lane i holding row i
+__global__ void __launch_bounds__(64) k_gm_backsolve(KState *st, int m)
 {
-    const int last = st->jlast;
-    const double *H = st->H;
-    for (int i = last - 1; i >= 0; --i) {
-        double s = 0;
-        for (int k = i + 1; k < last; ++k) s += H[i * m + k] * st->y[k];
-        st->y[i] = (st->g[i] - s) / H[i * m + i];
+    __shared__ double H[GM_MAX * GM_MAX];
+    const int last = st->jlast, i = threadIdx.x;
+    for (int k = i; k < last * last; k += 64) H[k] = st->H[(k / last) * m + k % last];
+    double s = i < last ? st->g[i] : 0.0, y = 0.0;
+    __syncthreads();
+    for (int c = last - 1; c >= 0; --c) {
+        const double yc = __shfl(s, c, 64) / H[c * last + c];
+        if (i == c) y = yc;
+        if (i < c) s -= H[i * last + c] * yc;
     }
+    if (i < last) st->y[i] = y;
 }
 
 // u = beta_u * u + sum_{i<last} y_i Z_i
@@ -579,7 +627,7 @@ void Solver::init(Context *c, const fem_solver_params &p)
     FEM_CHECK(p.method >= FEM_SOLVER_CG && p.method <= FEM_SOLVER_BICGSTAB, FEM_ERR_ARG, "solver method");
     FEM_CHECK(p.restart >= 1 && p.restart <= GM_MAX, FEM_ERR_ARG, "gmres restart must be in 1..64");
     state.alloc(sizeof(KState));
-    partials.alloc(sizeof(double) * RED_BLOCKS * (GM_MAX + 2));
+    partials.alloc(sizeof(double) * (RED_BLOCKS * (GM_MAX + 2) + NORM_PARTS));
     counters.alloc(sizeof(unsigned) * 8);
     FEM_HIP(hipMemset(counters.p, 0, counters.bytes));
     FEM_HIP(hipHostMalloc((void **)&hstate, sizeof(KState), hipHostMallocDefault));
@@ -673,7 +721,7 @@ void *Solver::workbuf(int i, size_t bytes)
 
 void Solver::fetch_state()
 {
-    FEM_HIP(hipMemcpyAsync(hstate, state.p, sizeof(KState), hipMemcpyDeviceToHost, ctx->stream));
+    FEM_HIP(hipMemcpyAsync(hstate, state.p, KSTATE_HEAD, hipMemcpyDeviceToHost, ctx->stream));
     FEM_HIP(hipStreamSynchronize(ctx->stream));
 }
 
@@ -846,38 +894,51 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
         bnorm = std::sqrt(hb);
     }
     {
-        KState init;
-        std::memset(&init, 0, sizeof(init));
-        init.gtol = criteria == FEM_ERRMEASURE_RELATIVE ? eps * bnorm : eps;
-        init.criteria = criteria;
-        init.maxit = maxit;
-        *S.hstate = init;
-        FEM_HIP(hipMemcpyAsync(st, S.hstate, sizeof(KState), hipMemcpyHostToDevice, s));
+        std::memset(S.hstate, 0, KSTATE_HEAD);
+        S.hstate->gtol = criteria == FEM_ERRMEASURE_RELATIVE ? eps * bnorm : eps;
+        S.hstate->criteria = criteria;
+        S.hstate->maxit = maxit;
+        FEM_HIP(hipMemcpyAsync(st, S.hstate, KSTATE_HEAD, hipMemcpyHostToDevice, s));
     }
+    // slices of the multi-dot and workgroups of the other square sums: about
+    // 1024 and 256 elements each while vectors are short (a step at 69 k DoFs:
+    // 33.4 us with slices of 2048, 29.6 with 1024, 31.1 with 512).  Workgroups
+    // go to the 8 XCDs in turn, so a multiple of 8 slices puts a slice of all
+    // basis vectors into one XCD's L2, for the multi-dot and the
+    // orthogonalisation alike (8.8 and 8.4 us without, 7.6 and 7.4 us with)
+    const unsigned slices = (unsigned)std::min<int64_t>(NORM_PARTS / 4, (N + 8191) / 8192 * 8);
+    const unsigned GN = grid_for(N, RED_THREADS, NORM_PARTS);
+    double *npart = part + (size_t)RED_BLOCKS * (GM_MAX + 2);
+    // Jacobi: its multiplication rides on the scaling of the basis vector
+    const T *gdinv = haspre && p->pointwise() ? (const T *)p->dinv.p : nullptr;
+    auto zvec = [&](int j) -> T * { return !gdinv ? nullptr : flex ? Z + (int64_t)j * N : z; };
     bool first = true;
     Learned *lp = p ? p->learned_part() : nullptr;
     T *xsave = lp ? (T *)S.workbuf(4, vb) : nullptr;
     while (true) {
         if (lp && lp->active()) FEM_HIP(hipMemcpyAsync(xsave, x, vb, hipMemcpyDeviceToDevice, s));
         o->apply_raw(x, V, nullptr);
-        hipLaunchKernelGGL(k_gm_start<T>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s, V, b, N, st, part, cnt, first ? 1 : 0);
-        hipLaunchKernelGGL(k_gm_scale<T>, dim3(G), dim3(256), 0, s, V, N, st);
+        hipLaunchKernelGGL(k_gm_start<T>, dim3(GN), dim3(RED_THREADS), 0, s, V, b, N, npart);
+        hipLaunchKernelGGL(k_gm_scale<T>, dim3(GN), dim3(RED_THREADS), 0, s, V, N, first ? -1 : -2, st, npart, (int)GN, m,
+                           gdinv, zvec(0));
         first = false;
         for (int j = 0; j < m; ++j) {
             T *vj = V + (int64_t)j * N, *w = V + (int64_t)(j + 1) * N;
             const int *skip = &st->cycle_done;
             if (haspre) {
                 T *zj = flex ? Z + (int64_t)j * N : z;
-                p->apply_raw(vj, zj, skip);
+                if (!gdinv) p->apply_raw(vj, zj, skip);
                 o->apply_raw(zj, w, skip);
             } else {
                 o->apply_raw(vj, w, skip);
             }
-            hipLaunchKernelGGL(k_gm_multidot<T>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s, V, w, N, j, st, part, cnt, m);
-            hipLaunchKernelGGL(k_gm_orth<T>, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, s, V, w, N, j, st, part, cnt, m);
-            hipLaunchKernelGGL(k_gm_scale<T>, dim3(G), dim3(256), 0, s, w, N, st);
+            hipLaunchKernelGGL(k_gm_multidot<T>, dim3(slices, (unsigned)(j / GRP + 1)), dim3(RED_THREADS), 0, s, V, w, N, j,
+                               st, part);
+            hipLaunchKernelGGL(k_gm_orth<T>, dim3(4 * slices), dim3(RED_THREADS), 0, s, V, w, N, j, st, part, (int)slices, npart, m);
+            hipLaunchKernelGGL(k_gm_scale<T>, dim3(GN), dim3(RED_THREADS), 0, s, w, N, j, st, npart, (int)(4 * slices), m,
+                               gdinv, j + 1 < m ? zvec(j + 1) : (T *)nullptr);
         }
-        hipLaunchKernelGGL(k_gm_backsolve, dim3(1), dim3(1), 0, s, st, m);
+        hipLaunchKernelGGL(k_gm_backsolve, dim3(1), dim3(64), 0, s, st, m);
         if (flex && haspre) {
             hipLaunchKernelGGL((k_gm_update<T, T>), dim3(G), dim3(256), 0, s, x, Z, N, st, 0);
         } else if (haspre) {
@@ -889,7 +950,7 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
         }
         FEM_HIP(hipGetLastError());
         S.fetch_state();
-        const double gres = std::fabs(S.hstate->g[S.hstate->jlast]);
+        const double gres = S.hstate->gres;
         if (verbose) { std::printf("Fem::%sGMRES it: %d : %g\n", flex ? "F" : "", S.hstate->it, gres); std::fflush(stdout); }
         if (lp && lp->active() && !S.hstate->converged && S.hstate->jlast > 0 && !(gres < 0.95 * S.hstate->res)) {
             // the learned correction stagnates or broke down: undo the cycle

@@ -1,6 +1,7 @@
 // Device-driven Krylov solvers behind the InverseOperator interface.
 #pragma once
 
+#include <cstddef>
 #include <functional>
 #include <memory>
 
@@ -18,16 +19,20 @@ struct KState {
     int crit_res;      // stop on ||r||^2 instead of <r, M^-1 r>
     double rr;         // ||r||^2 of the current residual
     // GMRES
-    double H[(GM_MAX + 1) * GM_MAX];
-    double g[GM_MAX + 1], cs[GM_MAX], sn[GM_MAX], y[GM_MAX];
-    double gtol, hinv;
+    double gtol;
+    double gres;     // the cycle's last residual estimate |g[jlast]|
     int jlast;       // inner steps done in the current cycle
     int converged;   // cycle ended by |g| < tol
     int cycle_done;  // stop inner loop (converged or maxit)
     // BiCGStab
     double nu, omega, bres;
     int fin;         // the iteration just reduced is the last one
+    // GMRES work (from here on never copied to the host)
+    double H[(GM_MAX + 1) * GM_MAX];
+    double g[GM_MAX + 1], cs[GM_MAX], sn[GM_MAX], y[GM_MAX];
 };
+// the part of KState that travels between host and device
+constexpr size_t KSTATE_HEAD = offsetof(KState, H);
 
 struct Solver {
     Context *ctx = nullptr;

@@ -288,3 +288,47 @@ def test_bicgstab_block_jacobi_diffusion_matches_oracle(ctx):
     assert info["converged"] and abs(info["iterations"] - ito) <= bicgstab_count_slack(ito)
     assert np.abs(X.download() - xo).max() <= 1e-7 * np.abs(xo).max()
     bicgstab_iterates_agree(ctx, op, oop, b, pre=True)
+
+
+@pytest.mark.parametrize("method", ["gmres", "fgmres"])
+@pytest.mark.parametrize("n,restart", [((1, 1, 1), 5), ((3, 2, 2), 1), ((3, 3, 3), 9), ((7, 6, 5), 33), ((23, 9, 8), 64)])
+def test_gmres_steps_minimise_the_residual(ctx, method, n, restart):
+    # after k steps the estimate |g_k| is the norm of b - A x over the Krylov
+    # space: the true residual of the returned iterate equals it.  Sizes: fewer
+    # DoFs than a slice of the dots, one and several groups of 8 basis vectors,
+    # the longest cycle.  Classical Gram-Schmidt loses orthogonality like the
+    # condition of the Krylov basis, far below 1e-8 of |b| over these few steps
+    rng = np.random.default_rng(restart)
+    op = fa.GalerkinOperator(ctx, fa.OP_DG_SIPG_3D, n, 2, 40.0, (1.0, -0.5, 0.25), 0.5, fa.KAPPA_CELL)
+    op.set_kappa_cell(rng.uniform(0.5, 2.0, size=n[0] * n[1] * n[2]))
+    b = rng.normal(size=op.N)
+    last = None
+    for k in (1, restart // 2 + 1, restart):
+        inv = fa.InverseOperator(ctx, method=getattr(fa, method.upper()), tolerance=1e-14, errormeasure=fa.RELATIVE,
+                                 maxiterations=k, restart=restart)
+        inv.bind(op, fa.Preconditioner(op, fa.PRE_JACOBI))
+        B, X, W = op.vector(b), op.vector(np.zeros(op.N)), op.vector()
+        inv(B, X)
+        assert abs(inv.iterations()) <= k
+        op(X, W)
+        r = np.linalg.norm(W.download() - b) / np.linalg.norm(b)
+        assert abs(r - inv.info()["true_rel_residual"]) < 1e-8
+        assert r < 1.0 + 1e-8 and (last is None or r <= last + 1e-8)
+        # the minimum over the same space, by dense least squares (small cases)
+        if op.N <= 800 and k <= 9:
+            A = np.empty((op.N, op.N))
+            e = np.zeros(op.N)
+            for i in range(op.N):
+                e[:] = 0
+                e[i] = 1
+                op(op.vector(e), W)
+                A[:, i] = W.download()
+            dinv = 1.0 / np.diag(A)
+            V = [b / np.linalg.norm(b)]
+            for _ in range(k - 1):
+                V.append(A @ (dinv * V[-1]))
+                V[-1] /= np.linalg.norm(V[-1])
+            M = np.array([A @ (dinv * v) for v in V]).T
+            y = np.linalg.lstsq(M, b, rcond=None)[0]
+            assert abs(r - np.linalg.norm(b - M @ y) / np.linalg.norm(b)) < 1e-7
+        last = r
