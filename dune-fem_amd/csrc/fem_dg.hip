@@ -28,7 +28,6 @@
 #include <type_traits>
 
 #include "fem_dg.hpp"
-#include "fem_dg_bj.hpp"
 #include "fem_dg_sync.hpp"
 
 namespace femamd {
@@ -878,13 +877,6 @@ int64_t dg_blocks(int k, const int *n)
     return (int64_t)((n[0] + epb - 1) / epb) * n[1] * n[2];
 }
 
-int64_t dg_bj_blocks(int k, int64_t E)
-{
-    FEM_CHECK(k >= 2 && k <= 5, FEM_ERR_UNSUPPORTED, "DG: order must be 1..4");
-    const int epb = 64 / (k * k);
-    return (E + epb - 1) / epb;
-}
-
 void dg_apply_bf16(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s)
 {
     switch (k) {
@@ -1299,75 +1291,5 @@ void dg_block_setup(const DGArgs<double> &a, int k, TO *Q, TO *lam, hipStream_t 
 }
 template void dg_block_setup<double>(const DGArgs<double> &, int, double *, double *, hipStream_t, bool);
 template void dg_block_setup<float>(const DGArgs<double> &, int, float *, float *, hipStream_t, bool);
-
-// one wavefront per block; lanes beyond EPB*K2 shadow element 0 (identical
-// LDS writes, no global writes)
-template <int K, typename T>
-__global__ void __launch_bounds__(64)
-    k_dg_block_apply(int64_t E, const T *__restrict__ Q, const T *__restrict__ lam, const T *__restrict__ x,
-                     T *__restrict__ y, const int *__restrict__ skip, double *__restrict__ dot)
-{
-    using S = DGShape<K>;
-    constexpr int K2 = S::K2, K3 = S::K3, EPB = S::EPB;
-    if (skip && *skip) return;
-    __shared__ T smem[EPB * K3];
-    __shared__ T qsm[EPB * (3 * K2 + 3 * K)];
-    const int tid = threadIdx.x, el0 = tid / K2, t = tid % K2, i = t / K, j = t % K;
-    const bool wr = el0 < EPB;
-    const int el = wr ? el0 : 0;
-    const int64_t e_raw = (int64_t)blockIdx.x * EPB + el;
-    const bool active = wr && e_raw < E;
-    const int64_t e = e_raw < E ? e_raw : 0;
-    T v[K];
-#pragma unroll
-    for (int c = 0; c < K; ++c) v[c] = x[e * K3 + i * K2 + j * K + c];
-    bj_element<K>(Q + e * 3 * K2, lam + e * 3 * K, smem + el * K3, qsm + el * (3 * K2 + 3 * K), i, j, wr, v);
-    if (active)
-#pragma unroll
-        for (int r = 0; r < K; ++r) y[e * K3 + i * K2 + j * K + r] = v[r];
-    if (dot) {
-        // this workgroup's <x, y> and <x, x> (fixed summation order)
-        double a1 = 0, a2 = 0;
-        if (active)
-#pragma unroll
-            for (int r = 0; r < K; ++r) {
-                const double xv = (double)x[e * K3 + i * K2 + j * K + r];
-                a1 += xv * (double)v[r];
-                a2 += xv * xv;
-            }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            a1 += __shfl_xor(a1, off, 64);
-            a2 += __shfl_xor(a2, off, 64);
-        }
-        if (tid == 0) {
-            dot[blockIdx.x] = a1;
-            dot[gridDim.x + blockIdx.x] = a2;
-        }
-    }
-}
-
-template <typename T>
-void dg_block_apply(int k, int64_t E, const T *Q, const T *lam, const T *x, T *y, const int *skip, hipStream_t s,
-                    double *dot)
-{
-#define BA_CASE(KK)                                                                                         \
-    case KK: {                                                                                              \
-        unsigned nb = (unsigned)((E + DGShape<KK>::EPB - 1) / DGShape<KK>::EPB);                            \
-        hipLaunchKernelGGL((k_dg_block_apply<KK, T>), dim3(nb), dim3(64), 0, s, E, Q, lam, x, y, skip, dot); \
-        break;                                                                                              \
-    }
-    switch (k) {
-        BA_CASE(2) BA_CASE(3) BA_CASE(4) BA_CASE(5)
-    default: throw Error(FEM_ERR_UNSUPPORTED, "block Jacobi: order must be 1..4");
-    }
-#undef BA_CASE
-    FEM_HIP(hipGetLastError());
-}
-
-template void dg_block_apply<double>(int, int64_t, const double *, const double *, const double *, double *, const int *,
-                                     hipStream_t, double *);
-template void dg_block_apply<float>(int, int64_t, const float *, const float *, const float *, float *, const int *,
-                                    hipStream_t, double *);
 
 }  // namespace femamd

@@ -189,11 +189,12 @@ void dg_rhs_bnd(const DGArgs<double> &a, int k, const double *const g[3], double
 template <typename TO>
 void dg_block_setup(const DGArgs<double> &a, int k, TO *Q /*[E][3][K][K]*/, TO *lam /*[E][3][K]*/,
                     hipStream_t s, bool bound = false);
-// `dot` (may be null): each workgroup writes its FP64 partials of <x, y> to
-// dot[workgroup] and of <x, x> to dot[dg_bj_blocks(k, E) + workgroup]
+// y = (add ? y : 0) + omega B^-1 (x - t), t may be null.  `dot` (may be null):
+// each workgroup writes its FP64 partials of <x, y> to dot[workgroup] and of
+// <x, x> to dot[dg_bj_blocks(k, E) + workgroup]
 template <typename T>
-void dg_block_apply(int k, int64_t E, const T *Q, const T *lam, const T *x, T *y, const int *skip, hipStream_t s,
-                    double *dot = nullptr);
+void dg_block_apply(int k, int64_t E, const T *Q, const T *lam, const T *x, const T *t, T *y, T omega, bool add,
+                    const int *skip, hipStream_t s, double *dot = nullptr);
 
 
 }  // namespace femamd

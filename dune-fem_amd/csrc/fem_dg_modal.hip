@@ -500,6 +500,62 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// y = (ADD ? y : 0) + omega B^-1 (x - t), t may be null; four wavefronts of
+// EPW elements each.  dot (may be null): the workgroup's <x, y> and <x, x>.
+// Reads and writes the vectors once and the eigen data (3 K^2 + 3 K values per
+// element) once, which is what bounds it.
+template <int K, typename T, bool ADD>
+__global__ void __launch_bounds__(256)
+    k_dg_block(int64_t E, const T *__restrict__ Qg, const T *__restrict__ lg, const T *__restrict__ x,
+               const T *__restrict__ t, T *__restrict__ y, T omega, const int *__restrict__ skip,
+               double *__restrict__ dot)
+{
+    using S = MShape<K>;
+    constexpr int K2 = S::K2, K3 = S::K3, EPW = S::EPW, R = 4, SZ = S::SZ;
+    if (skip && *skip) return;
+    __shared__ T smem[R * EPW * (SZ + S::SQ)];
+    const int g = threadIdx.x >> 6, tid = threadIdx.x & 63;
+    const bool wr = tid < EPW * K2;
+    const int el = wr ? tid / K2 : 0, i = (tid % K2) / K, j = tid % K2 % K, lane = i * K + j;
+    const int64_t e_raw = ((int64_t)blockIdx.x * R + g) * EPW + el;
+    const bool active = wr && e_raw < E;
+    const int64_t e = e_raw < E ? e_raw : E - 1;
+    T *const A = smem + (g * EPW + el) * SZ, *const Q = smem + R * EPW * SZ + (g * EPW + el) * S::SQ;
+    const T *xe = x + e * K3 + lane;
+    T v[K], xv[K];
+#pragma unroll
+    for (int m = 0; m < K; ++m) xv[m] = v[m] = xe[m * K2];
+    if (t) {
+        const T *te = t + e * K3 + lane;
+#pragma unroll
+        for (int m = 0; m < K; ++m) v[m] -= te[m * K2];
+    }
+    if (wr) {
+        const T *Qe = Qg + e * 3 * K2, *le = lg + e * 3 * K;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) Q[k * K2 + lane] = Qe[k * K2 + lane];
+        for (int k = lane; k < 3 * K; k += K2) Q[3 * K2 + k] = le[k];
+    }
+    wave_lds_sync();
+    bj_transform_x<K, T, 64>([&](int a_, int b_, int c_) -> T & { return A[midx<K>(a_, b_, c_)]; }, Q, i, j, wr, v);
+    double a1 = 0, a2 = 0;
+    if (active) {
+        T *ye = y + e * K3 + lane;
+#pragma unroll
+        for (int m = 0; m < K; ++m) {
+            const T r = ADD ? fma(omega, v[m], ye[m * K2]) : omega * v[m];
+            ye[m * K2] = r;
+            a1 += (double)xv[m] * (double)r;
+            a2 += (double)xv[m] * (double)xv[m];
+        }
+    }
+    if (dot) {
+        modal_dot<256>(a1, dot);
+        __syncthreads();
+        modal_dot<256>(a2, dot + gridDim.x);
+    }
+}
+
 template <int K, typename T, bool SM>
 void launch_rows(const DGArgs<T> &a, const T *u, T *w, const DGSmooth<T> &sm, const int *skip, hipStream_t s,
                  double *dot)
@@ -526,7 +582,7 @@ void launch_apply(const DGArgs<T> &a, const T *u, T *w, const int *skip, hipStre
     case 3: CALL(3); break;                                                            \
     case 4: CALL(4); break;                                                            \
     case 5: CALL(5); break;                                                            \
-    default: throw Error(FEM_ERR_UNSUPPORTED, "DG apply: order must be 1..4");         \
+    default: throw Error(FEM_ERR_UNSUPPORTED, "DG: order must be 1..4");               \
     }                                                                                  \
     FEM_HIP(hipGetLastError())
 
@@ -556,6 +612,17 @@ void modal_smooth(const DGArgs<T> &a, int k, const T *u, const DGSmooth<T> &sm, 
 #define CALL(KK) launch_rows<KK, T, true>(a, u, (T *)nullptr, sm, skip, s, (double *)nullptr)
     MODAL_SWITCH(CALL);
 #undef CALL
+}
+
+template <int K, typename T>
+void launch_block(int64_t E, const T *Q, const T *lam, const T *x, const T *t, T *y, T omega, bool add,
+                  const int *skip, hipStream_t s, double *dot)
+{
+    const unsigned nb = (unsigned)dg_bj_blocks(K, E);
+    if (add)
+        hipLaunchKernelGGL((k_dg_block<K, T, true>), dim3(nb), dim3(256), 0, s, E, Q, lam, x, t, y, omega, skip, dot);
+    else
+        hipLaunchKernelGGL((k_dg_block<K, T, false>), dim3(nb), dim3(256), 0, s, E, Q, lam, x, t, y, omega, skip, dot);
 }
 
 }  // namespace
@@ -616,6 +683,26 @@ int64_t dg_modal_blocks(int k, const int *n)
 {
     return k == 2 ? dg_modal_rows(k, n).blocks : dg_modal_tile(k, n).blocks;
 }
+
+int64_t dg_bj_blocks(int k, int64_t E)
+{
+    FEM_CHECK(k >= 2 && k <= 5, FEM_ERR_UNSUPPORTED, "DG: order must be 1..4");
+    const int epb = 4 * (64 / (k * k));
+    return (E + epb - 1) / epb;
+}
+
+template <typename T>
+void dg_block_apply(int k, int64_t E, const T *Q, const T *lam, const T *x, const T *t, T *y, T omega, bool add,
+                    const int *skip, hipStream_t s, double *dot)
+{
+#define CALL(KK) launch_block<KK, T>(E, Q, lam, x, t, y, omega, add, skip, s, dot)
+    MODAL_SWITCH(CALL);
+#undef CALL
+}
+template void dg_block_apply<double>(int, int64_t, const double *, const double *, const double *, const double *,
+                                     double *, double, bool, const int *, hipStream_t, double *);
+template void dg_block_apply<float>(int, int64_t, const float *, const float *, const float *, const float *, float *,
+                                    float, bool, const int *, hipStream_t, double *);
 
 void dg_modal_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                         double *dot)

@@ -38,7 +38,6 @@
 #include <type_traits>
 
 #include "fem_blas.hpp"
-#include "fem_dg_bj.hpp"
 #include "fem_mg.hpp"
 
 namespace femamd {
@@ -54,35 +53,6 @@ inline unsigned mg_grid(int64_t n) { return grid_for(n, MGT, 16384); }
     if (skip && *skip) return
 
 // ---- DG levels ----------------------------------------------------------------------
-// mode 0: x = omega B^-1 r;  mode 1: x += omega B^-1 (r - t), t = A x.  B^-1 is
-// the exact element-block inverse (fem_dg_bj.hpp); EPB elements of K*K lanes
-// per wavefront, extra lanes shadow element 0 without writing.
-template <int K, typename T>
-__global__ void __launch_bounds__(64)
-    k_mg_bj(int64_t E, const T *__restrict__ Q, const T *__restrict__ lam, const T *__restrict__ r,
-            const T *__restrict__ t, T *__restrict__ x, T omega, int mode, const int *__restrict__ skip)
-{
-    using S = BJShape<K>;
-    constexpr int K2 = S::K2, K3 = S::K3, EPB = S::EPB;
-    MG_SKIP;
-    __shared__ T smem[EPB * K3];
-    __shared__ T qsm[EPB * (3 * K2 + 3 * K)];
-    const int tid = threadIdx.x, el0 = tid / K2, tl = tid % K2, i = tl / K, j = tl % K;
-    const bool wr = el0 < EPB;
-    const int el = wr ? el0 : 0;
-    const int64_t e_raw = (int64_t)blockIdx.x * EPB + el;
-    const bool active = wr && e_raw < E;
-    const int64_t e = e_raw < E ? e_raw : 0;
-    const int64_t base = e * K3 + i * K2 + j * K;
-    T v[K];
-#pragma unroll
-    for (int c = 0; c < K; ++c) v[c] = mode ? r[base + c] - t[base + c] : r[base + c];
-    bj_element<K>(Q + e * 3 * K2, lam + e * 3 * K, smem + el * K3, qsm + el * (3 * K2 + 3 * K), i, j, wr, v);
-    if (active)
-#pragma unroll
-        for (int c = 0; c < K; ++c) x[base + c] = mode ? x[base + c] + omega * v[c] : omega * v[c];
-}
-
 // rc = (r - t) on the modes a, b, c < Kc (local index a Kf^2 + b Kf + c)
 template <typename T>
 __global__ void k_mg_restrict_modes(int64_t E, int Kf, int Kc, const T *__restrict__ r, const T *__restrict__ t,
@@ -919,21 +889,11 @@ void Multigrid::cycle_vertex(size_t l, const T *r, T *x, const int *skip)
     FEM_HIP(hipGetLastError());
 }
 
+// mode 0: x = omega B^-1 r;  mode 1: x += omega B^-1 (r - t), t = A x
 template <typename T>
 static void mg_bj(const MGDGLevel &L, const T *r, const T *t, T *x, T omega, int mode, const int *skip, hipStream_t s)
 {
-    const int64_t E = L.op->E;
-    const T *Q = L.bj.Q.as<T>(), *lam = L.bj.lam.as<T>();
-#define MGBJ_CASE(KK)                                                                                        \
-    case KK:                                                                                                 \
-        hipLaunchKernelGGL((k_mg_bj<KK, T>), dim3((unsigned)((E + BJShape<KK>::EPB - 1) / BJShape<KK>::EPB)), \
-                           dim3(64), 0, s, E, Q, lam, r, t, x, omega, mode, skip);                           \
-        break;
-    switch (L.k) {
-        MGBJ_CASE(2) MGBJ_CASE(3) MGBJ_CASE(4) MGBJ_CASE(5)
-    default: throw Error(FEM_ERR_UNSUPPORTED, "multigrid: order must be 1..4");
-    }
-#undef MGBJ_CASE
+    dg_block_apply<T>(L.k, L.op->E, L.bj.Q.as<T>(), L.bj.lam.as<T>(), r, mode ? t : nullptr, x, omega, mode != 0, skip, s);
 }
 
 // one damped block-Jacobi sweep on a level, out = in + omega B^-1 (r - A in),

@@ -149,11 +149,12 @@ struct Precond {
     bool updatable_for(const Operator *o, int k) const;
     void init_widening(Operator *o64, const Precond *p32);
     Learned *learned_part() const { return lowp ? lowp->learned : learned; }
-    // `dot` (block Jacobi only, may be null): per-workgroup FP64 partials of
-    // <x, y> and then of <x, x>, op->dot_blocks() entries each
+    // `dot` (where fused_dot(), may be null): per-workgroup FP64 partials of
+    // <x, y> and then of <x, x>, dot_parts() entries each
     void apply_raw(const void *x, void *y, const int *skip, double *dot = nullptr) const;
     bool pointwise() const { return kind == FEM_PRE_JACOBI; }
-    bool fused_dot() const { return kind == FEM_PRE_BLOCK_JACOBI; }
+    bool fused_dot() const { return kind == FEM_PRE_BLOCK_JACOBI || lowp != nullptr; }
+    int64_t dot_parts() const;
     ~Precond();
 };
 

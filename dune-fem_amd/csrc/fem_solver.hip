@@ -28,25 +28,36 @@
 namespace femamd {
 
 constexpr int GRP = 8;   // vectors per register group in the multi-dot
+// partials that every workgroup of the next kernel sums in CG at most, and
+// what more are brought down to
+constexpr int CG_PARTS = 4096, CG_FEWER = 256;
 // partials of a square sum at most (after the multi-dot's in the workspace)
 constexpr int NORM_PARTS = 1024;
-// the CG reductions use RED_DOT_BLOCKS partial slots per quantity (two)
-static_assert(2 * RED_DOT_BLOCKS <= RED_BLOCKS * (GM_MAX + 1), "solver partials buffer");
 
-__device__ __forceinline__ void fin_cg_alpha(KState *st, double qh)
-{
-    st->qh = qh;
-    st->alpha = st->res / qh;
-}
+// Reductions of CG and GMRES: a reduction leaves one partial per workgroup,
+// and the kernel that needs the result sums the partials itself, each
+// workgroup all of them in the same order.  A kernel boundary orders the two,
+// where a finish by the last workgroup to arrive waits for a chain of atomics
+// (69 k DoFs, restart 30: multi-dot 37 us and orthogonalisation 15 us with
+// that finish on 512 workgroups, 7.6 and 7.4 us so).  The grids grow with the
+// vector, so that few partials are left where the sums are short.
 
-__device__ __forceinline__ void fin_cg_res(KState *st, double r, double rr)
+// the sum of n partials, in every thread, for every workgroup alike: thread t
+// takes t, t + 256, ..., then a tree over the workgroup
+__device__ __forceinline__ double sum_parts(const double *__restrict__ part, int n, double *lds)
 {
-    st->prev = st->res;
-    st->res = r;
-    st->rr = rr;
-    st->beta = r / st->prev;
-    st->it += 1;
-    st->done = !((st->crit_res ? rr : r) > st->tol) || st->it >= st->maxit;
+    double v = 0;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < n; k += RED_THREADS) v += part[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = 0;
+#pragma unroll
+    for (int w = 0; w < RED_THREADS / 64; ++w) s += lds[w];
+    return s;
 }
 
 // ---- CG kernels ---------------------------------------------------------------
@@ -70,174 +81,222 @@ __global__ void k_cg_init(KState *st, double eps, int criteria, int maxit, int c
     st->maxit = maxit;
     st->crit_res = crit_res;
     st->done = !(r0 > st->tol) || maxit <= 0;
+    st->fresh = 1;
+    st->n_res = st->res;
+    st->n_rr = st->rr;
+    st->n_it = 0;
 }
 
-template <typename T>
-__global__ void k_cg_qupd(T *__restrict__ q, const T *__restrict__ s, T *__restrict__ p, const T *__restrict__ r,
-                          int64_t n, const KState *__restrict__ st, int haspre)
+// A CG step is: direction (k_cg_dir), apply with the partials of <q, h>,
+// update (k_cg_update), preconditioner with the partials of <p, s> and
+// <p, p>.  The direction kernel sums the latter, forms beta and the stopping
+// test, and leaves the new scalars in n_*; the update kernel sums <q, h>,
+// forms alpha and makes n_* current.  No workgroup of either reads what its
+// first workgroup writes there.
+
+// two sums at once, of part[0..n) and part[n..2n)
+__device__ __forceinline__ void sum_parts2(const double *__restrict__ part, int n, double *lds, double &s0, double &s1)
 {
-    if (st->done || st->it == 0) return;
-    const double beta = st->beta;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        if (haspre) q[i] = (T)(beta * (double)q[i] + (double)s[i]);
-        else p[i] = (T)(beta * (double)p[i] - (double)r[i]);
+    double v = 0, u = 0;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < n; k += RED_THREADS) {
+        v += part[k];
+        u += part[n + k];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        v += __shfl_xor(v, off, 64);
+        u += __shfl_xor(u, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        lds[threadIdx.x >> 6] = v;
+        lds[RED_THREADS / 64 + (threadIdx.x >> 6)] = u;
+    }
+    __syncthreads();
+    s0 = s1 = 0;
+#pragma unroll
+    for (int w = 0; w < RED_THREADS / 64; ++w) {
+        s0 += lds[w];
+        s1 += lds[RED_THREADS / 64 + w];
     }
 }
 
-// reduction kernels share one pattern: grid-stride update + partial dot,
-// block sum, deterministic finish by the last block
+// <p, s> and <p, p> from pp[2][np], and what follows: whether the solve is done
+__device__ __forceinline__ bool cg_end_of_step(KState *st, const double *__restrict__ pp, int np, double *lds,
+                                               bool keeper, double &beta)
+{
+    double r, rr;
+    sum_parts2(pp, np, lds, r, rr);
+    const int it = st->it + 1;
+    beta = r / st->res;
+    const bool done = !((st->crit_res ? rr : r) > st->tol) || it >= st->maxit;
+    __syncthreads();   // every thread has read the scalars
+    if (keeper && threadIdx.x == 0) {
+        st->n_res = r;
+        st->n_rr = rr;
+        st->n_it = it;
+        if (done) {
+            st->res = r;
+            st->rr = rr;
+            st->it = it;
+            st->done = 1;
+        }
+    }
+    return done;
+}
+
+// the same test after the last step of a batch, for the host to read (the
+// next direction kernel repeats it if the solve goes on)
+__global__ void __launch_bounds__(RED_THREADS) k_cg_check(KState *st, const double *__restrict__ pp, int np)
+{
+    if (st->done || st->fresh) return;
+    __shared__ double lds[2 * (RED_THREADS / 64)];
+    double beta;
+    cg_end_of_step(st, pp, np, lds, true, beta);
+}
+
+// q = beta q + s, without a preconditioner p = beta p - r
+template <typename T>
+__global__ void __launch_bounds__(RED_THREADS)
+    k_cg_dir(T *__restrict__ q, const T *__restrict__ s, const T *__restrict__ r, int64_t n, KState *st,
+             const double *__restrict__ pp, int np, int haspre)
+{
+    if (st->done || st->fresh) return;
+    __shared__ double lds[2 * (RED_THREADS / 64)];
+    double beta;
+    if (cg_end_of_step(st, pp, np, lds, blockIdx.x == 0, beta)) return;
+    const int64_t stride = (int64_t)gridDim.x * RED_THREADS;
+    int64_t i = blockIdx.x * (int64_t)RED_THREADS + threadIdx.x;
+    const T *a = haspre ? s : r;
+    const double sg = haspre ? 1.0 : -1.0;
+    // four independent elements in flight per thread
+    for (; i + 3 * stride < n; i += 4 * stride) {
+        T vq[4], va[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            vq[k] = q[i + k * stride];
+            va[k] = a[i + k * stride];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[i + k * stride] = (T)(beta * (double)vq[k] + sg * (double)va[k]);
+    }
+    for (; i < n; i += stride) q[i] = (T)(beta * (double)q[i] + sg * (double)a[i]);
+}
+
+// MODE 0: x += a q, p -= a h (a general preconditioner follows)
+// MODE 1: the same, s = dinv p and the partials of <p, s>, <p, p> (Jacobi)
+// MODE 2: x += a q, r += a h and the partials of <r, r>, twice (no
+//         preconditioner; p is r here)
 template <typename T, int MODE>
 __global__ void __launch_bounds__(RED_THREADS)
-    k_cg_step(T *__restrict__ x, T *__restrict__ p, const T *__restrict__ q, const T *__restrict__ h,
-              T *__restrict__ s, T *__restrict__ r, const T *__restrict__ dinv, int64_t n, KState *st,
-              double *partials, unsigned *counter)
+    k_cg_update(T *__restrict__ x, T *__restrict__ p, const T *__restrict__ q, const T *__restrict__ h,
+                T *__restrict__ s, const T *__restrict__ dinv, int64_t n, KState *st, const double *__restrict__ qp,
+                int nq, double *__restrict__ pp)
 {
     if (st->done) return;
     __shared__ double lds[RED_THREADS / 64];
+    const double qh = sum_parts(qp, nq, lds);
+    const double alpha = st->n_res / qh;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->qh = qh;
+        st->alpha = alpha;
+        st->res = st->n_res;
+        st->rr = st->n_rr;
+        st->it = st->n_it;
+        st->fresh = 0;
+    }
     double acc = 0, acc2 = 0;
-    const double alpha = st->alpha;
-    int64_t i0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (MODE == 0 || MODE == 3) {
-        // pure reductions: four independent loads of each operand in flight
-        // per thread before they are used
-        const T *A = MODE == 0 ? q : p;
-        const T *Bv = MODE == 0 ? h : s;
-        constexpr int U = 4;
-        const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-        for (; i0 + (U - 1) * stride < n; i0 += U * stride) {
-            T va[U], vb[U];
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-                va[k] = A[i0 + k * stride];
-                vb[k] = Bv[i0 + k * stride];
-            }
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-                acc += (double)va[k] * (double)vb[k];
-                if (MODE == 3) acc2 += (double)va[k] * (double)va[k];
-            }
-        }
-    }
-    for (int64_t i = i0; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        if (MODE == 0) {          // dot(q, h) -> alpha
-            acc += (double)q[i] * (double)h[i];
-        } else if (MODE == 1) {   // pointwise Jacobi: x += a q, p -= a h, s = d p, <p, s>
-            x[i] = (T)((double)x[i] + alpha * (double)q[i]);
-            const double pn = (double)p[i] - alpha * (double)h[i];
-            const T pt = (T)pn;
-            p[i] = pt;
-            const T sv = dinv[i] * pt;
+    auto one = [&](int64_t i, T xv, T pv, T qv, T hv, T dv) {
+        x[i] = (T)((double)xv + alpha * (double)qv);
+        const T pn = (T)((double)pv + (MODE == 2 ? alpha : -alpha) * (double)hv);
+        p[i] = pn;
+        if (MODE == 1) {
+            const T sv = dv * pn;
             s[i] = sv;
-            acc += (double)pt * (double)sv;
-            acc2 += (double)pt * (double)pt;
-        } else if (MODE == 2) {   // general M: x += a q, p -= a h (no reduction)
-            x[i] = (T)((double)x[i] + alpha * (double)q[i]);
-            p[i] = (T)((double)p[i] - alpha * (double)h[i]);
-        } else if (MODE == 3) {   // <p, s> after a general M
-            acc += (double)p[i] * (double)s[i];
-            acc2 += (double)p[i] * (double)p[i];
-        } else {                  // no preconditioner: x += a p, r += a h, <r, r>
-            x[i] = (T)((double)x[i] + alpha * (double)q[i]);
-            const T rn = (T)((double)r[i] + alpha * (double)h[i]);
-            r[i] = rn;
-            acc += (double)rn * (double)rn;
-            acc2 = acc;
+            acc += (double)pn * (double)sv;
         }
+        if (MODE != 0) acc2 += (double)pn * (double)pn;
+    };
+    const int64_t stride = (int64_t)gridDim.x * RED_THREADS;
+    int64_t i = blockIdx.x * (int64_t)RED_THREADS + threadIdx.x;
+    for (; i + 3 * stride < n; i += 4 * stride) {
+        T xv[4], pv[4], qv[4], hv[4], dv[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t o = i + k * stride;
+            xv[k] = x[o];
+            pv[k] = p[o];
+            qv[k] = q[o];
+            hv[k] = h[o];
+            dv[k] = MODE == 1 ? dinv[o] : T(0);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) one(i + k * stride, xv[k], pv[k], qv[k], hv[k], dv[k]);
     }
-    if (MODE == 2) return;
-    double b = block_sum(acc, lds);
+    for (; i < n; i += stride) one(i, x[i], p[i], q[i], h[i], MODE == 1 ? dinv[i] : T(0));
+    if (MODE == 0) return;
     __syncthreads();
-    double b2 = block_sum(acc2, lds);
-    __shared__ bool amLast;
+    const double b2 = block_sum(acc2, lds);
+    __syncthreads();
+    const double b = MODE == 1 ? block_sum(acc, lds) : b2;
     if (threadIdx.x == 0) {
-        publish_partial(&partials[blockIdx.x], b);
-        publish_partial(&partials[gridDim.x + blockIdx.x], b2);
-        amLast = atomicAdd(counter, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!amLast) return;
-    double v = 0, v2 = 0;
-    for (unsigned k = threadIdx.x; k < gridDim.x; k += blockDim.x) {
-        v += read_partial(&partials[k]);
-        v2 += read_partial(&partials[gridDim.x + k]);
-    }
-    double tot = block_sum(v, lds);
-    __syncthreads();
-    double tot2 = block_sum(v2, lds);
-    if (threadIdx.x == 0) {
-        if (MODE == 0) fin_cg_alpha(st, tot);
-        else fin_cg_res(st, tot, tot2);
-        reset_counter(counter);
+        pp[blockIdx.x] = b;
+        pp[gridDim.x + blockIdx.x] = b2;
     }
 }
 
-// Finish of a dot whose per-workgroup partials were written by the DG apply
-// (MODE 0: <q, h> -> alpha) or by block Jacobi (MODE 3: <p, s> and <p, p> ->
-// beta, residual, convergence).  The partials are summed in a fixed order, so
-// the result is reproducible run to run.
-template <int MODE>
+// partials of <a, b> and (NQ = 2) of <a, a>
+template <typename T, int NQ>
 __global__ void __launch_bounds__(RED_THREADS)
-    k_cg_fin_parts(const double *__restrict__ ext, int64_t nb, KState *st, double *partials, unsigned *counter)
+    k_cg_dots(const T *__restrict__ a, const T *__restrict__ b, int64_t n, const KState *__restrict__ st,
+              double *__restrict__ out)
 {
     if (st->done) return;
     __shared__ double lds[RED_THREADS / 64];
     double acc = 0, acc2 = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nb; i += (int64_t)gridDim.x * blockDim.x) {
-        acc += ext[i];
-        if (MODE == 3) acc2 += ext[nb + i];
+    const int64_t stride = (int64_t)gridDim.x * RED_THREADS;
+    int64_t i = blockIdx.x * (int64_t)RED_THREADS + threadIdx.x;
+    for (; i + 3 * stride < n; i += 4 * stride) {
+        T va[4], vb[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            va[k] = a[i + k * stride];
+            vb[k] = b[i + k * stride];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            acc += (double)va[k] * (double)vb[k];
+            if (NQ == 2) acc2 += (double)va[k] * (double)va[k];
+        }
     }
-    double b = block_sum(acc, lds);
+    for (; i < n; i += stride) {
+        acc += (double)a[i] * (double)b[i];
+        if (NQ == 2) acc2 += (double)a[i] * (double)a[i];
+    }
+    const double s = block_sum(acc, lds);
     __syncthreads();
-    double b2 = block_sum(acc2, lds);
-    __shared__ bool amLast;
+    const double s2 = NQ == 2 ? block_sum(acc2, lds) : 0.0;
     if (threadIdx.x == 0) {
-        publish_partial(&partials[blockIdx.x], b);
-        publish_partial(&partials[gridDim.x + blockIdx.x], b2);
-        amLast = atomicAdd(counter, 1u) == gridDim.x - 1;
+        out[blockIdx.x] = s;
+        if (NQ == 2) out[gridDim.x + blockIdx.x] = s2;
     }
-    __syncthreads();
-    if (!amLast) return;
-    double v = 0, v2 = 0;
-    for (unsigned k = threadIdx.x; k < gridDim.x; k += blockDim.x) {
-        v += read_partial(&partials[k]);
-        v2 += read_partial(&partials[gridDim.x + k]);
-    }
-    double tot = block_sum(v, lds);
-    __syncthreads();
-    double tot2 = block_sum(v2, lds);
-    if (threadIdx.x == 0) {
-        if (MODE == 0) fin_cg_alpha(st, tot);
-        else fin_cg_res(st, tot, tot2);
-        reset_counter(counter);
+}
+
+// many partials to fewer: workgroup b sums its part of each of the nq lists
+// in[k * n ..] into out[k * gridDim.x + b]
+__global__ void __launch_bounds__(RED_THREADS)
+    k_cg_fewer(const double *__restrict__ in, int64_t n, int nq, double *__restrict__ out, const KState *__restrict__ st)
+{
+    if (st->done) return;
+    __shared__ double lds[RED_THREADS / 64];
+    const int64_t lo = n * blockIdx.x / gridDim.x, hi = n * (blockIdx.x + 1) / gridDim.x;
+    for (int k = 0; k < nq; ++k) {
+        const double t = sum_parts(in + k * n + lo, (int)(hi - lo), lds);
+        if (threadIdx.x == 0) out[(int64_t)k * gridDim.x + blockIdx.x] = t;
     }
 }
 
 // ---- GMRES kernels --------------------------------------------------------------
-// A reduction leaves one partial per workgroup, and the kernel that needs the
-// result sums the partials itself, each workgroup all of them in the same
-// order: a kernel boundary orders the two, where a finish by the last
-// workgroup to arrive waits for a chain of atomics (at 69 k DoFs, restart 30:
-// multi-dot 37 us and orthogonalisation 15 us with that finish on 512
-// workgroups, 7.6 and 7.4 us so).  The grids grow with the vector, so that few
-// partials are left where the sums are short.
-
-// the sum of n partials, in every thread, for every workgroup alike: thread t
-// takes t, t + 256, ..., then a tree over the workgroup
-__device__ __forceinline__ double sum_parts(const double *__restrict__ part, int n, double *lds)
-{
-    double v = 0;
-    for (int k = threadIdx.x; k < n; k += RED_THREADS) v += part[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double s = 0;
-#pragma unroll
-    for (int w = 0; w < RED_THREADS / 64; ++w) s += lds[w];
-    return s;
-}
-
 // v0 -= b (v0 = A x on entry), partials of ||v0||^2
 template <typename T>
 __global__ void __launch_bounds__(RED_THREADS)
@@ -725,6 +784,8 @@ void Solver::fetch_state()
     FEM_HIP(hipStreamSynchronize(ctx->stream));
 }
 
+static bool pfused_bj(const Precond *p) { return p->kind == FEM_PRE_BLOCK_JACOBI; }
+
 template <typename T>
 static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b, T *x, double eps, int criteria,
                       int maxit, int m, int64_t N, int verbose)
@@ -751,20 +812,24 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
         dot_async(*S.ctx, N, b, b, &st->bnorm2, cnt + 1, part);
         hipLaunchKernelGGL(k_cg_init, dim3(1), dim3(1), 0, s, st, eps, criteria, maxit, S.prm.residual_check);
         FEM_HIP(hipGetLastError());
-        const T *dinv = (haspre && p->pointwise()) ? (p->prec == FEM_F64 ? (const T *)p->dinv.p : (const T *)p->dinv.p) : nullptr;
-        // DG operator with block Jacobi: the apply and the preconditioner
-        // write per-workgroup partials of the two CG dots, which a small
-        // kernel finishes, instead of two more passes over the vectors
-        const bool fuse = o->is_dg() && haspre && p->fused_dot() && o->desc.precision != FEM_BF16MFMA;
-        const int64_t nbd = fuse ? o->dot_blocks() : 0;        // apply workgroups
-        const int64_t nbj = fuse ? dg_bj_blocks(p->op->k, p->op->E) : 0;   // block-Jacobi workgroups
-        // about 4 partials per thread: a small launch finishes quickly
-        auto fin_grid = [](int64_t n) {
-            return (unsigned)std::min<int64_t>(RED_DOT_BLOCKS, std::max<int64_t>(1, (n + 4 * RED_THREADS - 1) / (4 * RED_THREADS)));
-        };
-        const unsigned GF = fin_grid(nbd), GJ = fin_grid(nbj);
-        double *dq = fuse ? (double *)S.workbuf(5, sizeof(double) * nbd) : nullptr;
-        double *dp = fuse ? (double *)S.workbuf(6, 2 * sizeof(double) * nbj) : nullptr;
+        const T *dinv = (haspre && p->pointwise()) ? (const T *)p->dinv.p : nullptr;
+        // workgroups of the vector kernels (about four elements per thread),
+        // and the partials of <q, h> and of <p, s>, <p, p>: from the DG apply
+        // and from the preconditioner where they write them, else from a pass
+        // over the vectors.  Every workgroup of the kernel that follows sums
+        // them, so more than CG_PARTS are first brought down to CG_FEWER
+        const unsigned GU = grid_for(N, 4 * RED_THREADS, CG_PARTS / 4);
+        const bool qfused = o->is_dg() && o->desc.precision != FEM_BF16MFMA;
+        const bool pfused = haspre && p->fused_dot();
+        const int64_t nq0 = qfused ? o->dot_blocks() : GU, np0 = pfused ? p->dot_parts() : GU;
+        const int nq = (int)(nq0 > CG_PARTS ? CG_FEWER : nq0), np = (int)(np0 > CG_PARTS ? CG_FEWER : np0);
+        double *dq = (double *)S.workbuf(5, sizeof(double) * (nq0 + CG_FEWER));
+        double *dp = (double *)S.workbuf(6, 2 * sizeof(double) * (np0 + CG_FEWER));
+        double *qparts = nq0 > CG_PARTS ? dq + nq0 : dq, *pparts = np0 > CG_PARTS ? dp + 2 * np0 : dp;
+        // steps between two looks of the host: a look costs about 20 us, a
+        // step past the end one idle launch per kernel, of which a multigrid
+        // step has some forty
+        const int most = haspre && !dinv && !pfused_bj(p) ? 4 : 32;
         int chunk = S.snapshot ? S.snap_chunk : 4;
         // one CG step as a HIP graph: every kernel of the step reads the
         // device done flag, so replays after convergence do nothing; the step
@@ -781,26 +846,27 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
             }
         } gguard{ graph, gexec };
         auto cg_step = [&]() {
-                hipLaunchKernelGGL(k_cg_qupd<T>, dim3(G), dim3(256), 0, s, q, ss, pp, r, N, st, haspre ? 1 : 0);
-                if (fuse) {
-                    o->apply_raw(q, h, &st->done, dq);
-                    hipLaunchKernelGGL(k_cg_fin_parts<0>, dim3(GF), dim3(RED_THREADS), 0, s, dq, nbd, st, part, cnt);
-                    hipLaunchKernelGGL((k_cg_step<T, 2>), dim3(RED_DOT_BLOCKS), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, r, dinv, N, st, part, cnt);
-                    p->apply_raw(pp, ss, &st->done, dp);
-                    hipLaunchKernelGGL(k_cg_fin_parts<3>, dim3(GJ), dim3(RED_THREADS), 0, s, dp, nbj, st, part, cnt);
-                    return;
-                }
-                o->apply_raw(q, h, &st->done);
-                hipLaunchKernelGGL((k_cg_step<T, 0>), dim3(RED_DOT_BLOCKS), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, r, dinv, N, st, part, cnt);
-                if (!haspre) {
-                    hipLaunchKernelGGL((k_cg_step<T, 4>), dim3(RED_DOT_BLOCKS), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, r, dinv, N, st, part, cnt);
-                } else if (dinv) {
-                    hipLaunchKernelGGL((k_cg_step<T, 1>), dim3(RED_DOT_BLOCKS), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, r, dinv, N, st, part, cnt);
-                } else {
-                    hipLaunchKernelGGL((k_cg_step<T, 2>), dim3(RED_DOT_BLOCKS), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, r, dinv, N, st, part, cnt);
-                    p->apply_raw(pp, ss, &st->done);
-                    hipLaunchKernelGGL((k_cg_step<T, 3>), dim3(RED_DOT_BLOCKS), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, r, dinv, N, st, part, cnt);
-                }
+            hipLaunchKernelGGL(k_cg_dir<T>, dim3(GU), dim3(RED_THREADS), 0, s, q, ss, r, N, st, pparts, np, haspre ? 1 : 0);
+            o->apply_raw(q, h, &st->done, qfused ? dq : nullptr);
+            if (!qfused)
+                hipLaunchKernelGGL((k_cg_dots<T, 1>), dim3(GU), dim3(RED_THREADS), 0, s, q, h, N, st, dq);
+            if (nq0 > CG_PARTS)
+                hipLaunchKernelGGL(k_cg_fewer, dim3(CG_FEWER), dim3(RED_THREADS), 0, s, dq, nq0, 1, qparts, st);
+            if (!haspre) {
+                hipLaunchKernelGGL((k_cg_update<T, 2>), dim3(GU), dim3(RED_THREADS), 0, s, x, r, q, h, (T *)nullptr, dinv,
+                                   N, st, qparts, nq, dp);
+            } else if (dinv) {
+                hipLaunchKernelGGL((k_cg_update<T, 1>), dim3(GU), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, dinv, N, st,
+                                   qparts, nq, dp);
+            } else {
+                hipLaunchKernelGGL((k_cg_update<T, 0>), dim3(GU), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, dinv, N, st,
+                                   qparts, nq, dp);
+                p->apply_raw(pp, ss, &st->done, pfused ? dp : nullptr);
+                if (!pfused)
+                    hipLaunchKernelGGL((k_cg_dots<T, 2>), dim3(GU), dim3(RED_THREADS), 0, s, pp, ss, N, st, dp);
+            }
+            if (np0 > CG_PARTS)
+                hipLaunchKernelGGL(k_cg_fewer, dim3(CG_FEWER), dim3(RED_THREADS), 0, s, dp, np0, 2, pparts, st);
         };
         if (S.prm.graph && !S.snapshot) {
             FEM_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -813,12 +879,13 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
                 if (gexec) FEM_HIP(hipGraphLaunch(gexec, s));
                 else cg_step();
             }
+            hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(RED_THREADS), 0, s, st, pparts, np);
             FEM_HIP(hipGetLastError());
             S.fetch_state();
-            if (verbose) { std::printf("Fem::CG it: %d : residual %g\n", S.hstate->it, std::sqrt(S.hstate->res)); std::fflush(stdout); }
+            if (verbose) { std::printf("Fem::CG it: %d : residual %g\n", S.hstate->n_it, std::sqrt(S.hstate->n_res)); std::fflush(stdout); }
             if (S.hstate->done) break;
             if (S.snapshot) S.snapshot(x, pp);
-            else if (chunk < 64) chunk *= 2;
+            else if (chunk < most) chunk *= 2;
         }
         const int it = S.hstate->it;
         return it < maxit ? it : -it;

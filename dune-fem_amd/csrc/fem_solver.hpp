@@ -18,6 +18,10 @@ struct KState {
     int it, done, maxit, criteria;
     int crit_res;      // stop on ||r||^2 instead of <r, M^-1 r>
     double rr;         // ||r||^2 of the current residual
+    // CG: the scalars after the step just reduced, and whether no step has
+    // been made yet
+    double n_res, n_rr;
+    int n_it, fresh;
     // GMRES
     double gtol;
     double gres;     // the cycle's last residual estimate |g[jlast]|

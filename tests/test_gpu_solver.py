@@ -332,3 +332,89 @@ def test_gmres_steps_minimise_the_residual(ctx, method, n, restart):
             y = np.linalg.lstsq(M, b, rcond=None)[0]
             assert abs(r - np.linalg.norm(b - M @ y) / np.linalg.norm(b)) < 1e-7
         last = r
+
+
+@pytest.mark.parametrize("case", ["none", "one_element", "jacobi", "jacobi_many_partials", "lagrange_jacobi", "bj",
+                                  "bj_fp32_inner", "mg", "mg32", "bf16"])
+@pytest.mark.parametrize("graph", [0, 1])
+def test_cg_steps_match_the_recurrence(ctx, case, graph):
+    # the iterate after k steps against the recurrence of cg.hh:19-117 on the
+    # host with the same apply and preconditioner.  Each way a step takes its
+    # dots: from the apply, from the preconditioner, from passes over the
+    # vectors, from more partials than a workgroup sums.  The recurrences differ
+    # by the rounding of the dots, about 1e-16 sqrt(N) per step, amplified by
+    # less than the condition number (below 1e5 here): 1e-8 in FP64, 1e-2 in
+    # FP32 and BF16
+    rng = np.random.default_rng(3)
+    n, p, prec, kind = (7, 6, 5), 2, fa.F64, fa.KAPPA_CELL
+    if case == "one_element":
+        n = (1, 1, 1)
+    if case == "jacobi_many_partials":
+        n, p, kind = (16, 66, 65), 1, fa.KAPPA_QP
+    if case == "bj_fp32_inner":
+        prec = fa.F32
+    if case == "bf16":
+        prec = fa.BF16MFMA
+    if case == "lagrange_jacobi":
+        op = fa.GalerkinOperator(ctx, fa.OP_CG_Q2_2D, (37, 29), 2, c=1.0)
+    else:
+        m, E = p + 1, n[0] * n[1] * n[2]
+        op = fa.GalerkinOperator(ctx, fa.OP_DG_SIPG_3D, n, p, 10.0 * p * p, (0, 0, 0), 0.0, kind, precision=prec)
+        if kind == fa.KAPPA_CELL:
+            op.set_kappa_cell(rng.uniform(0.5, 2.0, size=E))
+        else:
+            op.set_kappa_qp(np.full((E, m ** 3), 1.5),
+                            [np.full(((n[0] + (d == 0)) * (n[1] + (d == 1)) * (n[2] + (d == 2)), m * m), 1.5)
+                             for d in range(3)])
+    pre = None
+    if "jacobi" in case:
+        pre = fa.Preconditioner(op, fa.PRE_JACOBI)
+    elif "bj" in case or case == "bf16":
+        pre = fa.Preconditioner(op, fa.PRE_BLOCK_JACOBI)
+    elif case == "mg":
+        pre = fa.Preconditioner(op, fa.PRE_MULTIGRID)
+    elif case == "mg32":
+        op32 = fa.GalerkinOperator(ctx, fa.OP_DG_SIPG_3D, n, p, 10.0 * p * p, (0, 0, 0), 0.0, kind, precision=fa.F32)
+        op32.set_kappa_cell(np.random.default_rng(3).uniform(0.5, 2.0, size=E))
+        pre = fa.Preconditioner(op32, fa.PRE_MULTIGRID)
+    U, W = op.vector(), op.vector()
+    P32 = (op32.vector(), op32.vector()) if case == "mg32" else None
+
+    def A(v):
+        U.upload(v)
+        op(U, W)
+        return W.download()
+
+    def M(v):
+        if pre is None:
+            return v.copy()
+        a, b = P32 or (U, W)
+        a.upload(v)
+        pre(a, b)
+        return b.download()
+
+    b = rng.normal(size=op.N)
+    if case == "lagrange_jacobi":
+        b = A(b)
+    for k in (1, 2, 6):
+        x = np.zeros(op.N)
+        r = b - A(x)
+        q = M(r)
+        s, res = q.copy(), np.dot(r, q)
+        for it in range(k):
+            if it:
+                q = s + beta * q
+            h = A(q)
+            alpha = res / np.dot(q, h)
+            x, r = x + alpha * q, r - alpha * h
+            s = M(r)
+            new = np.dot(r, s)
+            beta, res = new / res, new
+        inv = fa.InverseOperator(ctx, method=fa.CG, tolerance=1e-30, errormeasure=fa.RELATIVE, maxiterations=k, graph=graph)
+        inv.bind(op, pre)
+        X = op.vector(np.zeros(op.N))
+        inv(op.vector(b), X)
+        assert inv.iterations() == -k
+        err = np.linalg.norm(X.download() - x) / np.linalg.norm(x)
+        print("cg", case, k, err, flush=True)
+        assert err < (1e-8 if prec == fa.F64 else 1e-2)
