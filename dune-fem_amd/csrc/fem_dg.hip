@@ -326,11 +326,10 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
     // values: loaded once as x-pencils, the y- and z-pencils come from LDS
     // (K = 4 only: the other orders keep the face-trace scratch there)
     constexpr bool KLDS = (K == 4) && KQ;
-    // the pointwise/nonlinear reaction is compiled into the applies with
-    // constant or cellwise kappa (which come here only with a reaction) and
-    // into a separate variant (RX) of the pointwise-kappa apply: the
-    // pointwise-kappa kernel without it keeps its code and registers
-    constexpr bool CV = (!KQ && !MF) || RX;
+    // the pointwise/nonlinear reaction is compiled into a variant (RX) of the
+    // pointwise-kappa apply: the kernel without it keeps its code and registers
+    // (with kappa constant per element the modal kernels have it)
+    constexpr bool CV = RX;
     constexpr int SZ = F64MF_ ? (KLDS ? 244 : 164) : D35 ? (K == 3 ? 107 : 361) : S::SZ;
     static_assert(!F64MF_ || SZ >= (KLDS ? 3 : 2) * K * S1, "tensors per element");
     static_assert(F64MF_ || SZ >= 2 * K * S1 + 4 * SXQ, "tensors and face-trace scratch per element");
@@ -828,13 +827,17 @@ static void launch_apply(const DGArgs<T> &a, const T *u, T *w, const int *skip, 
     const int64_t E = (int64_t)a.n[0] * a.n[1] * a.n[2];
     FEM_CHECK(E * S::K3 < (int64_t)1 << 31, FEM_ERR_UNSUPPORTED, "DG apply: more than 2^31 DoFs");
     const unsigned nb = (unsigned)dg_blocks(K, a.n);
-    if (a.kappa_mode == FEM_KAPPA_QP && (a.cvol || a.nl_pow)) {
-        if constexpr (!MF)
+    if constexpr (MF) {
+        if (a.kappa_mode == FEM_KAPPA_QP)
+            hipLaunchKernelGGL((k_dg_apply<K, T, true, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
+        else
+            hipLaunchKernelGGL((k_dg_apply<K, T, true, false>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
+    } else {
+        if (a.cvol || a.nl_pow)
             hipLaunchKernelGGL((k_dg_apply<K, T, false, true, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
-    } else if (a.kappa_mode == FEM_KAPPA_QP)
-        hipLaunchKernelGGL((k_dg_apply<K, T, MF, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
-    else
-        hipLaunchKernelGGL((k_dg_apply<K, T, MF, false>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
+        else
+            hipLaunchKernelGGL((k_dg_apply<K, T, false, true>), dim3(nb), dim3(A::WG), 0, s, a, u, w, skip, dot);
+    }
     FEM_HIP(hipGetLastError());
 }
 
@@ -1274,6 +1277,7 @@ __global__ void k_dg_block_setup(const DGArgs<double> a, int K, TO *__restrict__
                         cm += tb.w[qx] * tb.w[qy] * tb.w[qz] * v;
                         cmax = fmax(cmax, v);
                     }
+        if (a.ccell) cm += a.ccell[e];
         shift = (a.c + (a.cvol && bound ? cmax : cm)) * a.h[0] * a.h[1] * a.h[2];
     }
     for (int r = 0; r < K; ++r) {

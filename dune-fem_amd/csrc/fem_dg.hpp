@@ -66,6 +66,9 @@ struct DGArgs {
     const T *cvol;
     T nl_coef;
     int nl_pow;
+    // a reaction per element added to c, [E], may be null (the coarse levels of
+    // a multigrid; kappa constant per element only)
+    const T *ccell;
     const Tab1D<T> *tab;   // device copy of the 1D tables
     // per direction d, set on the host: beta / h_d, the face area of the
     // faces normal to d, |K| / h_d^2, b_d h_d, max(b_d, 0), max(-b_d, 0)
@@ -78,8 +81,8 @@ struct DGArgs {
     int slabs, rpb, ty;
     UDiv dv_slab, dv_zrow, dv_rpb;   // by rpb ty nz, rpb ty, rpb
     // of the modal kernel: 2 |K| / h^2, 2 |F| b, |F| beta / (2 h), |F| / (2 h),
-    // |F| max(b, 0), |F| max(-b, 0) per direction, and c |K|
-    T m_kv[3], m_ad[3], m_pen[3], m_w[3], m_bp[3], m_bm[3], m_c;
+    // |F| max(b, 0), |F| max(-b, 0) per direction, c |K| and |K|
+    T m_kv[3], m_ad[3], m_pen[3], m_w[3], m_bp[3], m_bm[3], m_c, m_vol;
     ModalRows mr;
     ModalTile mt;   // traversal of the modal kernel (fem_dg_modal.hip)
 };
@@ -94,6 +97,17 @@ struct DGSmooth {
     const T *lam = nullptr;
     T omega = T(0);
     T *xout = nullptr;
+};
+
+// the residual r - A u in the form a coarser level takes: on the modes
+// a, b, c < kc (rc [E][kc^3], the next DG level), or at Q1 as the trilinear
+// functionals at each element's corners (corners [E][8], the vertex level)
+template <typename T>
+struct DGResidual {
+    const T *r = nullptr;
+    T *rc = nullptr;
+    int kc = 0;
+    double *corners = nullptr;
 };
 
 // elements per workgroup of the apply for k points per direction
@@ -116,7 +130,8 @@ inline void dg_derived(DGArgs<T> &a, int k)
     }
     a.mt = dg_modal_tile(k, a.n);
     a.mr = dg_modal_rows(k, a.n);
-    a.m_c = a.c * a.h[0] * a.h[1] * a.h[2];
+    a.m_vol = a.h[0] * a.h[1] * a.h[2];
+    a.m_c = a.c * a.m_vol;
     for (int d = 0; d < 3; ++d) {
         const int t1 = (d == 0) ? 1 : 0, t2 = (d == 2) ? 1 : 2;
         a.pen[d] = a.beta * a.ih[d];
@@ -134,14 +149,19 @@ inline void dg_derived(DGArgs<T> &a, int k)
     }
 }
 
-// the modal kernel (fem_dg_modal.hip): kappa constant per element and no
-// reaction beyond c.  The apply, and the damped block-Jacobi sweep of
-// dg_smooth_*; `dot` as in dg_apply_*, dg_modal_blocks(k, n) entries
-int64_t dg_modal_blocks(int k, const int *n);
+// the modal kernels (fem_dg_modal.hip): kappa constant per element.  The
+// apply, the residual for a coarser level, and the damped block-Jacobi sweep;
+// `dot` as in dg_apply_*, dg_modal_blocks(k, n, reaction) entries (reaction:
+// at the volume points)
+int64_t dg_modal_blocks(int k, const int *n, bool reaction);
 void dg_modal_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                         double *dot);
 void dg_modal_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                         double *dot);
+void dg_modal_residual_f64(const DGArgs<double> &a, int k, const double *u, const DGResidual<double> &rs,
+                           const int *skip, hipStream_t s);
+void dg_modal_residual_f32(const DGArgs<float> &a, int k, const float *u, const DGResidual<float> &rs, const int *skip,
+                           hipStream_t s);
 void dg_modal_smooth_f64(const DGArgs<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
                          hipStream_t s);
 void dg_modal_smooth_f32(const DGArgs<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
@@ -149,7 +169,7 @@ void dg_modal_smooth_f32(const DGArgs<float> &a, int k, const float *u, const DG
 template <typename T>
 inline bool dg_is_modal(const DGArgs<T> &a)
 {
-    return a.kappa_mode != FEM_KAPPA_QP && !a.cvol && !a.nl_pow;
+    return a.kappa_mode != FEM_KAPPA_QP;
 }
 
 // w = A u.  `skip` (device flag, may be null): when *skip != 0 the launch

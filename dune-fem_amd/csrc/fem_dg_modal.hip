@@ -149,7 +149,9 @@ __device__ __forceinline__ void modal_dot(double acc, double *__restrict__ dot)
     }
 }
 
-// w = A u.  A workgroup holds a tile of elements in y and z (K x K lanes
+// w = A u; RES: with a reaction per element, and (rs.rc) the residual r - A u on
+// the low modes a, b, c < kc in its place, the restriction to the next DG level
+// (compiled apart: the apply keeps its 128 registers at Q4).  A workgroup holds a tile of elements in y and z (K x K lanes
 // each) and walks along x.  What bounds it is the traffic to memory and the
 // loads in flight, so every value is fetched about once per tile:
 //   * lane (b, c) loads the x pencils, whose K loads are K^2 contiguous values
@@ -162,10 +164,10 @@ __device__ __forceinline__ void modal_dot(double acc, double *__restrict__ dot)
 // six neighbour pencils from memory (7 loads of a vector through the vector
 // caches), 565 us so (3.1 TB/s of vectors read and written; 2.2 GB moved per
 // apply).  Q3 at 64^3: 131, 93, 80 us; Q2 at 96^3: 287, 183, 144 us.
-template <int K, typename T>
+template <int K, typename T, bool RES>
 __global__ void __launch_bounds__(MShape<K>::NT)
     k_dg_modal(const DGArgs<T> a, const T *__restrict__ u, T *__restrict__ w, const int *__restrict__ skip,
-               double *__restrict__ dot)
+               double *__restrict__ dot, const DGResidual<T> rs)
 {
     using S = MShape<K>;
     constexpr int K2 = S::K2, K3 = S::K3, EPB = S::EPB, SZ = S::SZ, NT = S::NT;
@@ -344,11 +346,28 @@ __global__ void __launch_bounds__(MShape<K>::NT)
             if (a.c != T(0))
 #pragma unroll
                 for (int m = 0; m < K; ++m) rx[m] = fma(a.m_c, v[m], rx[m]);
+            if constexpr (RES)
+                if (a.ccell) {
+                    const T cm = a.m_vol * a.ccell[valid ? e + x - x0 : 0];
+#pragma unroll
+                    for (int m = 0; m < K; ++m) rx[m] = fma(cm, v[m], rx[m]);
+                }
         }
         wave_lds_sync();
         if (valid)
 #pragma unroll
             for (int m = 0; m < K; ++m) rx[m] += B[L(m, i, j)];
+        if (RES && rs.rc) {
+            const int kc = rs.kc;
+            if (valid && i < kc && j < kc) {
+                const size_t ex = (size_t)(e + x - x0);
+                const T *re = rs.r + ex * K3 + lane;
+                T *ce = rs.rc + ex * (kc * kc * kc) + i * kc + j;
+#pragma unroll
+                for (int m = 0; m < K; ++m)
+                    if (m < kc) ce[m * kc * kc] = re[m * K2] - rx[m];
+            }
+        } else {
             if (valid) {
                 T *we = reinterpret_cast<T *>(reinterpret_cast<char *>(const_cast<T *>(ue)) + uw);
 #pragma unroll
@@ -357,6 +376,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
                     acc += (double)v[m] * (double)rx[m];
                 }
             }
+        }
 #pragma unroll
         for (int m = 0; m < K; ++m) {
             v[m] = vn[m];
@@ -369,21 +389,56 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     if (dot) modal_dot<NT>(acc, dot);
 }
 
+// 1D passes between the modes of a pencil and its Gauss points, by the parity
+// of the basis on the symmetric points: B[K-1-q][a] = (-1)^a B[q][a]
+template <int K, typename T>
+__device__ __forceinline__ void to_points(const Tab1D<T> &tb, const T (&v)[K], T (&out)[K])
+{
+#pragma unroll
+    for (int q = 0; q < (K + 1) / 2; ++q) {
+        T ev = 0, od = 0;
+#pragma unroll
+        for (int a = 0; a < K; ++a) {
+            if (a & 1) od = fma(tb.B[q][a], v[a], od);
+            else ev = fma(tb.B[q][a], v[a], ev);
+        }
+        out[q] = ev + od;
+        if (q != K - 1 - q) out[K - 1 - q] = ev - od;
+    }
+}
+
+template <int K, typename T>
+__device__ __forceinline__ void from_points(const Tab1D<T> &tb, const T (&v)[K], T (&out)[K])
+{
+#pragma unroll
+    for (int a = 0; a < K; ++a) {
+        T s = (K & 1) ? tb.B[K / 2][a] * v[K / 2] : T(0);
+#pragma unroll
+        for (int q = 0; q < K / 2; ++q) s = fma(tb.B[q][a], (a & 1) ? v[q] - v[K - 1 - q] : v[q] + v[K - 1 - q], s);
+        out[a] = s;
+    }
+}
+
 // The same lines without the walk: a wavefront holds EPW elements of an x-row
-// and every lane loads the six neighbour pencils itself.  SM: the sweep
-// xout = u + omega B^-1 (r - A u) of a multigrid level, with the element-block
-// inverse in the same pass; otherwise w = A u.  The sweep needs the registers
-// and the LDS of a walk for the element block (48^3 Q3 FP64: the V-cycle with
-// a walking sweep 458 us, with this one 415 us), and at Q1 a step of a walk is
-// too short for its barriers (48^3: FP64 apply 8.6 us against 10.4 us, FP32
-// 6.3 us against 7.5 us).
-template <int K, typename T, bool SM>
+// and every lane loads the six neighbour pencils itself.
+//   SM: the sweep xout = u + omega B^-1 (r - A u) of a multigrid level, with the
+//     element-block inverse in the same pass; otherwise w = A u, the residual on
+//     the low modes (rs.rc), or at Q1 the residual's trilinear functionals at
+//     the element's corners (rs.corners, see fem_mg.hip).
+//   RX: the reaction at the volume points (cvol and the law), by three passes to
+//     the Gauss points and back.
+// The sweep needs the registers and the LDS of a walk for the element block
+// (48^3 Q3 FP64: the V-cycle with a walking sweep 458 us, with this one 415 us),
+// and at Q1 a step of a walk is too short for its barriers (48^3: FP64 apply
+// 8.6 us against 10.4 us, FP32 6.3 us against 7.5 us).
+template <int K, typename T, bool SM, bool RX>
 __global__ void __launch_bounds__(256)
     k_dg_rows(const DGArgs<T> a, const T *__restrict__ u, T *__restrict__ w, const int *__restrict__ skip,
-              double *__restrict__ dot, const DGSmooth<T> sm)
+              double *__restrict__ dot, const DGSmooth<T> sm, const DGResidual<T> rs)
 {
     using S = MShape<K>;
     constexpr int K2 = S::K2, K3 = S::K3, EPW = S::EPW, R = 4, SZ = S::SZ;
+    constexpr int KC = (K + 1) / 2;   // modes of the next DG level: order (K - 1) / 2
     if (skip && *skip) return;
     __shared__ T smem[R * EPW * (SZ + (SM ? S::SQ : 0))];
     const int g = threadIdx.x >> 6, tid = threadIdx.x & 63;
@@ -413,10 +468,15 @@ __global__ void __launch_bounds__(256)
     const int stride[3] = { 1, nx, nx * ny };
     T *const A = smem + (g * EPW + el) * SZ, *const Q = smem + R * EPW * SZ + (g * EPW + el) * S::SQ;
     auto L = [&](int a_, int b_, int c_) { return midx<K>(a_, b_, c_); };
-    const T *ue = u + (size_t)e * K3;
-    T v[K], rr[K];   // own x pencil: lane (b, c)
+    // the pencil of element en along d through this lane
+    auto pencil = [&](int d, int en, T (&n)[K]) {
+        const T *un = u + (size_t)en * K3;
 #pragma unroll
-    for (int m = 0; m < K; ++m) v[m] = ue[m * K2 + lane];
+        for (int m = 0; m < K; ++m)
+            n[m] = un[d == 0 ? m * K2 + lane : d == 1 ? i * K2 + m * K + j : i * K2 + j * K + m];
+    };
+    T v[K], rr[K];   // own x pencil: lane (b, c)
+    pencil(0, e, v);
     bool has[3][2];
     const bool kcell = a.kappa_mode == FEM_KAPPA_CELL;
     const T kin = kcell ? a.kcell[e] : a.kappa_const;
@@ -428,17 +488,18 @@ __global__ void __launch_bounds__(256)
             has[d][s] = s ? ec[d] + 1 < a.n[d] : ec[d] > 0;
             const int en = has[d][s] ? e + (s ? stride[d] : -stride[d]) : e;
             ks[d][s] = kcell ? a.kcell[en] : kin;
-            const T *un = u + (size_t)en * K3;
             T n[K];
-#pragma unroll
-            for (int m = 0; m < K; ++m)
-                n[m] = un[d == 0 ? m * K2 + lane : d == 1 ? i * K2 + m * K + j : i * K2 + j * K + m];
+            pencil(d, en, n);
             if (s) nbr_trace<K, true>(n, nv[d][s], nd[d][s]);
             else nbr_trace<K, false>(n, nv[d][s], nd[d][s]);
             nv[d][s] = has[d][s] ? nv[d][s] : T(0);
             nd[d][s] = has[d][s] ? nd[d][s] : T(0);
         }
     }
+    T cq[K];
+    if constexpr (RX)
+#pragma unroll
+        for (int q = 0; q < K; ++q) cq[q] = a.cvol ? a.cvol[(size_t)e * K3 + i + K * j + K2 * q] : T(0);
     if constexpr (SM) {
         const T *re = sm.r + (size_t)e * K3, *Qg = sm.Q + (size_t)e * 3 * K2, *lg = sm.lam + (size_t)e * 3 * K;
 #pragma unroll
@@ -473,10 +534,93 @@ __global__ void __launch_bounds__(256)
     if (a.c != T(0))
 #pragma unroll
         for (int m = 0; m < K; ++m) rx[m] = fma(a.m_c, v[m], rx[m]);
+    if (a.ccell) {
+        const T cm = a.m_vol * a.ccell[e];
+#pragma unroll
+        for (int m = 0; m < K; ++m) rx[m] = fma(cm, v[m], rx[m]);
+    }
     wave_lds_sync();
 #pragma unroll
     for (int m = 0; m < K; ++m) rx[m] += A[L(m, i, j)];
+    if constexpr (RX) {
+        // int (cvol + coef u^pw) u v
+        const Tab1D<T> &tb = *a.tab;
+        T f[K], h[K];
+        auto put = [&](int d, const T (&x)[K]) {
+            if (wr)
+#pragma unroll
+                for (int m = 0; m < K; ++m) A[d == 0 ? L(m, i, j) : d == 1 ? L(i, m, j) : L(i, j, m)] = x[m];
+            wave_lds_sync();
+        };
+        auto get = [&](int d, T (&x)[K]) {
+#pragma unroll
+            for (int m = 0; m < K; ++m) x[m] = A[d == 0 ? L(m, i, j) : d == 1 ? L(i, m, j) : L(i, j, m)];
+            wave_lds_sync();
+        };
+        to_points<K>(tb, v, f);
+        wave_lds_sync();
+        put(0, f);
+        get(1, f);
+        to_points<K>(tb, f, h);
+        put(1, h);
+        get(2, f);
+        to_points<K>(tb, f, h);
+        const T wij = a.m_vol * tb.w[i] * tb.w[j];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            T c = cq[k];
+            if (a.nl_pow) {
+                T pw = a.nl_coef;
+                for (int n = 0; n < a.nl_pow; ++n) pw *= h[k];
+                c += pw;
+            }
+            f[k] = wij * tb.w[k] * c * h[k];
+        }
+        from_points<K>(tb, f, h);
+        put(2, h);
+        get(1, f);
+        from_points<K>(tb, f, h);
+        put(1, h);
+        get(0, f);
+        from_points<K>(tb, f, h);
+#pragma unroll
+        for (int m = 0; m < K; ++m) rx[m] += h[m];
+    }
     if constexpr (!SM) {
+        if (rs.rc) {
+            const int kc = rs.kc;
+            if (active && i < kc && j < kc) {
+                const T *re = rs.r + (size_t)e * K3 + lane;
+                T *ce = rs.rc + (size_t)e * (kc * kc * kc) + i * kc + j;
+#pragma unroll
+                for (int m = 0; m < K; ++m)
+                    if (m < kc) ce[m * kc * kc] = re[m * K2] - rx[m];
+            }
+            return;
+        }
+        if constexpr (K == 2)
+            if (rs.corners) {
+                // the residual's modes in FP64, then this lane's two corners
+                // (0, i, j) and (1, i, j)
+                __shared__ double cs[R * EPW * 8];
+                double *C = cs + (g * EPW + el) * 8;
+                const T *re = rs.r + (size_t)e * K3 + lane;
+#pragma unroll
+                for (int m = 0; m < 2; ++m) C[m * 4 + lane] = (double)re[m * K2] - (double)rx[m];
+                wave_lds_sync();
+                const double s1 = 0.28867513459481287;   // 1 / (2 sqrt 3)
+                const double ti = i ? s1 : -s1, tj = j ? s1 : -s1;
+                double x[2];
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    x[m] = 0.5 * (0.5 * C[m * 4] + tj * C[m * 4 + 1]) + ti * (0.5 * C[m * 4 + 2] + tj * C[m * 4 + 3]);
+                if (active) {
+                    double *ce = rs.corners + (size_t)e * 8 + 2 * i + 4 * j;
+                    ce[0] = 0.5 * x[0] - s1 * x[1];
+                    ce[1] = 0.5 * x[0] + s1 * x[1];
+                }
+                return;
+            }
         double acc = 0;
         if (active) {
             T *we = w + (size_t)e * K3 + lane;
@@ -556,24 +700,42 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-template <int K, typename T, bool SM>
-void launch_rows(const DGArgs<T> &a, const T *u, T *w, const DGSmooth<T> &sm, const int *skip, hipStream_t s,
-                 double *dot)
+template <int K, typename T, bool SM, bool RX>
+void launch_rows(const DGArgs<T> &a, const T *u, T *w, const DGSmooth<T> &sm, const DGResidual<T> &rs, const int *skip,
+                 hipStream_t s, double *dot)
 {
-    hipLaunchKernelGGL((k_dg_rows<K, T, SM>), dim3((unsigned)a.mr.blocks), dim3(256), 0, s, a, u, w, skip, dot, sm);
+    hipLaunchKernelGGL((k_dg_rows<K, T, SM, RX>), dim3((unsigned)a.mr.blocks), dim3(256), 0, s, a, u, w, skip, dot,
+                       sm, rs);
 }
 
 template <int K, typename T>
-void launch_apply(const DGArgs<T> &a, const T *u, T *w, const int *skip, hipStream_t s, double *dot)
+void launch_apply(const DGArgs<T> &a, const T *u, T *w, const DGResidual<T> &rs, const int *skip, hipStream_t s,
+                  double *dot)
 {
-    if constexpr (K == 2) {
-        launch_rows<K, T, false>(a, u, w, DGSmooth<T>{}, skip, s, dot);
+    if (a.cvol || a.nl_pow) {
+        launch_rows<K, T, false, true>(a, u, w, DGSmooth<T>{}, rs, skip, s, dot);
+    } else if constexpr (K == 2) {
+        launch_rows<K, T, false, false>(a, u, w, DGSmooth<T>{}, rs, skip, s, dot);
     } else {
         using S = MShape<K>;
         const ModalTile &t = a.mt;
         const size_t lds = sizeof(T) * ((size_t)(t.slots + 1 + S::EPB) * S::SZ + (size_t)t.slots * t.ks);
-        hipLaunchKernelGGL((k_dg_modal<K, T>), dim3((unsigned)t.blocks), dim3(S::NT), lds, s, a, u, w, skip, dot);
+        if (rs.rc || a.ccell)
+            hipLaunchKernelGGL((k_dg_modal<K, T, true>), dim3((unsigned)t.blocks), dim3(S::NT), lds, s, a, u, w, skip, dot,
+                               rs);
+        else
+            hipLaunchKernelGGL((k_dg_modal<K, T, false>), dim3((unsigned)t.blocks), dim3(S::NT), lds, s, a, u, w, skip, dot,
+                               rs);
     }
+}
+
+template <int K, typename T>
+void launch_sweep(const DGArgs<T> &a, const T *u, const DGSmooth<T> &sm, const int *skip, hipStream_t s)
+{
+    const bool rx = a.cvol || a.nl_pow;
+    const DGResidual<T> rs;
+    if (rx) launch_rows<K, T, true, true>(a, u, nullptr, sm, rs, skip, s, nullptr);
+    else launch_rows<K, T, true, false>(a, u, nullptr, sm, rs, skip, s, nullptr);
 }
 
 #define MODAL_SWITCH(CALL)                                                             \
@@ -594,10 +756,12 @@ void modal_check(const DGArgs<T> &a, int k)
 }
 
 template <typename T>
-void modal_apply(const DGArgs<T> &a, int k, const T *u, T *w, const int *skip, hipStream_t s, double *dot)
+void modal_apply(const DGArgs<T> &a, int k, const T *u, T *w, const DGResidual<T> &rs, const int *skip, hipStream_t s,
+                 double *dot)
 {
     modal_check(a, k);
-#define CALL(KK) launch_apply<KK, T>(a, u, w, skip, s, dot)
+    FEM_CHECK(!rs.corners || k == 2, FEM_ERR_ARG, "corner functionals: Q1 only");
+#define CALL(KK) launch_apply<KK, T>(a, u, w, rs, skip, s, dot)
     MODAL_SWITCH(CALL);
 #undef CALL
 }
@@ -609,7 +773,7 @@ void modal_smooth(const DGArgs<T> &a, int k, const T *u, const DGSmooth<T> &sm, 
     FEM_CHECK(dg_is_modal(a), FEM_ERR_UNSUPPORTED, "smoothing sweep: cellwise or constant kappa");
     FEM_CHECK(sm.r && sm.Q && sm.lam && sm.xout && sm.xout != u, FEM_ERR_ARG,
               "smoothing sweep: r, eigen data and an output other than the input");
-#define CALL(KK) launch_rows<KK, T, true>(a, u, (T *)nullptr, sm, skip, s, (double *)nullptr)
+#define CALL(KK) launch_sweep<KK, T>(a, u, sm, skip, s)
     MODAL_SWITCH(CALL);
 #undef CALL
 }
@@ -679,9 +843,9 @@ ModalRows dg_modal_rows(int k, const int *n)
     return r;
 }
 
-int64_t dg_modal_blocks(int k, const int *n)
+int64_t dg_modal_blocks(int k, const int *n, bool reaction)
 {
-    return k == 2 ? dg_modal_rows(k, n).blocks : dg_modal_tile(k, n).blocks;
+    return k == 2 || reaction ? dg_modal_rows(k, n).blocks : dg_modal_tile(k, n).blocks;
 }
 
 int64_t dg_bj_blocks(int k, int64_t E)
@@ -707,12 +871,22 @@ template void dg_block_apply<float>(int, int64_t, const float *, const float *, 
 void dg_modal_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                         double *dot)
 {
-    modal_apply<double>(a, k, u, w, skip, s, dot);
+    modal_apply<double>(a, k, u, w, DGResidual<double>{}, skip, s, dot);
 }
 void dg_modal_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                         double *dot)
 {
-    modal_apply<float>(a, k, u, w, skip, s, dot);
+    modal_apply<float>(a, k, u, w, DGResidual<float>{}, skip, s, dot);
+}
+void dg_modal_residual_f64(const DGArgs<double> &a, int k, const double *u, const DGResidual<double> &rs,
+                           const int *skip, hipStream_t s)
+{
+    modal_apply<double>(a, k, u, nullptr, rs, skip, s, nullptr);
+}
+void dg_modal_residual_f32(const DGArgs<float> &a, int k, const float *u, const DGResidual<float> &rs, const int *skip,
+                           hipStream_t s)
+{
+    modal_apply<float>(a, k, u, nullptr, rs, skip, s, nullptr);
 }
 void dg_modal_smooth_f64(const DGArgs<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
                          hipStream_t s)

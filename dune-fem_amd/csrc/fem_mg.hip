@@ -53,25 +53,9 @@ inline unsigned mg_grid(int64_t n) { return grid_for(n, MGT, 16384); }
     if (skip && *skip) return
 
 // ---- DG levels ----------------------------------------------------------------------
-// rc = (r - t) on the modes a, b, c < Kc (local index a Kf^2 + b Kf + c)
-template <typename T>
-__global__ void k_mg_restrict_modes(int64_t E, int Kf, int Kc, const T *__restrict__ r, const T *__restrict__ t,
-                                    T *__restrict__ rc, const int *__restrict__ skip)
-{
-    MG_SKIP;
-    const int Kc3 = Kc * Kc * Kc, Kf3 = Kf * Kf * Kf;
-    const int64_t n = E * Kc3;
-    const bool narrow = n < (int64_t(1) << 31);
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t e = narrow ? (int64_t)((unsigned)q / (unsigned)Kc3) : q / Kc3;
-        const int l = (int)(q - e * Kc3);
-        const int a = l / (Kc * Kc), b = (l / Kc) % Kc, c = l % Kc;
-        const int64_t f = e * Kf3 + a * Kf * Kf + b * Kf + c;
-        rc[q] = r[f] - t[f];
-    }
-}
-
-// xf += P xc (embedding of the low modes)
+// xf += P xc (embedding of the low modes), a pass of its own: a sweep that adds
+// P xc as it reads its seven pencils came out slower or the same (V-cycle 64^3
+// Q4 FP32 1230 us against 1172 us, 48^3 Q3 FP64 392 us against 366 us)
 template <typename T>
 __global__ void k_mg_prolong_modes(int64_t E, int Kf, int Kc, const T *__restrict__ xc, T *__restrict__ xf,
                                    const int *__restrict__ skip)
@@ -96,30 +80,12 @@ __device__ __forceinline__ double tq1(int a, int i)
     return a == 0 ? 0.5 : (i ? 0.28867513459481287 : -0.28867513459481287);   // 1 / (2 sqrt 3)
 }
 
-// rv = P_c^T (r - t) (t may be null), in two passes.  First, per element,
-// the trilinear functional of its Q1 modes at each of its 8 vertices,
-// c[e][q] with q = i + 2 j + 4 k for the vertex (cx + i, cy + j, cz + k),
-// kept in FP64; then per vertex the sum over the (up to) 8 elements around
-// it.  A single per-vertex pass would gather 8 x 8 mode values per vertex.
-template <typename T>
-__global__ void k_mg_dg1_corners(int64_t E, const T *__restrict__ r, const T *__restrict__ t,
-                                 double *__restrict__ c, const int *__restrict__ skip)
-{
-    MG_SKIP;
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < E * 8; q += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t e = q >> 3;
-        const int cq = (int)(q & 7), i = cq & 1, j = (cq >> 1) & 1, k = cq >> 2;
-        double acc = 0;
-#pragma unroll
-        for (int l = 0; l < 8; ++l) {
-            const int a = l >> 2, b = (l >> 1) & 1, cc = l & 1;
-            const double val = (double)r[e * 8 + l] - (t ? (double)t[e * 8 + l] : 0.0);
-            acc = fma(tq1(a, i) * tq1(b, j) * tq1(cc, k), val, acc);
-        }
-        c[q] = acc;
-    }
-}
-
+// rv = P_c^T (r - A x), in two passes.  First, per element, the trilinear
+// functional of the residual's Q1 modes at each of its 8 vertices, c[e][q]
+// with q = i + 2 j + 4 k for the vertex (cx + i, cy + j, cz + k), kept in
+// FP64, by the Q1 level's residual pass (fem_dg_modal.hip); then per vertex
+// the sum over the (up to) 8 elements around it.  A single per-vertex pass
+// would gather 8 x 8 mode values per vertex.
 template <typename T>
 __global__ void k_mg_corners_to_vertex(int nx, int ny, int nz, const double *__restrict__ c, T *__restrict__ rv,
                                        const int *__restrict__ skip)
@@ -141,17 +107,6 @@ __global__ void k_mg_corners_to_vertex(int nx, int ny, int nz, const double *__r
         }
         rv[v] = (T)acc;
     }
-}
-
-template <typename T>
-void dg1_to_vertex(const int *n, const T *r, const T *t, double *corners, T *rv, const int *skip, hipStream_t s)
-{
-    const int64_t E = (int64_t)n[0] * n[1] * n[2];
-    const int64_t V = (int64_t)(n[0] + 1) * (n[1] + 1) * (n[2] + 1);
-    hipLaunchKernelGGL(k_mg_dg1_corners<T>, dim3(mg_grid(E * 8)), dim3(MGT), 0, s, E, r, t, corners, skip);
-    hipLaunchKernelGGL(k_mg_corners_to_vertex<T>, dim3(mg_grid(V)), dim3(MGT), 0, s, n[0], n[1], n[2],
-                       (const double *)corners, rv, skip);
-    FEM_HIP(hipGetLastError());
 }
 
 // x += P_c xv: the Q1 modes of the trilinear interpolant of the vertex values
@@ -181,31 +136,66 @@ struct VDims {
     int n[3];
 };
 
-// t = sg * (A x) + (r ? r : 0) with sg = -1 (residual r - A x) or +1 (A x,
-// r null).  The stencil is stored by offset, A[s * V + v] with s = (dx+1) +
-// 3 (dy+1) + 9 (dz+1), so each of the 27 coefficient loads is coalesced; the
-// 27 terms are unrolled, and a neighbour outside the lattice reads x[v] with
-// weight 0, so all loads are issued together.
+// The stencil is stored by offset, A[s * V + v] with s = (dx+1) + 3 (dy+1) +
+// 9 (dz+1), so each of the 27 coefficient loads is coalesced; a neighbour outside
+// the lattice reads v itself with weight 0, so all loads are issued together.
+//
+// Vertex sweeps: three lanes per vertex, one per z-plane of its stencil (the
+// block is VS vertices by 3 planes, the plane sums meet in LDS).  The levels are
+// small (33^3 vertices and fewer behind a 32^3 mesh), so what bounds them is the
+// chain of loads of one vertex and the workgroups in flight, not the bandwidth:
+// with a thread per vertex the 27 + 27 loads of a sweep took up to 256 registers
+// and 33^3 vertices made 141 workgroups (FP32 hierarchy of 33^3 vertices: down
+// 8.6 us, up 9.8 us; V-cycle 48^3 Q1 FP64 143 us, now 122 us).
+constexpr int VS = 64;
+
+// the sum over the three planes of a vertex, valid in plane 1
 template <typename T>
-__global__ void k_mg_v_apply(VDims d, const T *__restrict__ A, const T *__restrict__ x, const T *__restrict__ r,
-                             T *__restrict__ t, int sg, const int *__restrict__ skip)
+__device__ __forceinline__ T plane_sum(T (*part)[VS], T acc)
+{
+    const int i = threadIdx.x, p = threadIdx.y;
+    __syncthreads();
+    if (p != 1) part[p >> 1][i] = acc;
+    __syncthreads();
+    return p == 1 ? (part[0][i] + acc) + part[1][i] : T(0);
+}
+
+// down: x0 = omega dinv r and t = r - A x0 (a Jacobi sweep from zero and the
+// residual it leaves) in one pass: the neighbours' x0 is formed from r
+template <typename T>
+__global__ void __launch_bounds__(3 * VS)
+    k_mg_v_down(VDims d, const T *__restrict__ A, const T *__restrict__ dinv, const T *__restrict__ r,
+                T *__restrict__ x0, T *__restrict__ t, T omega, const int *__restrict__ skip)
 {
     MG_SKIP;
+    __shared__ T part[2][VS];
     const int64_t V = (int64_t)d.n[0] * d.n[1] * d.n[2];
     const int64_t sy = d.n[0], sz = (int64_t)d.n[0] * d.n[1];
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < V; v += (int64_t)gridDim.x * blockDim.x) {
+    const int dz = (int)threadIdx.y - 1;
+    for (int64_t v0 = blockIdx.x * (int64_t)VS; v0 < V; v0 += (int64_t)gridDim.x * VS) {
+        const bool ok = v0 + threadIdx.x < V;
+        const int64_t v = ok ? v0 + threadIdx.x : V - 1;
         const int vx = (int)(v % d.n[0]), vy = (int)((v / d.n[0]) % d.n[1]), vz = (int)(v / sz);
-        T acc = 0;
+        const bool inz = vz + dz >= 0 && vz + dz < d.n[2];
+        T acc = 0, xv = 0, rv = 0;
 #pragma unroll
-        for (int s = 0; s < 27; ++s) {
-            const int dx = s % 3 - 1, dy = (s / 3) % 3 - 1, dz = s / 9 - 1;
-            const bool in = vx + dx >= 0 && vx + dx < d.n[0] && vy + dy >= 0 && vy + dy < d.n[1] && vz + dz >= 0 &&
-                            vz + dz < d.n[2];
-            const T a = A[s * V + v];
-            const T xv = x[in ? v + dx + dy * sy + dz * sz : v];
-            acc = fma(in ? a : T(0), xv, acc);
+        for (int q = 0; q < 9; ++q) {
+            const int dx = q % 3 - 1, dy = q / 3 - 1;
+            const bool in = inz && vx + dx >= 0 && vx + dx < d.n[0] && vy + dy >= 0 && vy + dy < d.n[1];
+            const T a = A[(threadIdx.y * 9 + q) * V + v];
+            const int64_t w = in ? v + dx + dy * sy + dz * sz : v;
+            const T rw = r[w], xw = omega * dinv[w] * rw;
+            if (q == 4) {
+                rv = rw;   // (of the vertex itself in plane 1)
+                xv = xw;
+            }
+            acc = fma(in ? a : T(0), xw, acc);
         }
-        t[v] = (r ? r[v] : T(0)) + (sg < 0 ? -acc : acc);
+        acc = plane_sum(part, acc);
+        if (threadIdx.y == 1 && ok) {
+            x0[v] = xv;
+            t[v] = rv - acc;
+        }
     }
 }
 
@@ -217,17 +207,6 @@ __global__ void k_mg_by_offset(int64_t V, const double *__restrict__ Av, double 
         const int s = (int)(q - v * 27);
         As[s * V + v] = Av[q];
     }
-}
-
-// mode 0: x = omega dinv r;  mode 1: x += omega dinv t (t = r - A x)
-template <typename T>
-__global__ void k_mg_v_jacobi(int64_t V, const T *__restrict__ dinv, const T *__restrict__ r,
-                              const T *__restrict__ t, T *__restrict__ x, T omega, int mode,
-                              const int *__restrict__ skip)
-{
-    MG_SKIP;
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < V; v += (int64_t)gridDim.x * blockDim.x)
-        x[v] = mode ? x[v] + omega * dinv[v] * t[v] : omega * dinv[v] * r[v];
 }
 
 // 1D trilinear interpolation from the coarse vertices (fine positions 0, 2,
@@ -281,36 +260,80 @@ __global__ void k_mg_v_restrict(VDims f, VDims cdim, const T *__restrict__ tf, T
     }
 }
 
-// xf += P xc
+// up: x = x0 + P xc (the coarse correction), then the Jacobi sweep
+// xout = x + omega dinv (r - A x), in one pass: a thread forms x on the 3 x 3
+// vertices of its plane.  A plane has two candidate coarse planes (the second
+// weighs in where the plane is odd), and the three vertices of a line have three
+// coarse ones; interpolated in FP64, direction by direction.
 template <typename T>
-__global__ void k_mg_v_prolong(VDims f, VDims cdim, const T *__restrict__ xc, T *__restrict__ xf,
-                               const int *__restrict__ skip)
+__global__ void __launch_bounds__(3 * VS)
+    k_mg_v_up(VDims f, VDims cdim, const T *__restrict__ A, const T *__restrict__ dinv, const T *__restrict__ r,
+              const T *__restrict__ x0, const T *__restrict__ xc, T *__restrict__ xout, T omega,
+              const int *__restrict__ skip)
 {
     MG_SKIP;
-    const int64_t Vf = (int64_t)f.n[0] * f.n[1] * f.n[2];
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < Vf; v += (int64_t)gridDim.x * blockDim.x) {
-        const int ix = (int)(v % f.n[0]), iy = (int)((v / f.n[0]) % f.n[1]), iz = (int)(v / ((int64_t)f.n[0] * f.n[1]));
-        double acc = 0;
-        for (int c = 0; c < 2; ++c) {
-            const int Jz = (iz >> 1) + c;
-            if (Jz >= cdim.n[2]) continue;
-            const double wz = w1(iz, Jz, f.n[2], cdim.n[2]);
-            if (wz == 0.0) continue;
-            for (int b = 0; b < 2; ++b) {
-                const int Jy = (iy >> 1) + b;
-                if (Jy >= cdim.n[1]) continue;
-                const double wy = w1(iy, Jy, f.n[1], cdim.n[1]);
-                if (wy == 0.0) continue;
-                for (int a = 0; a < 2; ++a) {
-                    const int Jx = (ix >> 1) + a;
-                    if (Jx >= cdim.n[0]) continue;
-                    const double wx = w1(ix, Jx, f.n[0], cdim.n[0]);
-                    if (wx == 0.0) continue;
-                    acc += wx * wy * wz * (double)xc[Jx + (int64_t)cdim.n[0] * (Jy + (int64_t)cdim.n[1] * Jz)];
+    __shared__ T part[2][VS];
+    const int64_t V = (int64_t)f.n[0] * f.n[1] * f.n[2];
+    const int64_t sy = f.n[0], sz = (int64_t)f.n[0] * f.n[1];
+    const int dz = (int)threadIdx.y - 1;
+    for (int64_t v0 = blockIdx.x * (int64_t)VS; v0 < V; v0 += (int64_t)gridDim.x * VS) {
+        const bool ok = v0 + threadIdx.x < V;
+        const int64_t v = ok ? v0 + threadIdx.x : V - 1;
+        const int pos[3] = { (int)(v % f.n[0]), (int)((v / f.n[0]) % f.n[1]), (int)(v / sz) };
+        const int iz = pos[2] + dz;
+        const bool inz = iz >= 0 && iz < f.n[2];
+        // x0 and the stencil of the plane
+        T a[9], xo[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const int dx = q % 3 - 1, dy = q / 3 - 1;
+            const bool in = inz && pos[0] + dx >= 0 && pos[0] + dx < f.n[0] && pos[1] + dy >= 0 && pos[1] + dy < f.n[1];
+            a[q] = A[(threadIdx.y * 9 + q) * V + v];
+            a[q] = in ? a[q] : T(0);
+            xo[q] = x0[in ? v + dx + dy * sy + dz * sz : v];
+        }
+        // the coarse vertices of the plane and of its lines in x and y
+        const int Jz = inz ? iz >> 1 : 0;
+        const int jz[2] = { min(Jz, cdim.n[2] - 1), min(Jz + 1, cdim.n[2] - 1) };
+        const double wz[2] = { inz && Jz < cdim.n[2] ? w1(iz, Jz, f.n[2], cdim.n[2]) : 0.0,
+                               inz && Jz + 1 < cdim.n[2] ? w1(iz, Jz + 1, f.n[2], cdim.n[2]) : 0.0 };
+        double w[2][3][3];
+        int jc[2][3];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            const int J0 = ((pos[d] + 1) >> 1) - 1;
+#pragma unroll
+            for (int J = 0; J < 3; ++J) {
+                const bool in = J0 + J >= 0 && J0 + J < cdim.n[d];
+                jc[d][J] = in ? J0 + J : 0;
+#pragma unroll
+                for (int m = 0; m < 3; ++m) {
+                    const int i = pos[d] - 1 + m;
+                    w[d][m][J] = in && i >= 0 && i < f.n[d] ? w1(i, J0 + J, f.n[d], cdim.n[d]) : 0.0;
                 }
             }
         }
-        xf[v] = (T)((double)xf[v] + acc);
+        double xp[9] = { 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+#pragma unroll
+        for (int Jy = 0; Jy < 3; ++Jy) {
+            const T *row0 = xc + (int64_t)cdim.n[0] * (jc[1][Jy] + (int64_t)cdim.n[1] * jz[0]);
+            const T *row1 = xc + (int64_t)cdim.n[0] * (jc[1][Jy] + (int64_t)cdim.n[1] * jz[1]);
+            double c[3], fx[3];
+#pragma unroll
+            for (int J = 0; J < 3; ++J) c[J] = wz[0] * (double)row0[jc[0][J]] + wz[1] * (double)row1[jc[0][J]];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) fx[m] = w[0][m][0] * c[0] + w[0][m][1] * c[1] + w[0][m][2] * c[2];
+#pragma unroll
+            for (int q = 0; q < 9; ++q) xp[q] = fma(w[1][q / 3][Jy], fx[q % 3], xp[q]);
+        }
+        T acc = 0;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            xo[q] = (T)((double)xo[q] + xp[q]);
+            acc = fma(a[q], xo[q], acc);
+        }
+        acc = plane_sum(part, acc);
+        if (threadIdx.y == 1 && ok) xout[v] = xo[4] + omega * dinv[v] * (r[v] - acc);
     }
 }
 
@@ -352,17 +375,6 @@ __global__ void k_mg_cvol_mean(int64_t E, int K, const Tab1D<double> *__restrict
         mean[e] = s;
     }
 }
-
-// a coarse level's pointwise coefficient: the element mean at each of its points
-__global__ void k_mg_cvol_fill(int64_t E, int K3, const double *__restrict__ mean, double *__restrict__ cvol)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < E * K3; i += (int64_t)gridDim.x * blockDim.x)
-        cvol[i] = mean[i / K3];
-}
-
-
-// row v of the stencil: the probe of colour col answers for the one stencil
-// neighbour of that colour (distinct colours within distance 1)
 
 // the conforming level's stencil in closed form: a(phi_W, phi_v) of the DG Q1
 // operator `a` on the trilinear hat functions of the (n+1)^3 vertices.  The
@@ -426,7 +438,8 @@ __global__ void k_mg_conforming(const DGArgs<double> a, VDims vd, double *__rest
                                         pa *= ca[d] ? xq : 1.0 - xq;
                                         pb *= cb[d] ? xq : 1.0 - xq;
                                     }
-                                    const double r = a.c + (a.cvol ? a.cvol[e * 8 + qx + 2 * qy + 4 * qz] : 0.0);
+                                    const double r = a.c + (a.cvol ? a.cvol[e * 8 + qx + 2 * qy + 4 * qz] : 0.0) +
+                                                     (a.ccell ? a.ccell[e] : 0.0);
                                     acc += tb.w[qx] * tb.w[qy] * tb.w[qz] * detJ * r * pa * pb;
                                 }
                     }
@@ -610,9 +623,13 @@ void Multigrid::init(Operator *fine)
     const int lp = prec == FEM_F64 ? FEM_F64 : FEM_F32;
     const int n[3] = { d0.n[0], d0.n[1], d0.n[2] };
     const int64_t E = fine->E;
+    if (reaction) {
+        cmean.alloc(sizeof(double) * E);
+        cmean32.alloc(sizeof(float) * E);
+    }
     // a coarse operator: the finest one's description at another order and
     // precision, with buffers for the coefficients update() fills (cellwise
-    // kappa; cvol as the element means)
+    // kappa; a pointwise reaction as its element means, shared by the levels)
     auto make_op = [&](int order, int precision) {
         std::unique_ptr<Operator> o(new Operator());
         fem_op_desc d = d0;
@@ -627,11 +644,8 @@ void Multigrid::init(Operator *fine)
             o->a64.kappa_mode = o->a32.kappa_mode = FEM_KAPPA_CELL;
         }
         if (reaction) {
-            const int64_t nq = E * o->k * o->k * o->k;
-            o->cvol64.alloc(sizeof(double) * nq);
-            o->cvol32.alloc(sizeof(float) * nq);
-            o->a64.cvol = o->cvol64.as<double>();
-            o->a32.cvol = o->cvol32.as<float>();
+            o->a64.ccell = cmean.as<double>();
+            o->a32.ccell = cmean32.as<float>();
         }
         return o;
     };
@@ -682,6 +696,7 @@ void Multigrid::init(Operator *fine)
         L->x.alloc(L->V * es);
         L->r.alloc(L->V * es);
         L->t.alloc(L->V * es);
+        L->x0.alloc(L->V * es);
     }
     d64.alloc(vx[0]->V * 8);
     As64.alloc(vx[0]->V * 27 * 8);
@@ -689,7 +704,6 @@ void Multigrid::init(Operator *fine)
     gjX.alloc((size_t)VC * VC * 8);
     gjY.alloc((size_t)VC * VC * 8);
     gjp.alloc((size_t)VC * 8);
-    if (reaction) cmean.alloc(sizeof(double) * E);
     update();
 }
 
@@ -725,18 +739,12 @@ void Multigrid::update()
         hipLaunchKernelGGL(k_mg_cvol_mean, dim3(mg_grid(E)), dim3(MGT), 0, s, E, fine->k, fine->a64.tab,
                            fine->cvol64.as<double>(), cmean.as<double>());
         FEM_HIP(hipGetLastError());
+        round_into(cmean32.p, cmean.p, E);
     }
     auto coefficients = [&](Operator *o) {
         if (desc.kappa_mode == FEM_KAPPA_CELL) {
             FEM_HIP(hipMemcpyAsync(o->kcell64.p, fine->kcell64.p, sizeof(double) * E, hipMemcpyDeviceToDevice, s));
             round_into(o->kcell32.p, o->kcell64.p, E);
-        }
-        if (reaction) {
-            const int64_t nq = E * o->k * o->k * o->k;
-            hipLaunchKernelGGL(k_mg_cvol_fill, dim3(mg_grid(nq)), dim3(MGT), 0, s, E, o->k * o->k * o->k,
-                               cmean.as<double>(), o->cvol64.as<double>());
-            FEM_HIP(hipGetLastError());
-            round_into(o->cvol32.p, o->cvol64.p, nq);
         }
     };
     for (auto &L : dg) {
@@ -863,29 +871,23 @@ void Multigrid::cycle_vertex(size_t l, const T *r, T *x, const int *skip)
 {
     MGVertexLevel &L = *vx[l];
     hipStream_t s = op->ctx->stream;
-    const unsigned G = mg_grid(L.V);
+    const unsigned G = grid_for(L.V, VS, 16384);
     if (l + 1 == vx.size()) {
         hipLaunchKernelGGL(k_mg_dense<T>, dim3((unsigned)((L.V + 3) / 4)), dim3(256), 0, s, (int)L.V,
                            coarse_inv.as<T>(), r, x, skip);
         return;
     }
     VDims d{ { L.nv[0], L.nv[1], L.nv[2] } };
-    T *t = L.t.as<T>();
+    T *t = L.t.as<T>(), *x0 = L.x0.as<T>();
     const T *A = L.A.as<T>(), *dv = L.dinv.as<T>();
     const T om = (T)omega_vertex;
-    auto sweep = [&]() {
-        hipLaunchKernelGGL(k_mg_v_apply<T>, dim3(G), dim3(MGT), 0, s, d, A, (const T *)x, r, t, -1, skip);
-        hipLaunchKernelGGL(k_mg_v_jacobi<T>, dim3(G), dim3(MGT), 0, s, L.V, dv, r, (const T *)t, x, om, 1, skip);
-    };
-    hipLaunchKernelGGL(k_mg_v_jacobi<T>, dim3(G), dim3(MGT), 0, s, L.V, dv, r, (const T *)nullptr, x, om, 0, skip);
-    for (int it = 1; it < nu_vertex; ++it) sweep();
-    hipLaunchKernelGGL(k_mg_v_apply<T>, dim3(G), dim3(MGT), 0, s, d, A, (const T *)x, r, t, -1, skip);
+    hipLaunchKernelGGL(k_mg_v_down<T>, dim3(G), dim3(VS, 3), 0, s, d, A, dv, r, x0, t, om, skip);
     MGVertexLevel &C = *vx[l + 1];
     VDims dc{ { C.nv[0], C.nv[1], C.nv[2] } };
-    hipLaunchKernelGGL(k_mg_v_restrict<T>, dim3(mg_grid(C.V)), dim3(MGT), 0, s, d, dc, (const T *)t, C.r.as<T>(), skip);
+    hipLaunchKernelGGL(k_mg_v_restrict<T>, dim3(grid_for(C.V, VS, 16384)), dim3(VS), 0, s, d, dc, (const T *)t, C.r.as<T>(), skip);
     cycle_vertex<T>(l + 1, C.r.as<T>(), C.x.as<T>(), skip);
-    hipLaunchKernelGGL(k_mg_v_prolong<T>, dim3(G), dim3(MGT), 0, s, d, dc, (const T *)C.x.as<T>(), x, skip);
-    for (int it = 0; it < nu_vertex; ++it) sweep();
+    hipLaunchKernelGGL(k_mg_v_up<T>, dim3(G), dim3(VS, 3), 0, s, d, dc, A, dv, r, (const T *)x0, (const T *)C.x.as<T>(), x,
+                       om, skip);
     FEM_HIP(hipGetLastError());
 }
 
@@ -897,15 +899,14 @@ static void mg_bj(const MGDGLevel &L, const T *r, const T *t, T *x, T omega, int
 }
 
 // one damped block-Jacobi sweep on a level, out = in + omega B^-1 (r - A in),
-// in one pass of the apply kernel (FP64 and FP32 operators) or as an apply
-// followed by the block-Jacobi kernel (BF16-MFMA operators, whose sweep
-// keeps the BF16 apply; then out == in and t is the scratch for A in)
+// in one pass (FP64 and FP32 operators) or as an apply followed by the
+// block-Jacobi kernel (BF16-MFMA operators, whose sweep keeps the BF16 apply;
+// then out == in, and t is the scratch for A in)
 template <typename T>
 static void mg_sweep(const MGDGLevel &L, const T *r, const T *in, T *out, T *t, T omega, const int *skip, hipStream_t s)
 {
     const Operator &o = *L.op;
-    // the fused sweep has no pointwise reaction: apply, then the sweep
-    if (o.desc.precision == FEM_BF16MFMA || o.cvol64.p) {
+    if (o.desc.precision == FEM_BF16MFMA) {
         L.op->apply_raw(in, t, skip);
         mg_bj<T>(L, r, t, out, omega, 1, skip, s);
         return;
@@ -932,7 +933,7 @@ void Multigrid::cycle_dg(size_t l, const T *r, T *x, const int *skip)
     // the fused sweeps write a second buffer (a sweep reads its input's
     // neighbours): cur is the buffer holding the current iterate, and the
     // first sweep is arranged so that the last one ends in x
-    const bool fused = L.op->desc.precision != FEM_BF16MFMA && !L.op->cvol64.p;
+    const bool fused = L.op->desc.precision != FEM_BF16MFMA;
     T *cur = x;
     auto sweep = [&]() {
         if (!fused) {
@@ -948,19 +949,28 @@ void Multigrid::cycle_dg(size_t l, const T *r, T *x, const int *skip)
     if (fused && ((2 * nu_dg - 1) & 1)) cur = t;
     mg_bj<T>(L, r, nullptr, cur, om, 0, skip, s);
     for (int it = 1; it < nu_dg; ++it) sweep();
-    // A cur for the restriction, in whichever buffer cur is not
-    T *ax = fused ? (cur == x ? t : x) : t;
-    (L.resop ? L.resop.get() : L.op)->apply_raw(cur, ax, skip);
+    // the residual in the form the next level takes
+    const Operator &ro = L.resop ? *L.resop : *L.op;
+    DGResidual<T> rs;
+    rs.r = r;
+    auto residual = [&]() {
+        if constexpr (std::is_same<T, double>::value) dg_modal_residual_f64(ro.a64, ro.k, cur, rs, skip, s);
+        else dg_modal_residual_f32(ro.a32, ro.k, cur, rs, skip, s);
+    };
     if (l + 1 < dg.size()) {
         MGDGLevel &C = *dg[l + 1];
-        hipLaunchKernelGGL(k_mg_restrict_modes<T>, dim3(mg_grid(E * C.k * C.k * C.k)), dim3(MGT), 0, s, E, L.k, C.k, r,
-                           (const T *)ax, C.r.as<T>(), skip);
+        rs.rc = C.r.as<T>();
+        rs.kc = C.k;
+        residual();
         cycle_dg<T>(l + 1, C.r.as<T>(), C.x.as<T>(), skip);
         hipLaunchKernelGGL(k_mg_prolong_modes<T>, dim3(mg_grid(E * C.k * C.k * C.k)), dim3(MGT), 0, s, E, L.k, C.k,
                            (const T *)C.x.as<T>(), cur, skip);
     } else {
         MGVertexLevel &V0 = *vx[0];
-        dg1_to_vertex<T>(n, r, (const T *)ax, corners.as<double>(), V0.r.as<T>(), skip, s);
+        rs.corners = corners.as<double>();
+        residual();
+        hipLaunchKernelGGL(k_mg_corners_to_vertex<T>, dim3(mg_grid(V0.V)), dim3(MGT), 0, s, n[0], n[1], n[2],
+                           (const double *)corners.as<double>(), V0.r.as<T>(), skip);
         cycle_vertex<T>(0, V0.r.as<T>(), V0.x.as<T>(), skip);
         hipLaunchKernelGGL(k_mg_vertex_to_dg1<T>, dim3(mg_grid(E * 8)), dim3(MGT), 0, s, n[0], n[1], n[2],
                            (const T *)V0.x.as<T>(), cur, skip);

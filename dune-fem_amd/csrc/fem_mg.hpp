@@ -26,7 +26,7 @@ struct MGDGLevel {
 struct MGVertexLevel {
     int nv[3] = { 0, 0, 0 };
     int64_t V = 0;
-    DevBuf A, dinv, x, r, t;
+    DevBuf A, dinv, x, r, t, x0;
 };
 
 struct Multigrid {
@@ -36,7 +36,7 @@ struct Multigrid {
     std::vector<std::unique_ptr<MGVertexLevel>> vx;
     DevBuf coarse_inv;               // dense inverse of the coarsest vertex level
     DevBuf corners;                  // [E][8] FP64: Q1 modes -> vertex functionals
-    int nu_dg = 2, nu_vertex = 1;    // smoothing sweeps before and after the coarse correction
+    int nu_dg = 2;   // smoothing sweeps of a DG level before and after the coarse correction (vertex levels: one)
     double omega_dg = 0.8, omega_vertex = 0.7;
     fem_op_desc desc{};              // the finest operator's, at init
     bool reaction = false;           // built with a pointwise reaction cvol
@@ -44,7 +44,7 @@ struct Multigrid {
     // element means of cvol, and scratch for the level data and the
     // coarsest inverse
     std::vector<std::unique_ptr<DevBuf>> A64;
-    DevBuf cmean, d64, As64, gjX, gjY, gjp;
+    DevBuf cmean, cmean32, d64, As64, gjX, gjY, gjp;
 
     // builds the hierarchy (levels, operators, buffers), then update()
     void init(Operator *fine);

@@ -445,12 +445,13 @@ void Operator::constrain(Vec &x, const Vec *add) const
 int64_t Operator::dot_blocks() const
 {
     if (!is_dg()) return 0;
-    return dg_is_modal(a64) ? dg_modal_blocks(k, desc.n) : dg_blocks(k, desc.n);
+    return dg_is_modal(a64) ? dg_modal_blocks(k, desc.n, a64.cvol || a64.nl_pow) : dg_blocks(k, desc.n);
 }
 
 int64_t Operator::dot_blocks_max() const
 {
-    return is_dg() ? std::max(dg_modal_blocks(k, desc.n), dg_blocks(k, desc.n)) : 0;
+    if (!is_dg()) return 0;
+    return std::max(std::max(dg_modal_blocks(k, desc.n, false), dg_modal_blocks(k, desc.n, true)), dg_blocks(k, desc.n));
 }
 
 void Operator::apply_raw(const void *x, void *y, const int *skip, double *dot) const

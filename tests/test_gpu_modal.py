@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import dunefem_amd as fa
+import mg_oracle as mgo
 import pyoracle as ora
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +84,54 @@ def test_sweep_equals_apply_and_block_inverse(ctx, n, p):
     # both stop at 1e-11 of |F|; the operator's smallest eigenvalue bounds the
     # distance of the two solutions by 2e-11 times its condition, about 1e4
     assert rel(X[0].download(), X[1].download()) < 1e-6
+
+
+@pytest.mark.parametrize("n,p", [((1, 1, 1), 2), ((6, 17, 5), 1), ((5, 9, 13), 2), ((4, 7, 11), 3), ((3, 5, 7), 4)])
+def test_reaction_apply_matches_oracle(ctx, n, p):
+    """The pass to the Gauss points and back, at rows with a remainder."""
+    rng = np.random.default_rng(sum(n) + p)
+    E = n[0] * n[1] * n[2]
+    kappa, cvol = np.exp(rng.normal(size=E)), rng.uniform(0.5, 2.0, size=(E, (p + 1) ** 3))
+    oop = ora.DGOperator(n, p, 10.0 * p * p, (1, -.5, .25), 0.3, kappa=("cell", kappa))
+    oop.set_reaction_qp(cvol)
+    u = rng.normal(size=oop.N)
+    ref = oop.apply(u)
+    for prec, tol in ((fa.F64, 1e-12), (fa.F32, 2e-5)):
+        op = operator(ctx, n, p, (1, -.5, .25), 0.3, kappa, prec)
+        op.set_reaction_qp(cvol)
+        U, W = op.vector(u), op.vector()
+        W.fill(np.nan)
+        op(U, W)
+        err = rel(W.download(), ref)
+        print("reaction", n, p, prec, err, flush=True)
+        assert err < tol
+
+
+@pytest.mark.parametrize("n,p,reaction", [
+    # one to three vertex levels, vertex counts with a remainder of the
+    # wavefront, even and odd last coarse cells, one cell in a direction
+    ((1, 30, 23), 1, True), ((6, 17, 9), 1, False), ((18, 23, 21), 1, True),
+    ((12, 9, 13), 2, True), ((9, 12, 6), 3, False),
+])
+def test_vcycle_matches_oracle_on_odd_lattices(ctx, n, p, reaction):
+    """Bars as in test_gpu_multigrid.py: the cycle's sums are those of its
+    levels' applies, 1e-12 of max |z| (FP64) and 1e-4 of |z| (FP32)."""
+    rng = np.random.default_rng(sum(n) + p)
+    E = n[0] * n[1] * n[2]
+    kappa, cvol = np.exp(rng.normal(size=E)), rng.uniform(0.5, 2.0, size=(E, (p + 1) ** 3)) if reaction else None
+    M = mgo.MGOracle(n, p, 10.0 * p * p, ("cell", kappa), **({"cvol": cvol} if reaction else {}))
+    r = rng.normal(size=E * (p + 1) ** 3)
+    ref = M.apply(r)
+    for prec in (fa.F64, fa.F32):
+        op = operator(ctx, n, p, (0, 0, 0), 0.0, kappa, prec)
+        if reaction:
+            op.set_reaction_qp(cvol)
+        R, Z = op.vector(r), op.vector()
+        Z.fill(np.nan)
+        fa.Preconditioner(op, fa.PRE_MULTIGRID)(R, Z)
+        z = Z.download()
+        print("vcycle", n, p, prec, rel(z, ref), flush=True)
+        if prec == fa.F64:
+            assert rel(z, ref) < 1e-12
+        else:
+            assert np.linalg.norm(z - ref) < 1e-4 * np.linalg.norm(ref)
