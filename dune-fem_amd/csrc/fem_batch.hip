@@ -279,23 +279,19 @@ void Batch::init(Context *c, int n, const int *nx_, const int *ny_, double c_)
     N = dof_off[n];
     E = elem_off[n];
     for (int sh = 0; sh < CG_NSHAPES; ++sh) {
-        const int TX = CG_SHAPES[sh][0], TY = CG_SHAPES[sh][1];
         std::vector<CGInst> v(n);
-        int off = 0;
+        std::vector<int> of;
         for (int i = 0; i < n; ++i) {
             CGInst &I = v[i];
-            I.nx = nx[i];
-            I.ny = ny[i];
+            I = cg_inst(nx[i], ny[i], sh, creac, 1.0);
             I.dof_off = dof_off[i];
             I.elem_off = elem_off[i];
-            I.tiles_x = (nx[i] + TX - 1) / TX;
-            I.ntiles = I.tiles_x * ((ny[i] + TY - 1) / TY);
-            I.tile_off = off;
-            I.c = creac;
-            I.kappa_const = 1.0;
-            off += I.ntiles;
+            I.tile_off = (int)of.size();
+            of.insert(of.end(), I.ntiles, i);
         }
-        tiles[sh] = off;
+        tile_inst[sh].alloc(sizeof(int) * of.size());
+        FEM_HIP(hipMemcpy(tile_inst[sh].p, of.data(), sizeof(int) * of.size(), hipMemcpyHostToDevice));
+        tiles[sh] = (int)of.size();
         inst_dev[sh].alloc(sizeof(CGInst) * n);
         FEM_HIP(hipMemcpy(inst_dev[sh].p, v.data(), sizeof(CGInst) * n, hipMemcpyHostToDevice));
     }
@@ -369,8 +365,9 @@ void Batch::set_kappa_qp(const double *kv)
     // Jacobi diagonal (FP64 and FP32 inverses)
     DevBuf d;
     d.alloc(sizeof(double) * N);
-    cg_launch_shape<double>(0, CG_MODE_DIAG, inst_dev[0].as<CGInst>(), count, tiles[0], tab.as<CGTab>(),
-                            kvol64.as<double>(), nullptr, d.as<double>(), nullptr, nullptr, ctx->stream);
+    cg_launch_shape<double>(0, CG_MODE_DIAG, inst_dev[0].as<CGInst>(), tile_inst[0].as<int>(), tiles[0], tab.as<CGTab>(),
+                            kvol64.as<double>(), nullptr, d.as<double>(), nullptr, nullptr, ctx->stream,
+                            CGReaction<double>(), true);
     hipLaunchKernelGGL(k_jacobi_inv_b<double>, dim3(grid_for(N, 256, 8192)), dim3(256), 0, ctx->stream, d.as<double>(), dinv64.as<double>(), N);
     hipLaunchKernelGGL(k_jacobi_inv_b<float>, dim3(grid_for(N, 256, 8192)), dim3(256), 0, ctx->stream, d.as<double>(), dinv32.as<float>(), N);
     FEM_HIP(hipGetLastError());
@@ -381,13 +378,13 @@ void Batch::apply_raw(int prec, const void *u, void *w, const int *inst_done) co
 {
     FEM_CHECK(kvol64.p, FEM_ERR_STATE, "batch: coefficient data not set");
     if (prec == FEM_F64)
-        cg_launch_shape<double>(shape, CG_MODE_APPLY, inst_dev[shape].as<CGInst>(), count, tiles[shape],
-                                tab.as<CGTab>(), kvol64.as<double>(), (const double *)u, (double *)w, nullptr,
-                                inst_done, ctx->stream);
+        cg_launch_shape<double>(shape, CG_MODE_APPLY, inst_dev[shape].as<CGInst>(), tile_inst[shape].as<int>(),
+                                tiles[shape], tab.as<CGTab>(), kvol64.as<double>(), (const double *)u, (double *)w,
+                                nullptr, inst_done, ctx->stream, CGReaction<double>(), creac != 0);
     else
-        cg_launch_shape<float>(shape, CG_MODE_APPLY, inst_dev[shape].as<CGInst>(), count, tiles[shape],
-                               tab.as<CGTab>(), kvol32.as<float>(), (const float *)u, (float *)w, nullptr,
-                               inst_done, ctx->stream);
+        cg_launch_shape<float>(shape, CG_MODE_APPLY, inst_dev[shape].as<CGInst>(), tile_inst[shape].as<int>(),
+                               tiles[shape], tab.as<CGTab>(), kvol32.as<float>(), (const float *)u, (float *)w, nullptr,
+                               inst_done, ctx->stream, CGReaction<float>(), creac != 0);
 }
 
 void Batch::rhs(const double *fq, Vec &F) const
@@ -396,8 +393,9 @@ void Batch::rhs(const double *fq, Vec &F) const
     DevBuf f;
     f.alloc(sizeof(double) * E * 9);
     FEM_HIP(hipMemcpy(f.p, fq, sizeof(double) * E * 9, hipMemcpyHostToDevice));
-    cg_launch_shape<double>(0, CG_MODE_RHS, inst_dev[0].as<CGInst>(), count, tiles[0], tab.as<CGTab>(),
-                            f.as<double>(), nullptr, (double *)F.data, nullptr, nullptr, ctx->stream);
+    cg_launch_shape<double>(0, CG_MODE_RHS, inst_dev[0].as<CGInst>(), tile_inst[0].as<int>(), tiles[0], tab.as<CGTab>(),
+                            f.as<double>(), nullptr, (double *)F.data, nullptr, nullptr, ctx->stream,
+                            CGReaction<double>(), false);
     FEM_HIP(hipStreamSynchronize(ctx->stream));
 }
 
@@ -457,8 +455,9 @@ void Batch::solve(const Vec &b, Vec &x, double tol, double inner_tol, int inner_
     auto step = [&](hipStream_t ss) {
         hipLaunchKernelGGL(k_seg_qupd<float>, dim3(nseg), dim3(SEG_THREADS), 0, ss, S, B, q, s);
         if (shape >= 0)
-            cg_launch_shape<float>(shape, CG_MODE_APPLY, inst_dev[shape].as<CGInst>(), count, tiles[shape],
-                                   tab.as<CGTab>(), kvol32.as<float>(), q, h, nullptr, B.done, ss);
+            cg_launch_shape<float>(shape, CG_MODE_APPLY, inst_dev[shape].as<CGInst>(), tile_inst[shape].as<int>(),
+                                   tiles[shape], tab.as<CGTab>(), kvol32.as<float>(), q, h, nullptr, B.done, ss,
+                                   CGReaction<float>(), creac != 0);
         hipLaunchKernelGGL((k_seg<float, SEG_QH>), dim3(nseg), dim3(SEG_THREADS), 0, ss, S, B, d, p, q, h, s, r32p, dv, 0.0);
         hipLaunchKernelGGL((k_seg<float, SEG_UPD>), dim3(nseg), dim3(SEG_THREADS), 0, ss, S, B, d, p, q, h, s, r32p, dv, 0.0);
     };

@@ -15,6 +15,7 @@ struct Batch {
     int shape = 0;                       // index into CG_SHAPES
     float tune_ms[CG_NSHAPES] = {};
     DevBuf inst_dev[CG_NSHAPES];
+    DevBuf tile_inst[CG_NSHAPES];        // the instance of each tile
     int tiles[CG_NSHAPES] = {};
     DevBuf tab, kvol64, kvol32, dinv64, dinv32;
     DevBuf seg_inst, seg_lo, seg_hi, seg_first, seg_counter, seg_partials;

@@ -6,13 +6,9 @@
 // addLocalDofs scatter (dune/fem/schemes/galerkin.hh:811-917, 929-934) and
 // DirichletWrapperOperator::operator() (dirichletwrapper.hh:101-105: w_D = u_D).
 //
-// Design: a workgroup owns a CG_TX x CG_TY tile of elements and the nodes at
-// their lower-left 2x2 node block; one thread per element of the tile plus a
-// lower halo row/column, so every contribution to an owned node is computed
-// inside the workgroup.  Element results are added into an LDS node lattice
-// in four colour phases (elements of one colour share no node), which makes
-// the summation order fixed: results are deterministic and need no atomics.
-#include "fem_cg.hpp"
+// The tile of a workgroup and the exchange between its elements: fem_cg_tile.hpp.
+#include "fem_blas.hpp"
+#include "fem_cg_tile.hpp"
 
 #include <algorithm>
 
@@ -33,113 +29,58 @@ CGTab make_cg_tab()
     return t;
 }
 
-template <int TX, int TY, typename T>
+// w = A u (APPLY), the diagonal, the load vector.  The apply moves 9 coefficients per
+// element and two vectors, and on a few hundred thousand elements it is a single set of
+// workgroups, so what counts is the chain of one of them: 517 x 386 FP64 with pointwise
+// kappa 7.1 us (27 MB; 12.8 us with FP64 tables converted at each use, four coloured
+// additions into LDS with a barrier each, and neighbouring tiles on different XCDs; of
+// that last 1.8 us), 1024^2 26 us (49.6 us).  tile_inst names the instance of a
+// workgroup, one load where a search over the instances' first tiles was a chain of five
+// to eight; a single instance comes with the arguments.
+template <int TX, int TY, typename T, bool APPLY, bool RX>
 __global__ void __launch_bounds__((TX + 1) * (TY + 1))
-    k_cg(int mode, const CGInst *__restrict__ insts, int ninst, const CGTab *__restrict__ tabp,
+    k_cg(int mode, const CGInst one, const CGInst *__restrict__ insts, const int *__restrict__ tile_inst, const CGTab *__restrict__ tabp,
          const T *__restrict__ kvol, const T *__restrict__ in, T *__restrict__ out, const int *__restrict__ skip,
-         const int *__restrict__ inst_done, const CGReaction<T> rx)
+         const int *__restrict__ inst_done, const CGReaction<T> rx, double *__restrict__ dot)
 {
-    constexpr int CG_LX = 2 * TX + 3, CG_LY = 2 * TY + 3;
+    constexpr int NT = (TX + 1) * (TY + 1);
     if (skip && *skip) return;
-    __shared__ T lat[CG_LX * CG_LY];
-    __shared__ int s_inst;
-    const unsigned bid = blockIdx.x;
-    if (threadIdx.x == 0) {
-        int lo = 0, hi = ninst - 1;
-        while (lo < hi) {  // last instance with tile_off <= bid
-            int mid = (lo + hi + 1) >> 1;
-            if ((unsigned)insts[mid].tile_off <= bid) lo = mid; else hi = mid - 1;
-        }
-        s_inst = lo;
-    }
-    for (int k = threadIdx.x; k < CG_LX * CG_LY; k += blockDim.x) lat[k] = 0;
-    __syncthreads();
-    if (inst_done && inst_done[s_inst]) return;   // uniform over the block
-    const CGInst P = insts[s_inst];
-    const CGTab &tb = *tabp;
-    const int tile = (int)bid - P.tile_off;
-    const int ex0 = (tile % P.tiles_x) * TX, ey0 = (tile / P.tiles_x) * TY;
-    const int tx = threadIdx.x % (TX + 1), ty = threadIdx.x / (TX + 1);
-    const int ex = ex0 - 1 + tx, ey = ey0 - 1 + ty;
-    const bool valid = ex >= 0 && ey >= 0 && ex < P.nx && ey < P.ny;
-    const int NX = 2 * P.nx + 1;
+    __shared__ T xch[5][NT];
+    const int bid = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int ii = tile_inst ? tile_inst[bid] : 0;
+    if (inst_done && inst_done[ii]) return;   // uniform over the block
+    const CGInst P = tile_inst ? insts[ii] : one;
+    const CGTile t = cg_tile<TX, TY>(P, bid);
     const T *u = in + P.dof_off;
-    T wl[3][3];
-    if (valid) {
-        const double hx = 1.0 / P.nx, hy = 1.0 / P.ny, detJ = hx * hy;
-        const int64_t e = P.elem_off + (int64_t)ey * P.nx + ex;
-        if (mode == CG_MODE_APPLY) {
-            T ul[3][3];
+    const int64_t e = P.elem_off + (int64_t)t.ey * P.nx + t.ex;
+    T wl[3][3] = {}, ul[3][3] = {};
+    if (t.valid) {
+        if constexpr (APPLY) {
+            T kap[9], cv[9];
 #pragma unroll
             for (int iy = 0; iy < 3; ++iy)
 #pragma unroll
-                for (int ix = 0; ix < 3; ++ix) ul[iy][ix] = u[(int64_t)(2 * ey + iy) * NX + 2 * ex + ix];
-            // sum factorisation: x then y
-            T t0[3][3], t1[3][3];
+                for (int ix = 0; ix < 3; ++ix) ul[iy][ix] = u[(int64_t)(2 * t.ey + iy) * t.NX + 2 * t.ex + ix];
 #pragma unroll
-            for (int iy = 0; iy < 3; ++iy)
-#pragma unroll
-                for (int qx = 0; qx < 3; ++qx) {
-                    T a = 0, b = 0;
-#pragma unroll
-                    for (int ix = 0; ix < 3; ++ix) {
-                        a += (T)tb.L[qx][ix] * ul[iy][ix];
-                        b += (T)tb.Ld[qx][ix] * ul[iy][ix];
-                    }
-                    t0[iy][qx] = a;
-                    t1[iy][qx] = b;
+            for (int q = 0; q < 9; ++q) {
+                kap[q] = kvol ? kvol[e * 9 + q] : (T)P.kappa_const;
+                cv[q] = RX && rx.cvol ? rx.cvol[e * 9 + q] : T(0);
+            }
+            // the reaction c + cvol + coef u^pw (the pointwise and nonlinear
+            // parts of a single instance)
+            const T c = (T)P.c, dj = (T)P.detJ;
+            cg_element<T, RX>(ul, kap, (T)P.sx, (T)P.sy, [&](T uq, int q) {
+                T r = c + cv[q];
+                if (rx.pw) {
+                    T pw = rx.coef;
+                    for (int n = 0; n < rx.pw; ++n) pw *= uq;
+                    r += pw;
                 }
-            T fx[3][3], fy[3][3], fm[3][3];
-#pragma unroll
-            for (int qy = 0; qy < 3; ++qy)
-#pragma unroll
-                for (int qx = 0; qx < 3; ++qx) {
-                    T uq = 0, gx = 0, gy = 0;
-#pragma unroll
-                    for (int iy = 0; iy < 3; ++iy) {
-                        uq += (T)tb.L[qy][iy] * t0[iy][qx];
-                        gx += (T)tb.L[qy][iy] * t1[iy][qx];
-                        gy += (T)tb.Ld[qy][iy] * t0[iy][qx];
-                    }
-                    const T W = (T)(tb.w[qx] * tb.w[qy] * detJ);
-                    const T kap = kvol ? kvol[e * 9 + qx + 3 * qy] : (T)P.kappa_const;
-                    fx[qy][qx] = W * kap * gx * (T)(1.0 / (hx * hx));
-                    fy[qy][qx] = W * kap * gy * (T)(1.0 / (hy * hy));
-                    // reaction c + cvol + coef u^pw (the pointwise and
-                    // nonlinear parts of a single instance)
-                    T r = (T)P.c;
-                    if (rx.cvol) r += rx.cvol[e * 9 + qx + 3 * qy];
-                    if (rx.pw) {
-                        T pw = rx.coef;
-                        for (int t = 0; t < rx.pw; ++t) pw *= uq;
-                        r += pw;
-                    }
-                    fm[qy][qx] = W * r * uq;
-                }
-            // transpose: y then x
-#pragma unroll
-            for (int qx = 0; qx < 3; ++qx)
-#pragma unroll
-                for (int iy = 0; iy < 3; ++iy) {
-                    T a = 0, b = 0;
-#pragma unroll
-                    for (int qy = 0; qy < 3; ++qy) {
-                        a += (T)tb.L[qy][iy] * (fx[qy][qx]);
-                        b += (T)tb.Ld[qy][iy] * fy[qy][qx] + (T)tb.L[qy][iy] * fm[qy][qx];
-                    }
-                    t0[iy][qx] = a;   // to be contracted with Ld in x
-                    t1[iy][qx] = b;   // with L in x
-                }
-#pragma unroll
-            for (int iy = 0; iy < 3; ++iy)
-#pragma unroll
-                for (int ix = 0; ix < 3; ++ix) {
-                    T a = 0;
-#pragma unroll
-                    for (int qx = 0; qx < 3; ++qx) a += (T)tb.Ld[qx][ix] * t0[iy][qx] + (T)tb.L[qx][ix] * t1[iy][qx];
-                    wl[iy][ix] = a;
-                }
+                return dj * r;
+            }, wl);
         } else {
+            const CGTab &tb = *tabp;
+            const double hx = 1.0 / P.nx, hy = 1.0 / P.ny, detJ = hx * hy;
 #pragma unroll
             for (int iy = 0; iy < 3; ++iy)
 #pragma unroll
@@ -162,36 +103,25 @@ __global__ void __launch_bounds__((TX + 1) * (TY + 1))
                 }
         }
     }
-    // coloured accumulation into the LDS node lattice
-#pragma unroll
-    for (int col = 0; col < 4; ++col) {
-        if (valid && (tx & 1) == (col & 1) && (ty & 1) == (col >> 1)) {
-#pragma unroll
-            for (int iy = 0; iy < 3; ++iy)
-#pragma unroll
-                for (int ix = 0; ix < 3; ++ix) lat[(2 * ty + iy) * CG_LX + 2 * tx + ix] += wl[iy][ix];
-        }
-        __syncthreads();
-    }
-    // owned nodes
-    const int I0 = 2 * ex0, J0 = 2 * ey0;
-    const int I1 = (ex0 + TX >= P.nx) ? 2 * P.nx + 1 : 2 * ex0 + 2 * TX;
-    const int J1 = (ey0 + TY >= P.ny) ? 2 * P.ny + 1 : 2 * ey0 + 2 * TY;
-    const int wx = I1 - I0, wy = J1 - J0;
     T *o = out + P.dof_off;
-    for (int k = threadIdx.x; k < wx * wy; k += blockDim.x) {
-        const int I = I0 + k % wx, J = J0 + k / wx;
-        const int64_t node = (int64_t)J * NX + I;
-        const bool bnd = I == 0 || J == 0 || I == 2 * P.nx || J == 2 * P.ny;
-        T val = lat[(J - J0 + 2) * CG_LX + (I - I0 + 2)];
-        if (mode == CG_MODE_RHS_ADD) {
+    double d = 0;
+    cg_gather<TX, TY, T>(P, t, wl, xch, [&](int64_t node, bool bnd, int iy, int ix, T v) {
+        if constexpr (APPLY) {
+            if (bnd) v = ul[iy][ix];
+            o[node] = v;
+            d += (double)ul[iy][ix] * (double)v;
+        } else if (mode == CG_MODE_RHS_ADD) {
             // accumulate into the interior rows; the Dirichlet rows keep what
             // the apply wrote there
-            if (!bnd) o[node] += val;
-            continue;
+            if (!bnd) o[node] += v;
+        } else {
+            o[node] = bnd ? (mode == CG_MODE_DIAG ? T(1) : T(0)) : v;
         }
-        if (bnd) val = mode == CG_MODE_APPLY ? u[node] : mode == CG_MODE_DIAG ? T(1) : T(0);
-        o[node] = val;
+    });
+    if (APPLY && dot) {
+        __shared__ double lds[(NT + 63) / 64];
+        const double tot = block_sum(d, lds);
+        if (threadIdx.x == 0) dot[bid] = tot;
     }
 }
 
@@ -235,16 +165,31 @@ template void cg_eval_qp<double>(int, int, const CGTab *, const double *, const 
 template void cg_eval_qp<float>(int, int, const CGTab *, const float *, const float *, float, int, float *,
                                 hipStream_t);
 
-template <typename T>
-void cg_launch_shape(int shape, int mode, const CGInst *d_inst, int ninst, int total_tiles, const CGTab *d_tab,
-                     const T *kvol, const T *in, T *out, const int *skip, const int *inst_done, hipStream_t s,
-                     const CGReaction<T> &rx)
+template <int TX, int TY, typename T>
+static void launch_tile(int mode, const CGInst &one, const CGInst *d_inst, const int *tile_inst, int tiles,
+                        const CGTab *d_tab, const T *kvol, const T *in, T *out, const int *skip, const int *inst_done, hipStream_t s,
+                        const CGReaction<T> &rx, bool reaction, double *dot)
 {
-    FEM_CHECK(ninst == 1 || (!rx.cvol && !rx.pw), FEM_ERR_ARG, "pointwise/nonlinear reaction: a single instance");
-#define CGS(ID, TX, TY)                                                                                       \
-    case ID:                                                                                                 \
-        hipLaunchKernelGGL((k_cg<TX, TY, T>), dim3(total_tiles), dim3((TX + 1) * (TY + 1)), 0, s, mode, d_inst, \
-                           ninst, d_tab, kvol, in, out, skip, inst_done, rx);                                \
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(tiles), dim3((TX + 1) * (TY + 1)), 0, s, mode, one, d_inst, tile_inst, d_tab, kvol,
+                           in, out, skip, inst_done, rx, dot);
+    };
+    if (mode != CG_MODE_APPLY) go(k_cg<TX, TY, T, false, false>);
+    else if (reaction) go(k_cg<TX, TY, T, true, true>);
+    else go(k_cg<TX, TY, T, true, false>);
+}
+
+template <typename T>
+void cg_launch_shape(int shape, int mode, const CGInst *inst, const int *tile_inst, int total_tiles, const CGTab *d_tab,
+                     const T *kvol, const T *in, T *out, const int *skip, const int *inst_done, hipStream_t s,
+                     const CGReaction<T> &rx, bool c, double *dot)
+{
+    FEM_CHECK(!tile_inst || (!rx.cvol && !rx.pw), FEM_ERR_ARG, "pointwise/nonlinear reaction: a single instance");
+    const bool reaction = c || rx.cvol || rx.pw;
+#define CGS(ID, TX, TY)                                                                                          \
+    case ID:                                                                                                     \
+        launch_tile<TX, TY, T>(mode, tile_inst ? CGInst{} : *inst, inst, tile_inst, total_tiles, d_tab, kvol, in, out, skip, inst_done, s, rx, \
+                               reaction, dot);                                                                   \
         break;
     switch (shape) {
         CGS(0, 15, 15) CGS(1, 7, 7) CGS(2, 15, 7) CGS(3, 31, 7) CGS(4, 7, 31)
@@ -254,22 +199,11 @@ void cg_launch_shape(int shape, int mode, const CGInst *d_inst, int ninst, int t
     FEM_HIP(hipGetLastError());
 }
 
-template <typename T>
-void cg_launch(int mode, const CGInst *d_inst, int ninst, int total_tiles, const CGTab *d_tab, const T *kvol,
-               const T *in, T *out, const int *skip, hipStream_t s, const CGReaction<T> &rx)
-{
-    cg_launch_shape<T>(0, mode, d_inst, ninst, total_tiles, d_tab, kvol, in, out, skip, nullptr, s, rx);
-}
-
-template void cg_launch<double>(int, const CGInst *, int, int, const CGTab *, const double *, const double *,
-                                double *, const int *, hipStream_t, const CGReaction<double> &);
-template void cg_launch<float>(int, const CGInst *, int, int, const CGTab *, const float *, const float *,
-                               float *, const int *, hipStream_t, const CGReaction<float> &);
-template void cg_launch_shape<double>(int, int, const CGInst *, int, int, const CGTab *, const double *,
+template void cg_launch_shape<double>(int, int, const CGInst *, const int *, int, const CGTab *, const double *,
                                       const double *, double *, const int *, const int *, hipStream_t,
-                                      const CGReaction<double> &);
-template void cg_launch_shape<float>(int, int, const CGInst *, int, int, const CGTab *, const float *,
+                                      const CGReaction<double> &, bool, double *);
+template void cg_launch_shape<float>(int, int, const CGInst *, const int *, int, const CGTab *, const float *,
                                      const float *, float *, const int *, const int *, hipStream_t,
-                                     const CGReaction<float> &);
+                                     const CGReaction<float> &, bool, double *);
 
 }  // namespace femamd

@@ -16,14 +16,32 @@ struct CGInst {
     int ntiles;
     double c;           // reaction coefficient
     double kappa_const; // used when kvol == nullptr
+    double sx, sy;      // hy / hx and hx / hy
+    double detJ;        // hx hy
 };
-
-constexpr int CG_TX = 15, CG_TY = 15;                  // default tile: owned elements per tile
-constexpr int CG_THREADS = (CG_TX + 1) * (CG_TY + 1);  // + lower halo row/column
 
 // tile shapes available to the autotuner (owned elements per tile)
 constexpr int CG_NSHAPES = 5;
 constexpr int CG_SHAPES[CG_NSHAPES][2] = { { 15, 15 }, { 7, 7 }, { 15, 7 }, { 31, 7 }, { 7, 31 } };
+// the shape of a single instance's operator: FP64, pointwise kappa, 517 x 386 elements
+// 7.1 us (7 x 7: 8.3, 15 x 7: 7.4, 31 x 7: 7.4), 1024^2 27.7 us (32.4, 27.7, 26.5)
+constexpr int CG_SINGLE = 0;
+
+// an instance of nx x ny elements in tiles of the given shape
+inline CGInst cg_inst(int nx, int ny, int shape, double c, double kappa_const)
+{
+    CGInst I{};
+    I.nx = nx;
+    I.ny = ny;
+    I.tiles_x = (nx + CG_SHAPES[shape][0] - 1) / CG_SHAPES[shape][0];
+    I.ntiles = I.tiles_x * ((ny + CG_SHAPES[shape][1] - 1) / CG_SHAPES[shape][1]);
+    I.c = c;
+    I.kappa_const = kappa_const;
+    I.sx = (double)nx / ny;
+    I.sy = (double)ny / nx;
+    I.detJ = 1.0 / ((double)nx * ny);
+    return I;
+}
 
 struct CGTab {
     double L[3][3];   // Q2 basis i at Gauss point q: L[q][i]
@@ -47,15 +65,14 @@ struct CGReaction {
 // mode DIAG   : out = diag(A) (Dirichlet rows: 1), `in` unused
 // mode RHS    : out = F from f at quadrature points (kvol slot carries f), Dirichlet rows 0
 // mode RHS_ADD: out += F on the interior rows (Dirichlet rows unchanged)
+// in tiles of CG_SHAPES[shape]; tile_inst: the instance of each tile, inst the table on
+// the device (null: a single instance, inst on the host); instances with inst_done[i] != 0 (may be null) are skipped; `c`: some
+// instance has a reaction c; `dot` (APPLY, may be null): the workgroups' FP64
+// partials of <in, out>, one per tile
 template <typename T>
-void cg_launch(int mode, const CGInst *d_inst, int ninst, int total_tiles, const CGTab *d_tab, const T *kvol,
-               const T *in, T *out, const int *skip, hipStream_t s, const CGReaction<T> &rx = CGReaction<T>());
-// same with an explicit tile shape (index into CG_SHAPES) and an optional
-// per-instance mask: instances with inst_done[i] != 0 are skipped
-template <typename T>
-void cg_launch_shape(int shape, int mode, const CGInst *d_inst, int ninst, int total_tiles, const CGTab *d_tab,
+void cg_launch_shape(int shape, int mode, const CGInst *inst, const int *tile_inst, int total_tiles, const CGTab *d_tab,
                      const T *kvol, const T *in, T *out, const int *skip, const int *inst_done, hipStream_t s,
-                     const CGReaction<T> &rx = CGReaction<T>());
+                     const CGReaction<T> &rx, bool c, double *dot = nullptr);
 // out[e*9 + qx + 3 qy] = base + coef u(x_q)^pw (base may be null) for a
 // single instance of nx x ny elements
 template <typename T>

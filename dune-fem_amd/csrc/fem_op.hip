@@ -92,18 +92,8 @@ void Operator::init(Context *c, const fem_op_desc &d)
         k = 3;
         E = (int64_t)d.n[0] * d.n[1];
         N = (int64_t)(2 * d.n[0] + 1) * (2 * d.n[1] + 1);
-        inst.nx = d.n[0];
-        inst.ny = d.n[1];
-        inst.dof_off = 0;
-        inst.elem_off = 0;
-        inst.tiles_x = (d.n[0] + CG_TX - 1) / CG_TX;
-        inst.ntiles = inst.tiles_x * ((d.n[1] + CG_TY - 1) / CG_TY);
-        inst.tile_off = 0;
-        inst.c = d.c;
-        inst.kappa_const = d.kappa_const;
+        inst = cg_inst(d.n[0], d.n[1], CG_SINGLE, d.c, d.kappa_const);
         tiles = inst.ntiles;
-        inst_dev.alloc(sizeof(CGInst));
-        FEM_HIP(hipMemcpy(inst_dev.p, &inst, sizeof(CGInst), hipMemcpyHostToDevice));
         CGTab t = make_cg_tab();
         cgtab.alloc(sizeof(t));
         FEM_HIP(hipMemcpy(cgtab.p, &t, sizeof(t), hipMemcpyHostToDevice));
@@ -444,13 +434,13 @@ void Operator::constrain(Vec &x, const Vec *add) const
 
 int64_t Operator::dot_blocks() const
 {
-    if (!is_dg()) return 0;
+    if (!is_dg()) return tiles;
     return dg_is_modal(a64) ? dg_modal_blocks(k, desc.n, a64.cvol || a64.nl_pow) : dg_blocks(k, desc.n);
 }
 
 int64_t Operator::dot_blocks_max() const
 {
-    if (!is_dg()) return 0;
+    if (!is_dg()) return tiles;
     return std::max(std::max(dg_modal_blocks(k, desc.n, false), dg_modal_blocks(k, desc.n, true)), dg_blocks(k, desc.n));
 }
 
@@ -482,7 +472,8 @@ void Operator::apply_raw(const void *x, void *y, const int *skip, double *dot) c
             dg_rhs(a64, k, ps.as<double>(), (double *)y, s, true);
         }
     } else {
-        FEM_CHECK(!dot, FEM_ERR_UNSUPPORTED, "fused dot: DG operators only");
+        FEM_CHECK(!plugin || !dot, FEM_ERR_STATE,
+                  "apply: an operator with a compiled reaction is nonlinear (no fused dot)");
         FEM_CHECK(desc.kappa_mode == FEM_KAPPA_CONST || kvol64.p, FEM_ERR_STATE, "coefficient data not set");
         FEM_CHECK(!plugin || !skip, FEM_ERR_STATE,
                   "apply: an operator with a compiled reaction is nonlinear (no captured solve)");
@@ -491,17 +482,17 @@ void Operator::apply_raw(const void *x, void *y, const int *skip, double *dot) c
             rx.cvol = cvol64.as<double>();
             rx.coef = nl_coef;
             rx.pw = nl_pow;
-            cg_launch<double>(CG_MODE_APPLY, inst_dev.as<CGInst>(), 1, tiles, cgtab.as<CGTab>(),
-                              desc.kappa_mode == FEM_KAPPA_QP ? kvol64.as<double>() : nullptr, (const double *)x,
-                              (double *)y, skip, s, rx);
+            cg_launch_shape<double>(CG_SINGLE, CG_MODE_APPLY, &inst, nullptr, tiles, cgtab.as<CGTab>(),
+                                    desc.kappa_mode == FEM_KAPPA_QP ? kvol64.as<double>() : nullptr,
+                                    (const double *)x, (double *)y, skip, nullptr, s, rx, desc.c != 0, dot);
         } else {
             CGReaction<float> rx;
             rx.cvol = cvol32.as<float>();
             rx.coef = (float)nl_coef;
             rx.pw = nl_pow;
-            cg_launch<float>(CG_MODE_APPLY, inst_dev.as<CGInst>(), 1, tiles, cgtab.as<CGTab>(),
-                             desc.kappa_mode == FEM_KAPPA_QP ? kvol32.as<float>() : nullptr, (const float *)x,
-                             (float *)y, skip, s, rx);
+            cg_launch_shape<float>(CG_SINGLE, CG_MODE_APPLY, &inst, nullptr, tiles, cgtab.as<CGTab>(),
+                                   desc.kappa_mode == FEM_KAPPA_QP ? kvol32.as<float>() : nullptr,
+                                   (const float *)x, (float *)y, skip, nullptr, s, rx, desc.c != 0, dot);
         }
         if (plugin) {
             // y += int r(u, x) v on the interior rows (the Dirichlet rows
@@ -511,8 +502,9 @@ void Operator::apply_raw(const void *x, void *y, const int *skip, double *dot) c
             const fem_qp_geometry g = qp_geometry();
             FEM_CHECK(plugin(&g, pq.as<double>(), ps.as<double>(), nullptr, (void *)s) == 0, FEM_ERR_HIP,
                       "compiled reaction: launch failed");
-            cg_launch<double>(CG_MODE_RHS_ADD, inst_dev.as<CGInst>(), 1, tiles, cgtab.as<CGTab>(), ps.as<double>(),
-                              nullptr, (double *)y, nullptr, s);
+            cg_launch_shape<double>(CG_SINGLE, CG_MODE_RHS_ADD, &inst, nullptr, tiles, cgtab.as<CGTab>(),
+                                    ps.as<double>(), nullptr, (double *)y, nullptr, nullptr, s, CGReaction<double>(),
+                                    false);
         }
     }
 }
@@ -542,7 +534,8 @@ void Operator::rhs(const double *fq_host, Vec &F) const
             dg_rhs_bnd(a64, k, g, dst, s);
         }
     } else {
-        cg_launch<double>(CG_MODE_RHS, inst_dev.as<CGInst>(), 1, tiles, cgtab.as<CGTab>(), fq.as<double>(), nullptr, dst, nullptr, s);
+        cg_launch_shape<double>(CG_SINGLE, CG_MODE_RHS, &inst, nullptr, tiles, cgtab.as<CGTab>(),
+                                fq.as<double>(), nullptr, dst, nullptr, nullptr, s, CGReaction<double>(), false);
         // R(u) = A u - F has Dirichlet rows u_D - g_D, as the reference's
         // DirichletWrapperOperator (dirichletwrapper.hh:101-105 with
         // subConstraints, dirichletconstraints.hh:494-554): F_D = g_D
@@ -573,8 +566,9 @@ void Operator::diagonal(Vec &d) const
     } else {
         CGReaction<double> rx;
         rx.cvol = cvol64.as<double>();
-        cg_launch<double>(CG_MODE_DIAG, inst_dev.as<CGInst>(), 1, tiles, cgtab.as<CGTab>(),
-                          desc.kappa_mode == FEM_KAPPA_QP ? kvol64.as<double>() : nullptr, nullptr, dst, nullptr, s, rx);
+        cg_launch_shape<double>(CG_SINGLE, CG_MODE_DIAG, &inst, nullptr, tiles, cgtab.as<CGTab>(),
+                                desc.kappa_mode == FEM_KAPPA_QP ? kvol64.as<double>() : nullptr, nullptr, dst, nullptr,
+                                nullptr, s, rx, true);
     }
     if (d.prec != FEM_F64) {
         Vec tmp;

@@ -48,8 +48,8 @@ struct Operator {
     DevBuf tab64, tab32;
     DevBuf kvol64, kface64[3], kcell64, kvol32, kface32[3], kcell32;
     // CG
+    DevBuf cgtab;
     CGInst inst{};
-    DevBuf inst_dev, cgtab;
     int tiles = 0;
 
     void init(Context *c, const fem_op_desc &d);
@@ -103,7 +103,7 @@ struct Operator {
     // refinement solve)
     void make_jacobian(Operator &jop, int precision = -1) const;
     // y = A x on raw device pointers of the operator's vector precision;
-    // `dot` (DG only, may be null): per-workgroup FP64 partials of <x, y>,
+    // `dot` (not BF16, may be null): per-workgroup FP64 partials of <x, y>,
     // dot_blocks() entries
     void apply_raw(const void *x, void *y, const int *skip, double *dot = nullptr) const;
     int64_t dot_blocks() const;

@@ -814,12 +814,12 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
         FEM_HIP(hipGetLastError());
         const T *dinv = (haspre && p->pointwise()) ? (const T *)p->dinv.p : nullptr;
         // workgroups of the vector kernels (about four elements per thread),
-        // and the partials of <q, h> and of <p, s>, <p, p>: from the DG apply
+        // and the partials of <q, h> and of <p, s>, <p, p>: from the apply
         // and from the preconditioner where they write them, else from a pass
         // over the vectors.  Every workgroup of the kernel that follows sums
         // them, so more than CG_PARTS are first brought down to CG_FEWER
         const unsigned GU = grid_for(N, 4 * RED_THREADS, CG_PARTS / 4);
-        const bool qfused = o->is_dg() && o->desc.precision != FEM_BF16MFMA;
+        const bool qfused = o->desc.precision != FEM_BF16MFMA;
         const bool pfused = haspre && p->fused_dot();
         const int64_t nq0 = qfused ? o->dot_blocks() : GU, np0 = pfused ? p->dot_parts() : GU;
         const int nq = (int)(nq0 > CG_PARTS ? CG_FEWER : nq0), np = (int)(np0 > CG_PARTS ? CG_FEWER : np0);
