@@ -10,224 +10,315 @@
 //
 // Layout: all instances' DoFs are concatenated (dof_off), their elements too
 // (elem_off, coefficient arrays [E][9]).  Reductions are segmented: every
-// reduction block belongs to one instance, the last block of an instance to
-// finish sums that instance's partials in block order (deterministic).
-// One inner CG step is four launches; they are captured once in a HIP graph
-// and replayed.
+// workgroup belongs to one instance and writes its partial, and the workgroups of
+// the kernel that needs the sum add that instance's partials in a fixed order.
+// One inner CG step is two launches; a few steps are captured in a HIP graph.  Most
+// batches are a few hundred workgroups per kernel, so a step costs what its chain of
+// launches and dependent loads costs: 24 instances of 32 to 128 elements a side
+// (616k DoFs) 32 us in four launches whose sums the last workgroup of an instance
+// finished behind atomics, now 16.7 us (apply 8.3, update 6.1).
 #include <algorithm>
 #include <chrono>
 #include <cmath>
 
 #include "fem_batch.hpp"
 #include "fem_blas.hpp"
+#include "fem_cg_tile.hpp"
 
 namespace femamd {
 
 constexpr int SEG_THREADS = 256;
-constexpr int SEG_ITEMS = 8;   // DoFs per thread of a segment
+constexpr int SEG_ITEMS = 4;     // DoFs in flight per thread
 constexpr int SEG_CHUNK = SEG_THREADS * SEG_ITEMS;
+constexpr int SEG_MOST = 1024;   // segments of an instance: each workgroup of its apply sums their partials
+constexpr int GRAPH_STEPS = 8;   // steps per captured graph (even: q has two buffers)
 
 struct SegTab {
-    const int *inst;       // [nblocks] instance of each block
-    const int64_t *lo;     // [nblocks] first DoF
-    const int64_t *hi;     // [nblocks] one past the last DoF
-    const int *first;      // [count + 1] first block of each instance
-    unsigned *counter;     // [count]
-    double *partials;      // [3 * nblocks]
+    const int *inst;       // [nseg] instance of each segment
+    const int64_t *lo;     // [nseg] first DoF
+    const int64_t *hi;     // [nseg] one past the last DoF
+    const int *first;      // [count + 1] first segment of each instance
+    double *parts;         // [2][nseg]
 };
 
-struct BState {            // per-instance scalars (device arrays)
-    double *res, *prev, *alpha, *beta, *tol, *rr, *bn2, *rn, *scale;
-    int *it, *done, *conv;
-    int maxit;
+// per-instance scalars (device arrays).  No kernel reads what one of its own
+// workgroups writes: res (<p, s>) and done are set by the apply and read by the
+// update that follows; prev (that of the step before), it and idle (done, as the
+// applies after it see it) are set by the update and read by the apply.
+struct BState {
+    double *res, *prev, *tol, *rn, *bn2, *scale, *eps2;
+    int *it, *done, *idle, *conv, *maxit;
 };
 
-__device__ __forceinline__ double bsum(double v, double *lds)
+// the sums of the instance's partials a[lo .. hi) and b[lo .. hi), in every thread,
+// for every workgroup of NT threads alike; two barriers
+template <int NT, int NQ>
+__device__ __forceinline__ void seg_sum(const double *__restrict__ a, const double *__restrict__ b, int lo, int hi,
+                                        double *lds, double (&sum)[NQ])
 {
-    return block_sum(v, lds);
-}
-
-// last block of an instance: sums that instance's partials in a fixed order
-// (thread t takes blocks first+t, first+t+256, ...; then a block tree)
-__device__ __forceinline__ bool seg_finish(const SegTab &S, int inst, int nq, const double *own, double *tot)
-{
-    __shared__ bool amLast;
-    __shared__ double lds2[SEG_THREADS / 64];
-    const int nb = gridDim.x;
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < nq; ++q) publish_partial(&S.partials[(size_t)q * nb + blockIdx.x], own[q]);
-        const int nblk = S.first[inst + 1] - S.first[inst];
-        amLast = atomicAdd(&S.counter[inst], 1u) == (unsigned)(nblk - 1);
+    double v[NQ] = {};
+#pragma unroll 4
+    for (int k = lo + (int)threadIdx.x; k < hi; k += NT) {
+        v[0] += a[k];
+        if constexpr (NQ > 1) v[1] += b[k];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
+        if ((threadIdx.x & 63) == 0) lds[q * (NT / 64) + (threadIdx.x >> 6)] = v[q];
     }
     __syncthreads();
-    if (!amLast) return false;
-    const int b0 = S.first[inst], b1 = S.first[inst + 1];
-    for (int q = 0; q < nq; ++q) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        sum[q] = 0;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) sum[q] += lds[q * (NT / 64) + w];
+    }
+    __syncthreads();
+}
+
+// the workgroup's sums of v, to parts[q * stride]
+template <int NT, int NQ>
+__device__ __forceinline__ void seg_part(double (&v)[NQ], double *lds, double *parts, int stride)
+{
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
+        if ((threadIdx.x & 63) == 0) lds[q * (NT / 64) + (threadIdx.x >> 6)] = v[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < NQ) {
         double s = 0;
-        for (int b = b0 + threadIdx.x; b < b1; b += SEG_THREADS)
-            s += read_partial(&S.partials[(size_t)q * nb + b]);
-        const double t = block_sum(s, lds2);
-        if (threadIdx.x == 0) tot[q] = t;
-        __syncthreads();
+        for (int w = 0; w < NT / 64; ++w) s += lds[threadIdx.x * (NT / 64) + w];
+        parts[(size_t)threadIdx.x * stride] = s;
     }
-    if (threadIdx.x == 0) reset_counter(&S.counter[inst]);
-    return true;
 }
 
-enum { SEG_INIT = 0, SEG_QH = 1, SEG_UPD = 2, SEG_RES64 = 3 };
-
-// MODE INIT  : p = b, q = s = dinv b; res = <p,s>, rr = <p,p>, bn2 = <b,b>
-// MODE QH    : alpha = res / <q, h>
-// MODE UPD   : x += a q, p -= a h, s = dinv p; res, rr, beta, it, done
-// MODE RES64 : r = b - h (FP64); rn = ||r||, bn2 = ||b||^2, conv
-template <typename T, int MODE>
-__global__ void __launch_bounds__(SEG_THREADS)
-    k_seg(SegTab S, BState B, T *__restrict__ x, T *__restrict__ p, T *__restrict__ q, const T *__restrict__ h,
-          T *__restrict__ s, const T *__restrict__ b, const T *__restrict__ dinv, double eps)
+// f(i, k): the loads of DoF i into slot k; g(i, k): its update
+template <typename F, typename G>
+__device__ __forceinline__ void seg_loop(int64_t lo, int64_t hi, F f, G g)
 {
-    __shared__ double lds[SEG_THREADS / 64];
+    for (int64_t i0 = lo; i0 < hi; i0 += SEG_CHUNK) {
+#pragma unroll
+        for (int k = 0; k < SEG_ITEMS; ++k) {
+            const int64_t i = i0 + threadIdx.x + (int64_t)k * SEG_THREADS;
+            f(i < hi ? i : lo, k);
+        }
+#pragma unroll
+        for (int k = 0; k < SEG_ITEMS; ++k) {
+            const int64_t i = i0 + threadIdx.x + (int64_t)k * SEG_THREADS;
+            if (i < hi) g(i, k);
+        }
+    }
+}
+
+// start of an inner solve: p = scale r (FP32), s = dinv p, x = 0; partials of
+// <p, s>, <p, p>
+__global__ void __launch_bounds__(SEG_THREADS)
+    k_bcg_init(SegTab S, BState B, const double *__restrict__ r, const float *__restrict__ dinv, float *__restrict__ x,
+               float *__restrict__ p, float *__restrict__ s, double eps, int maxit)
+{
+    __shared__ double lds[2 * SEG_THREADS / 64];
     const int inst = S.inst[blockIdx.x];
-    const bool skip = (MODE == SEG_RES64) ? B.conv[inst] != 0 : B.done[inst] != 0;
+    const bool skip = B.conv[inst] != 0;
+    if (threadIdx.x == 0) {
+        if (blockIdx.x == 0) {
+            *B.eps2 = eps * eps;   // relative reduction of the true residual
+            *B.maxit = maxit;
+        }
+        if (S.first[inst] == (int)blockIdx.x) {
+            B.done[inst] = B.idle[inst] = skip;
+            B.it[inst] = 0;
+        }
+    }
     if (skip) return;   // uniform over the block
-    const int64_t lo = S.lo[blockIdx.x], hi = S.hi[blockIdx.x];
-    double a0 = 0, a1 = 0, a2 = 0;
-    const double alpha = (MODE == SEG_UPD) ? B.alpha[inst] : 0.0;
-    // a segment is at most SEG_CHUNK = SEG_ITEMS * SEG_THREADS DoFs: every
-    // thread issues all of its loads before it uses them (memory-level
-    // parallelism), then updates and accumulates
-    constexpr int U = SEG_ITEMS;
-    T va[U], vb[U], vc[U];
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-        const int64_t i = lo + threadIdx.x + (int64_t)k * SEG_THREADS;
-        va[k] = vb[k] = vc[k] = T(0);
-        if (i < hi) {
-            if (MODE == SEG_INIT) {
-                va[k] = b[i];
-                vb[k] = dinv[i];
-            } else if (MODE == SEG_QH) {
-                va[k] = q[i];
-                vb[k] = h[i];
-            } else if (MODE == SEG_UPD) {
-                va[k] = p[i];
-                vb[k] = h[i];
-                vc[k] = dinv[i];
-            } else {
-                va[k] = b[i];
-                vb[k] = h[i];
-            }
-        }
-    }
-    T vx[U], vq[U];
-    if (MODE == SEG_UPD) {
-#pragma unroll
-        for (int k = 0; k < U; ++k) {
-            const int64_t i = lo + threadIdx.x + (int64_t)k * SEG_THREADS;
-            vx[k] = vq[k] = T(0);
-            if (i < hi) {
-                vx[k] = x[i];
-                vq[k] = q[i];
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-        const int64_t i = lo + threadIdx.x + (int64_t)k * SEG_THREADS;
-        if (i >= hi) continue;
-        if (MODE == SEG_INIT) {
-            const T bv = va[k];
-            const T sv = vb[k] * bv;
-            p[i] = bv;
-            q[i] = sv;
-            s[i] = sv;
-            a0 += (double)bv * (double)sv;
-            a1 += (double)bv * (double)bv;
-        } else if (MODE == SEG_QH) {
-            a0 += (double)va[k] * (double)vb[k];
-        } else if (MODE == SEG_UPD) {
-            x[i] = (T)((double)vx[k] + alpha * (double)vq[k]);
-            const T pn = (T)((double)va[k] - alpha * (double)vb[k]);
-            p[i] = pn;
-            const T sv = vc[k] * pn;
-            s[i] = sv;
-            a0 += (double)pn * (double)sv;
-            a1 += (double)pn * (double)pn;
-        } else {
-            const double r = (double)va[k] - (double)vb[k];
-            p[i] = (T)r;
-            a0 += r * r;
-            a2 += (double)va[k] * (double)va[k];
-        }
-    }
-    double own[3];
-    own[0] = bsum(a0, lds);
-    __syncthreads();
-    own[1] = bsum(a1, lds);
-    __syncthreads();
-    own[2] = bsum(a2, lds);
-    double tot[3];
-    if (!seg_finish(S, inst, 3, own, tot) || threadIdx.x != 0) return;
-    if (MODE == SEG_INIT) {
-        B.res[inst] = tot[0];
-        B.rr[inst] = tot[1];
-        B.tol[inst] = eps * eps * tot[1];   // relative reduction of the true residual
-        B.it[inst] = 0;
-        B.done[inst] = !(tot[1] > B.tol[inst]) || B.maxit <= 0;
-    } else if (MODE == SEG_QH) {
-        B.alpha[inst] = B.res[inst] / tot[0];
-    } else if (MODE == SEG_UPD) {
-        const double r = tot[0];
-        B.prev[inst] = B.res[inst];
-        B.beta[inst] = r / B.res[inst];
-        B.res[inst] = r;
-        B.rr[inst] = tot[1];
-        B.it[inst] += 1;
-        B.done[inst] = !(tot[1] > B.tol[inst]) || B.it[inst] >= B.maxit;
-    } else {
-        const double rn = sqrt(tot[0]);
-        B.rn[inst] = rn;
-        B.bn2[inst] = tot[2];
-        B.conv[inst] = rn <= eps * sqrt(tot[2]);
-        B.scale[inst] = rn > 0 ? 1.0 / rn : 1.0;
-    }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(SEG_THREADS)
-    k_seg_qupd(SegTab S, BState B, T *__restrict__ q, const T *__restrict__ s)
-{
-    const int inst = S.inst[blockIdx.x];
-    if (B.done[inst] || B.it[inst] == 0) return;
-    const double beta = B.beta[inst];
-    const int64_t lo = S.lo[blockIdx.x], hi = S.hi[blockIdx.x];
-    T vq[SEG_ITEMS], vs[SEG_ITEMS];
-#pragma unroll
-    for (int k = 0; k < SEG_ITEMS; ++k) {
-        const int64_t i = lo + threadIdx.x + (int64_t)k * SEG_THREADS;
-        vq[k] = vs[k] = T(0);
-        if (i < hi) {
-            vq[k] = q[i];
-            vs[k] = s[i];
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < SEG_ITEMS; ++k) {
-        const int64_t i = lo + threadIdx.x + (int64_t)k * SEG_THREADS;
-        if (i < hi) q[i] = (T)(beta * (double)vq[k] + (double)vs[k]);
-    }
-}
-
-// r32 = r64 * scale_i, d = 0, inner done = outer converged
-__global__ void __launch_bounds__(SEG_THREADS)
-    k_seg_to32(SegTab S, BState B, const double *__restrict__ r, float *__restrict__ r32, float *__restrict__ d)
-{
-    const int inst = S.inst[blockIdx.x];
     const double a = B.scale[inst];
-    for (int64_t i = S.lo[blockIdx.x] + threadIdx.x; i < S.hi[blockIdx.x]; i += SEG_THREADS) {
-        r32[i] = (float)(r[i] * a);
-        d[i] = 0.f;
+    double v[2] = {};
+    double vr[SEG_ITEMS];
+    float vd[SEG_ITEMS];
+    seg_loop(S.lo[blockIdx.x], S.hi[blockIdx.x],
+             [&](int64_t i, int k) {
+                 vr[k] = r[i];
+                 vd[k] = dinv[i];
+             },
+             [&](int64_t i, int k) {
+                 const float b = (float)(vr[k] * a), sv = vd[k] * b;
+                 x[i] = 0.f;
+                 p[i] = b;
+                 s[i] = sv;
+                 v[0] += (double)b * (double)sv;
+                 v[1] += (double)b * (double)b;
+             });
+    seg_part<SEG_THREADS, 2>(v, lds, S.parts + blockIdx.x, gridDim.x);
+}
+
+// first half of a step: the end of the last one (<p, s>, <p, p>, whether the
+// instance is done, beta), q = s + beta q on the way into the apply, h = A q and the
+// partials of <q, h>.  The nodes of an element are combined as they are read, by up
+// to four elements, so the new q goes to a second buffer.
+template <int TX, int TY>
+__global__ void __launch_bounds__((TX + 1) * (TY + 1))
+    k_bcg_apply(SegTab S, BState B, const CGInst *__restrict__ insts, const int *__restrict__ tile_inst,
+                const float *__restrict__ kvol, const float *__restrict__ s, const float *__restrict__ q,
+                float *__restrict__ qn, float *__restrict__ h, double *__restrict__ dot, int nseg)
+{
+    constexpr int NT = (TX + 1) * (TY + 1);
+    __shared__ float xch[5][NT];
+    __shared__ double lds[2 * ((NT + 63) / 64)];
+    const int bid = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int ii = tile_inst[bid];
+    if (B.idle[ii]) return;
+    const CGInst P = insts[ii];
+    const CGTile t = cg_tile<TX, TY>(P, bid);
+    const int it = B.it[ii];
+    float ul[3][3] = {}, uo[3][3] = {}, wl[3][3] = {}, kap[9] = {};
+    const int64_t e = P.elem_off + (int64_t)t.ey * P.nx + t.ex;
+    if (t.valid) {
+        const float *se = s + P.dof_off, *qe = q + P.dof_off;
+#pragma unroll
+        for (int iy = 0; iy < 3; ++iy)
+#pragma unroll
+            for (int ix = 0; ix < 3; ++ix) {
+                const int64_t n = (int64_t)(2 * t.ey + iy) * t.NX + 2 * t.ex + ix;
+                ul[iy][ix] = se[n];
+                if (it) uo[iy][ix] = qe[n];
+            }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) kap[k] = kvol[e * 9 + k];
     }
-    if (threadIdx.x == 0 && S.first[inst] == (int)blockIdx.x) B.done[inst] = B.conv[inst];
+    double r[2];
+    seg_sum<NT, 2>(S.parts, S.parts + nseg, S.first[ii], S.first[ii + 1], lds, r);
+    const double tol = it ? B.tol[ii] : *B.eps2 * r[1];
+    const bool done = !(r[1] > tol) || it >= *B.maxit;
+    const double beta = it ? r[0] / B.prev[ii] : 0.0;
+    if (bid == P.tile_off && threadIdx.x == 0) {
+        B.res[ii] = r[0];
+        B.done[ii] = done;
+        if (!it) B.tol[ii] = tol;
+    }
+    if (done) return;
+    if (it)
+#pragma unroll
+        for (int iy = 0; iy < 3; ++iy)
+#pragma unroll
+            for (int ix = 0; ix < 3; ++ix) ul[iy][ix] = (float)(beta * (double)uo[iy][ix] + (double)ul[iy][ix]);
+    if (t.valid) {
+        const float c = (float)P.c * (float)P.detJ;
+        cg_element<float, true>(ul, kap, (float)P.sx, (float)P.sy, [&](float, int) { return c; }, wl);
+    }
+    float *he = h + P.dof_off, *qo = qn + P.dof_off;
+    double d[1] = {};
+    cg_gather<TX, TY, float>(P, t, wl, xch, [&](int64_t node, bool bnd, int iy, int ix, float v) {
+        if (bnd) v = ul[iy][ix];
+        he[node] = v;
+        qo[node] = ul[iy][ix];
+        d[0] += (double)ul[iy][ix] * (double)v;
+    });
+    seg_part<NT, 1>(d, lds, dot + bid, 0);
+}
+
+// second half: alpha = <p, s> / <q, h>, x += alpha q, p -= alpha h, s = dinv p, and
+// the partials of <p, s>, <p, p>
+__global__ void __launch_bounds__(SEG_THREADS)
+    k_bcg_update(SegTab S, BState B, const int *__restrict__ tile_first, const double *__restrict__ dot,
+                 const float *__restrict__ dinv, const float *__restrict__ q, const float *__restrict__ h,
+                 float *__restrict__ x, float *__restrict__ p, float *__restrict__ s)
+{
+    __shared__ double lds[2 * SEG_THREADS / 64];
+    const int inst = S.inst[blockIdx.x];
+    if (B.done[inst]) {
+        if (S.first[inst] == (int)blockIdx.x && threadIdx.x == 0) B.idle[inst] = 1;
+        return;
+    }
+    float vp[SEG_ITEMS], vh[SEG_ITEMS], vd[SEG_ITEMS], vx[SEG_ITEMS], vq[SEG_ITEMS];
+    const int64_t lo = S.lo[blockIdx.x], hi = S.hi[blockIdx.x];
+    double qh[1], v[2] = {};
+    seg_sum<SEG_THREADS, 1>(dot, nullptr, tile_first[inst], tile_first[inst + 1], lds, qh);
+    const double res = B.res[inst], alpha = res / qh[0];
+    if (S.first[inst] == (int)blockIdx.x && threadIdx.x == 0) {
+        B.prev[inst] = res;
+        B.it[inst] += 1;
+    }
+    seg_loop(lo, hi,
+             [&](int64_t i, int k) {
+                 vp[k] = p[i];
+                 vh[k] = h[i];
+                 vd[k] = dinv[i];
+                 vx[k] = x[i];
+                 vq[k] = q[i];
+             },
+             [&](int64_t i, int k) {
+                 x[i] = (float)((double)vx[k] + alpha * (double)vq[k]);
+                 const float pn = (float)((double)vp[k] - alpha * (double)vh[k]), sv = vd[k] * pn;
+                 p[i] = pn;
+                 s[i] = sv;
+                 v[0] += (double)pn * (double)sv;
+                 v[1] += (double)pn * (double)pn;
+             });
+    seg_part<SEG_THREADS, 2>(v, lds, S.parts + blockIdx.x, gridDim.x);
+}
+
+// the sum of part[lo .. hi) by one wavefront
+__device__ __forceinline__ double wave_parts(const double *part, int lo, int hi)
+{
+    double v = 0;
+    for (int k = lo + (int)(threadIdx.x & 63); k < hi; k += 64) v += part[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// the instances still at work, a wavefront per instance: RES64 = false, after a
+// step (the test of the next apply); true, after the residual (rn, bn2, conv, scale)
+template <bool RES64>
+__global__ void __launch_bounds__(1024) k_batch_look(SegTab S, BState B, int count, int nseg, double eps, int *out)
+{
+    __shared__ int active;
+    if (threadIdx.x == 0) active = 0;
+    __syncthreads();
+    for (int i = threadIdx.x >> 6; i < count; i += 1024 / 64) {
+        const double a = wave_parts(S.parts, S.first[i], S.first[i + 1]),
+                     b = wave_parts(S.parts + nseg, S.first[i], S.first[i + 1]);
+        if ((threadIdx.x & 63) != 0) continue;
+        if (RES64) {
+            if (!B.conv[i]) {
+                const double rn = sqrt(a);
+                B.rn[i] = rn;
+                B.bn2[i] = b;
+                B.conv[i] = rn <= eps * sqrt(b);
+                B.scale[i] = rn > 0 ? 1.0 / rn : 1.0;
+            }
+            if (!B.conv[i]) atomicAdd(&active, 1);
+        } else if (!B.done[i]) {
+            if (!(b > B.tol[i]) || B.it[i] >= *B.maxit) B.done[i] = B.idle[i] = 1;
+            else atomicAdd(&active, 1);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) *out = active;
+}
+
+// r = b - h (FP64) and the partials of <r, r>, <b, b>
+__global__ void __launch_bounds__(SEG_THREADS)
+    k_seg_res64(SegTab S, BState B, const double *__restrict__ b, const double *__restrict__ h, double *__restrict__ r)
+{
+    __shared__ double lds[2 * SEG_THREADS / 64];
+    if (B.conv[S.inst[blockIdx.x]]) return;
+    double vb[SEG_ITEMS], vh[SEG_ITEMS], v[2] = {};
+    seg_loop(S.lo[blockIdx.x], S.hi[blockIdx.x],
+             [&](int64_t i, int k) {
+                 vb[k] = b[i];
+                 vh[k] = h[i];
+             },
+             [&](int64_t i, int k) {
+                 const double d = vb[k] - vh[k];
+                 r[i] = d;
+                 v[0] += d * d;
+                 v[1] += vb[k] * vb[k];
+             });
+    seg_part<SEG_THREADS, 2>(v, lds, S.parts + blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(SEG_THREADS)
@@ -238,18 +329,6 @@ __global__ void __launch_bounds__(SEG_THREADS)
     const double a = 1.0 / B.scale[inst];
     for (int64_t i = S.lo[blockIdx.x] + threadIdx.x; i < S.hi[blockIdx.x]; i += SEG_THREADS)
         x[i] += a * (double)d[i];
-}
-
-__global__ void k_count_active(const int *done, int n, int *out)
-{
-    __shared__ int c;
-    if (threadIdx.x == 0) c = 0;
-    __syncthreads();
-    int mine = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) mine += done[i] ? 0 : 1;
-    atomicAdd(&c, mine);
-    __syncthreads();
-    if (threadIdx.x == 0) *out = c;
 }
 
 template <typename T>
@@ -289,6 +368,11 @@ void Batch::init(Context *c, int n, const int *nx_, const int *ny_, double c_)
             I.tile_off = (int)of.size();
             of.insert(of.end(), I.ntiles, i);
         }
+        std::vector<int> tf(n + 1);
+        for (int i = 0; i < n; ++i) tf[i] = v[i].tile_off;
+        tf[n] = (int)of.size();
+        tile_first[sh].alloc(sizeof(int) * (n + 1));
+        FEM_HIP(hipMemcpy(tile_first[sh].p, tf.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice));
         tile_inst[sh].alloc(sizeof(int) * of.size());
         FEM_HIP(hipMemcpy(tile_inst[sh].p, of.data(), sizeof(int) * of.size(), hipMemcpyHostToDevice));
         tiles[sh] = (int)of.size();
@@ -303,10 +387,12 @@ void Batch::init(Context *c, int n, const int *nx_, const int *ny_, double c_)
     std::vector<int64_t> slo, shi;
     for (int i = 0; i < n; ++i) {
         first[i] = (int)sinst.size();
-        for (int64_t a = dof_off[i]; a < dof_off[i + 1]; a += SEG_CHUNK) {
+        const int64_t nd = dof_off[i + 1] - dof_off[i], most = (int64_t)SEG_MOST * SEG_CHUNK;
+        const int64_t len = SEG_CHUNK * ((nd + most - 1) / most);
+        for (int64_t a = dof_off[i]; a < dof_off[i + 1]; a += len) {
             sinst.push_back(i);
             slo.push_back(a);
-            shi.push_back(std::min<int64_t>(a + SEG_CHUNK, dof_off[i + 1]));
+            shi.push_back(std::min<int64_t>(a + len, dof_off[i + 1]));
         }
     }
     first[n] = (int)sinst.size();
@@ -315,16 +401,14 @@ void Batch::init(Context *c, int n, const int *nx_, const int *ny_, double c_)
     seg_lo.alloc(sizeof(int64_t) * nseg);
     seg_hi.alloc(sizeof(int64_t) * nseg);
     seg_first.alloc(sizeof(int) * (n + 1));
-    seg_counter.alloc(sizeof(unsigned) * n);
-    seg_partials.alloc(sizeof(double) * 3 * nseg);
+    seg_parts.alloc(sizeof(double) * 2 * nseg);
     FEM_HIP(hipMemcpy(seg_inst.p, sinst.data(), sizeof(int) * nseg, hipMemcpyHostToDevice));
     FEM_HIP(hipMemcpy(seg_lo.p, slo.data(), sizeof(int64_t) * nseg, hipMemcpyHostToDevice));
     FEM_HIP(hipMemcpy(seg_hi.p, shi.data(), sizeof(int64_t) * nseg, hipMemcpyHostToDevice));
     FEM_HIP(hipMemcpy(seg_first.p, first.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice));
-    FEM_HIP(hipMemset(seg_counter.p, 0, sizeof(unsigned) * n));
     // per-instance state
-    sdbl.alloc(sizeof(double) * 9 * n);
-    sint.alloc(sizeof(int) * 3 * n);
+    sdbl.alloc(sizeof(double) * (6 * n + 1));
+    sint.alloc(sizeof(int) * (4 * n + 1));
     FEM_HIP(hipMemset(sdbl.p, 0, sdbl.bytes));
     FEM_HIP(hipMemset(sint.p, 0, sint.bytes));
     active.alloc(sizeof(int));
@@ -440,68 +524,80 @@ void Batch::solve(const Vec &b, Vec &x, double tol, double inner_tol, int inner_
         drop_graph();
         h64.alloc(sizeof(double) * N);
         r64.alloc(sizeof(double) * N);
-        for (DevBuf *v : { &r32, &d32, &p32, &q32, &s32, &h32 }) v->alloc(sizeof(float) * N);
+        for (DevBuf *v : { &d32, &p32, &q32[0], &q32[1], &s32, &h32 }) v->alloc(sizeof(float) * N);
+        dot_parts.alloc(sizeof(double) * *std::max_element(tiles, tiles + CG_NSHAPES));
     }
     const int n = count;
     double *D = sdbl.as<double>();
     int *I = sint.as<int>();
-    BState B{ D, D + n, D + 2 * n, D + 3 * n, D + 4 * n, D + 5 * n, D + 6 * n, D + 7 * n, D + 8 * n,
-              I, I + n, I + 2 * n, inner_maxit };
+    BState B{ D, D + n, D + 2 * n, D + 3 * n, D + 4 * n, D + 5 * n, D + 6 * n, I, I + n, I + 2 * n, I + 3 * n, I + 4 * n };
     SegTab S{ seg_inst.as<int>(), seg_lo.as<int64_t>(), seg_hi.as<int64_t>(), seg_first.as<int>(),
-              seg_counter.as<unsigned>(), seg_partials.as<double>() };
-    float *r32p = r32.as<float>(), *d = d32.as<float>(), *p = p32.as<float>(), *q = q32.as<float>(),
-          *s = s32.as<float>(), *h = h32.as<float>();
+              seg_parts.as<double>() };
+    float *d = d32.as<float>(), *p = p32.as<float>(), *s = s32.as<float>(), *h = h32.as<float>();
     const float *dv = dinv32.as<float>();
-    auto step = [&](hipStream_t ss) {
-        hipLaunchKernelGGL(k_seg_qupd<float>, dim3(nseg), dim3(SEG_THREADS), 0, ss, S, B, q, s);
-        if (shape >= 0)
-            cg_launch_shape<float>(shape, CG_MODE_APPLY, inst_dev[shape].as<CGInst>(), tile_inst[shape].as<int>(),
-                                   tiles[shape], tab.as<CGTab>(), kvol32.as<float>(), q, h, nullptr, B.done, ss,
-                                   CGReaction<float>(), creac != 0);
-        hipLaunchKernelGGL((k_seg<float, SEG_QH>), dim3(nseg), dim3(SEG_THREADS), 0, ss, S, B, d, p, q, h, s, r32p, dv, 0.0);
-        hipLaunchKernelGGL((k_seg<float, SEG_UPD>), dim3(nseg), dim3(SEG_THREADS), 0, ss, S, B, d, p, q, h, s, r32p, dv, 0.0);
+    auto step = [&](hipStream_t ss, int k) {
+        const float *q = q32[k & 1].as<float>();
+        float *qn = q32[(k + 1) & 1].as<float>();
+        const auto apply = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(tiles[shape]),
+                               dim3((CG_SHAPES[shape][0] + 1) * (CG_SHAPES[shape][1] + 1)), 0, ss, S, B,
+                               inst_dev[shape].as<CGInst>(), tile_inst[shape].as<int>(), kvol32.as<float>(), s, q, qn, h,
+                               dot_parts.as<double>(), nseg);
+        };
+        switch (shape) {
+        case 0: apply(k_bcg_apply<15, 15>); break;
+        case 1: apply(k_bcg_apply<7, 7>); break;
+        case 2: apply(k_bcg_apply<15, 7>); break;
+        case 3: apply(k_bcg_apply<31, 7>); break;
+        default: apply(k_bcg_apply<7, 31>); break;
+        }
+        hipLaunchKernelGGL(k_bcg_update, dim3(nseg), dim3(SEG_THREADS), 0, ss, S, B, tile_first[shape].as<int>(),
+                           dot_parts.as<double>(), dv, qn, h, d, p, s);
+        FEM_HIP(hipGetLastError());
     };
     if (use_graph && !graph_exec) {
         FEM_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        step(st);
+        for (int k = 0; k < GRAPH_STEPS; ++k) step(st, k);
         FEM_HIP(hipStreamEndCapture(st, &graph));
         FEM_HIP(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
     }
     FEM_HIP(hipMemsetAsync(B.conv, 0, sizeof(int) * n, st));   // not captured
+    // the number of instances still at work
+    auto look = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), 0, st, S, B, n, nseg, tol, active.as<int>());
+        FEM_HIP(hipGetLastError());
+        FEM_HIP(hipMemcpyAsync(hactive, active.p, sizeof(int), hipMemcpyDeviceToHost, st));
+        FEM_HIP(hipStreamSynchronize(st));
+        return *hactive;
+    };
     int outer = 0, total_inner = 0;
     std::vector<int> its(n, 0);
     while (true) {
-        // FP64 true residual per instance
-        apply_raw(FEM_F64, x.data, h64.p, nullptr);
-        hipLaunchKernelGGL((k_seg<double, SEG_RES64>), dim3(nseg), dim3(SEG_THREADS), 0, st, S, B, (double *)nullptr,
-                           r64.as<double>(), (double *)nullptr, h64.as<double>(), (double *)nullptr,
-                           (const double *)b.data, (const double *)nullptr, tol);
-        FEM_HIP(hipGetLastError());
-        // clear conv flags only on the first pass (k_seg RES64 skips converged instances)
-        hipLaunchKernelGGL(k_count_active, dim3(1), dim3(256), 0, st, B.conv, n, active.as<int>());
-        FEM_HIP(hipMemcpyAsync(hactive, active.p, sizeof(int), hipMemcpyDeviceToHost, st));
-        FEM_HIP(hipStreamSynchronize(st));
-        if (*hactive == 0 || outer >= max_outer) break;
-        hipLaunchKernelGGL(k_seg_to32, dim3(nseg), dim3(SEG_THREADS), 0, st, S, B, r64.as<double>(), r32p, d);
-        hipLaunchKernelGGL((k_seg<float, SEG_INIT>), dim3(nseg), dim3(SEG_THREADS), 0, st, S, B, d, p, q, h, s, r32p, dv, inner_tol);
-        FEM_HIP(hipGetLastError());
-        int chunk = 8, done_steps = 0;
+        // FP64 true residual per instance (those that have converged are skipped)
+        apply_raw(FEM_F64, x.data, h64.p, B.conv);
+        hipLaunchKernelGGL(k_seg_res64, dim3(nseg), dim3(SEG_THREADS), 0, st, S, B, (const double *)b.data,
+                           h64.as<double>(), r64.as<double>());
+        if (look(k_batch_look<true>) == 0 || outer >= max_outer) break;
+        hipLaunchKernelGGL(k_bcg_init, dim3(nseg), dim3(SEG_THREADS), 0, st, S, B, r64.as<double>(), dv, d, p, s, inner_tol,
+                           inner_maxit);
+        int chunk = 8, done_steps = 0;   // multiples of GRAPH_STEPS
         while (true) {
-            for (int c = 0; c < chunk; ++c) {
+            for (int c = 0; c < chunk; c += use_graph ? GRAPH_STEPS : 1) {
                 if (use_graph) FEM_HIP(hipGraphLaunch(graph_exec, st));
-                else step(st);
+                else step(st, c);
             }
             done_steps += chunk;
-            hipLaunchKernelGGL(k_count_active, dim3(1), dim3(256), 0, st, B.done, n, active.as<int>());
-            FEM_HIP(hipMemcpyAsync(hactive, active.p, sizeof(int), hipMemcpyDeviceToHost, st));
-            FEM_HIP(hipStreamSynchronize(st));
-            if (*hactive == 0 || done_steps >= inner_maxit) break;
+            if (look(k_batch_look<false>) == 0 || done_steps >= inner_maxit) break;
             if (chunk < 64) chunk *= 2;
         }
         std::vector<int> it(n);
         FEM_HIP(hipMemcpy(it.data(), B.it, sizeof(int) * n, hipMemcpyDeviceToHost));
         int mx = 0;
-        for (int i = 0; i < n; ++i) { its[i] += it[i]; mx = std::max(mx, it[i]); total_inner += it[i]; }
+        for (int i = 0; i < n; ++i) {
+            its[i] += it[i];
+            mx = std::max(mx, it[i]);
+            total_inner += it[i];
+        }
         info.max_inner_iterations += mx;
         hipLaunchKernelGGL(k_seg_upd64, dim3(nseg), dim3(SEG_THREADS), 0, st, S, B, (double *)x.data, d);
         FEM_HIP(hipGetLastError());

@@ -15,16 +15,16 @@ struct Batch {
     int shape = 0;                       // index into CG_SHAPES
     float tune_ms[CG_NSHAPES] = {};
     DevBuf inst_dev[CG_NSHAPES];
-    DevBuf tile_inst[CG_NSHAPES];        // the instance of each tile
+    DevBuf tile_inst[CG_NSHAPES], tile_first[CG_NSHAPES];   // the instance of each tile, the first tile of each
     int tiles[CG_NSHAPES] = {};
     DevBuf tab, kvol64, kvol32, dinv64, dinv32;
-    DevBuf seg_inst, seg_lo, seg_hi, seg_first, seg_counter, seg_partials;
+    DevBuf seg_inst, seg_lo, seg_hi, seg_first, seg_parts, dot_parts;
     int nseg = 0;
     DevBuf sdbl, sint, active;
     int *hactive = nullptr;
-    DevBuf h64, r64, r32, d32, p32, q32, s32, h32;
-    // one captured inner CG step; it holds the addresses of the work,
-    // coefficient and Jacobi buffers, so it is dropped whenever one of them
+    DevBuf h64, r64, d32, p32, q32[2], s32, h32;
+    // a few captured inner CG steps; they hold the addresses of the work,
+    // coefficient and Jacobi buffers, so they are dropped whenever one of them
     // is (re)allocated or the tile shape changes
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;

@@ -54,3 +54,29 @@ def test_q2_cg_with_the_applys_partials(ctx, n):
     # 1e-12 of |F| times the condition of the Jacobi-scaled operator, below 1e5
     # on these meshes and coefficients
     assert np.abs(X.download() - u).max() < 1e-6 * np.abs(u).max()
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_batch_steps_over_uneven_instances(ctx, use_graph):
+    """Instances of one tile and of many, one with a zero load (done at its
+    first step), two solves with different step limits: a limit of one step
+    per refinement must hold in a replayed graph as well."""
+    sides = [(1, 1), (15, 15), (31, 46), (64, 3), (16, 16)]
+    rng = np.random.default_rng(4)
+    kv = [np.exp(rng.normal(size=(a * b, 9))) for a, b in sides]
+    fq = [rng.normal(size=(a * b, 9)) * (i != 4) for i, (a, b) in enumerate(sides)]
+    B = fa.Batch(ctx, sides)
+    B.set_kappa_qp(np.concatenate(kv))
+    F = B.rhs(np.concatenate(fq))
+    X = B.vector()
+    info = B.solve(F, X, tol=1e-10, use_graph=use_graph)
+    assert info["converged"] == len(sides) and info["iterations"][4] == 0
+    x, f = X.download(), F.download()
+    for i, s in enumerate(sides):
+        lo, hi = B.offsets[i], B.offsets[i + 1]
+        r = f[lo:hi] - ora.CGOperator(s, kappa=kv[i]).apply(x[lo:hi])
+        assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(f[lo:hi])
+    Y = B.vector()
+    info = B.solve(F, Y, tol=1e-10, inner_maxit=1, max_outer=3, use_graph=use_graph)
+    assert info["outer_iterations"] == 3 and info["max_inner_iterations"] == 3
+    assert all(n <= 3 for n in info["iterations"])
