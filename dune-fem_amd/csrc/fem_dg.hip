@@ -1179,34 +1179,44 @@ void dg_diagonal(const DGArgs<double> &a, int k, double *d, hipStream_t s)
 // exact element-block inverse for cellwise kappa without advection
 // ---------------------------------------------------------------------------
 // cyclic Jacobi eigenvalue iteration for a symmetric K x K matrix
-__device__ void sym_eig(int K, double (*A)[KMAX], double (*Q)[KMAX])
+template <int K>
+__device__ __forceinline__ void sym_eig(double (&A)[K][K], double (&Q)[K][K])
 {
+#pragma unroll
     for (int r = 0; r < K; ++r)
+#pragma unroll
         for (int c = 0; c < K; ++c) Q[r][c] = (r == c) ? 1.0 : 0.0;
     for (int sweep = 0; sweep < 50; ++sweep) {
         double off = 0, tot = 0;
+#pragma unroll
         for (int r = 0; r < K; ++r)
+#pragma unroll
             for (int c = 0; c < K; ++c) {
                 tot += A[r][c] * A[r][c];
                 if (r != c) off += A[r][c] * A[r][c];
             }
         if (off <= 1e-30 * tot) break;
+#pragma unroll
         for (int p = 0; p < K - 1; ++p)
+#pragma unroll
             for (int q = p + 1; q < K; ++q) {
                 if (A[p][q] == 0.0) continue;
                 const double theta = (A[q][q] - A[p][p]) / (2.0 * A[p][q]);
                 const double tt = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
                 const double cs = 1.0 / sqrt(tt * tt + 1.0), sn = tt * cs;
+#pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const double akp = A[k][p], akq = A[k][q];
                     A[k][p] = cs * akp - sn * akq;
                     A[k][q] = sn * akp + cs * akq;
                 }
+#pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const double apk = A[p][k], aqk = A[q][k];
                     A[p][k] = cs * apk - sn * aqk;
                     A[q][k] = sn * apk + cs * aqk;
                 }
+#pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const double qkp = Q[k][p], qkq = Q[k][q];
                     Q[k][p] = cs * qkp - sn * qkq;
@@ -1216,9 +1226,12 @@ __device__ void sym_eig(int K, double (*A)[KMAX], double (*Q)[KMAX])
     }
 }
 
-template <typename TO>
-__global__ void k_dg_block_setup(const DGArgs<double> a, int K, TO *__restrict__ Qout, TO *__restrict__ lam,
-                                 bool bound)
+// One thread per element and direction.  K is a template argument so that the
+// matrices of the iteration stay in registers: with run-time loops they lay in
+// scratch (24^3 elements, K = 3: 34 us, now 13.7 us).
+template <int K, typename TO>
+__global__ void __launch_bounds__(128)
+    k_dg_block_setup(const DGArgs<double> a, TO *__restrict__ Qout, TO *__restrict__ lam, bool bound)
 {
     const int64_t E = (int64_t)a.n[0] * a.n[1] * a.n[2];
     const int64_t gid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1238,8 +1251,10 @@ __global__ void k_dg_block_setup(const DGArgs<double> a, int K, TO *__restrict__
         for (int q = 0; q < K * K * K; ++q) s += a.kvol[e * K * K * K + q];
         kin = s / (K * K * K);
     } else kin = a.kappa_const;
-    double M[KMAX][KMAX], Q[KMAX][KMAX];
+    double M[K][K], Q[K][K];
+#pragma unroll
     for (int r = 0; r < K; ++r)
+#pragma unroll
         for (int c = 0; c < K; ++c) M[r][c] = cd * kin / a.h[d] * tb.S[r][c];
     for (int s = 0; s < 2; ++s) {
         const double nrm = s ? 1.0 : -1.0;
@@ -1253,12 +1268,14 @@ __global__ void k_dg_block_setup(const DGArgs<double> a, int K, TO *__restrict__
             kp = 0.5 * (kin + kout);
         } else kp = kin;
         const double symw = interior ? 0.5 : 1.0;
+#pragma unroll
         for (int r = 0; r < K; ++r)
+#pragma unroll
             for (int c = 0; c < K; ++c)
                 M[r][c] += cd * (kp * a.beta / a.h[d] * tb.P[s][r] * tb.P[s][c] -
                                  symw * kin * nrm / a.h[d] * (tb.dP[s][c] * tb.P[s][r] + tb.P[s][c] * tb.dP[s][r]));
     }
-    sym_eig(K, M, Q);
+    sym_eig<K>(M, Q);
     // the reaction c + cvol (orthonormal basis: mass block |K| I) shifts
     // every eigenvalue sum; taken into the x direction, with the element's
     // weighted mean of cvol (exact for an element-constant reaction), or
@@ -1280,8 +1297,10 @@ __global__ void k_dg_block_setup(const DGArgs<double> a, int K, TO *__restrict__
         if (a.ccell) cm += a.ccell[e];
         shift = (a.c + (a.cvol && bound ? cmax : cm)) * a.h[0] * a.h[1] * a.h[2];
     }
+#pragma unroll
     for (int r = 0; r < K; ++r) {
         lam[(e * 3 + d) * K + r] = (TO)(M[r][r] + shift);
+#pragma unroll
         for (int c = 0; c < K; ++c) Qout[((e * 3 + d) * K + r) * K + c] = (TO)Q[r][c];
     }
 }
@@ -1290,7 +1309,16 @@ template <typename TO>
 void dg_block_setup(const DGArgs<double> &a, int k, TO *Q, TO *lam, hipStream_t s, bool bound)
 {
     const int64_t E = (int64_t)a.n[0] * a.n[1] * a.n[2];
-    hipLaunchKernelGGL(k_dg_block_setup<TO>, dim3(grid_for(E * 3, 128)), dim3(128), 0, s, a, k, Q, lam, bound);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid_for(E * 3, 128)), dim3(128), 0, s, a, Q, lam, bound);
+    };
+    switch (k) {
+    case 2: go(k_dg_block_setup<2, TO>); break;
+    case 3: go(k_dg_block_setup<3, TO>); break;
+    case 4: go(k_dg_block_setup<4, TO>); break;
+    case 5: go(k_dg_block_setup<5, TO>); break;
+    default: throw Error(FEM_ERR_UNSUPPORTED, "DG: order must be 1..4");
+    }
     FEM_HIP(hipGetLastError());
 }
 template void dg_block_setup<double>(const DGArgs<double> &, int, double *, double *, hipStream_t, bool);

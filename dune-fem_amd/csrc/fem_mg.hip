@@ -428,6 +428,10 @@ __global__ void k_mg_conforming(const DGArgs<double> a, VDims vd, double *__rest
                                 acc += area * mt * kap * (a.beta / a.h[d] * va * vb - nrm / a.h[d] * (da * vb + va * db));
                             }
                         }
+                        // (the 2-point rule integrates the products exactly)
+                        acc += (a.c + (a.ccell ? a.ccell[e] : 0.0)) * detJ * mg_m1(ca[0], cb[0]) * mg_m1(ca[1], cb[1]) *
+                               mg_m1(ca[2], cb[2]);
+                        if (!a.cvol) continue;
                         for (int qz = 0; qz < 2; ++qz)
                             for (int qy = 0; qy < 2; ++qy)
                                 for (int qx = 0; qx < 2; ++qx) {
@@ -438,9 +442,8 @@ __global__ void k_mg_conforming(const DGArgs<double> a, VDims vd, double *__rest
                                         pa *= ca[d] ? xq : 1.0 - xq;
                                         pb *= cb[d] ? xq : 1.0 - xq;
                                     }
-                                    const double r = a.c + (a.cvol ? a.cvol[e * 8 + qx + 2 * qy + 4 * qz] : 0.0) +
-                                                     (a.ccell ? a.ccell[e] : 0.0);
-                                    acc += tb.w[qx] * tb.w[qy] * tb.w[qz] * detJ * r * pa * pb;
+                                    acc += tb.w[qx] * tb.w[qy] * tb.w[qz] * detJ * a.cvol[e * 8 + qx + 2 * qy + 4 * qz] *
+                                           pa * pb;
                                 }
                     }
         }
@@ -448,65 +451,48 @@ __global__ void k_mg_conforming(const DGArgs<double> a, VDims vd, double *__rest
     }
 }
 
-// the Galerkin product P^T A_f P of a vertex level, directly: one thread per
-// coarse vertex V and stencil offset s (W = V + d(s)) sums
-// P(i, V) A_f(i, j) P(j, W) over the fine vertices i in the support of V
-// (per direction 2V-1 .. 2V+1, which holds the last fine vertex when it
-// belongs to V) and the 27 stencil neighbours j of i.  Offsets that leave
-// the coarse lattice hold 0.
-__global__ void k_mg_galerkin(VDims f, VDims cd, const double *__restrict__ Af, double *__restrict__ Ac)
+// The Galerkin product P^T A P of a vertex level, one direction at a time: P is the
+// product of three 1D interpolations, so coarsening direction D of the rows and of
+// the stencil's columns is a pass of its own,
+//   out(V, s) = sum_i P(i, V) sum_t P(i + t, V + s_D) in(i, s with s_D = t),
+// i = 2V-1 .. 2V+1 (which holds the last fine vertex when it belongs to V), t = -1 ..
+// 1: nine coefficients per entry, loaded together, 0 where a vertex lies outside.
+// All three directions in one kernel are up to 343 terms per entry behind branches
+// (25^3 and 13^3 vertices: 110 us each, now 11 us in three launches).  One thread per row of the lattice
+// c (coarse along D, as `f` along the others) and stencil offset.
+template <int D>
+__global__ void __launch_bounds__(MGT)
+    k_mg_galerkin(VDims f, VDims c, const double *__restrict__ in, double *__restrict__ out)
 {
-    const int64_t Vc = (int64_t)cd.n[0] * cd.n[1] * cd.n[2];
-    for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < Vc * 27; g += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t n = (int64_t)c.n[0] * c.n[1] * c.n[2] * 27;
+    const int nf = f.n[D], nc = c.n[D];
+    constexpr int SD = D == 0 ? 1 : D == 1 ? 3 : 9;
+    const int64_t fs = D == 0 ? 1 : D == 1 ? f.n[0] : (int64_t)f.n[0] * f.n[1];
+    for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n; g += (int64_t)gridDim.x * blockDim.x) {
         const int64_t v = g / 27;
         const int so = (int)(g - v * 27);
-        const int V[3] = { (int)(v % cd.n[0]), (int)((v / cd.n[0]) % cd.n[1]), (int)(v / ((int64_t)cd.n[0] * cd.n[1])) };
-        const int W[3] = { V[0] + so % 3 - 1, V[1] + (so / 3) % 3 - 1, V[2] + so / 9 - 1 };
+        int p[3] = { (int)(v % c.n[0]), (int)((v / c.n[0]) % c.n[1]), (int)(v / ((int64_t)c.n[0] * c.n[1])) };
+        const int V = p[D], W = V + (so / SD) % 3 - 1;
+        const int s0 = so - ((so / SD) % 3) * SD;
+        p[D] = 0;
+        const double *row = in + (p[0] + (int64_t)f.n[0] * (p[1] + (int64_t)f.n[1] * p[2])) * 27 + s0;
+        const bool wok = W >= 0 && W < nc;
         double acc = 0;
-        if (W[0] >= 0 && W[1] >= 0 && W[2] >= 0 && W[0] < cd.n[0] && W[1] < cd.n[1] && W[2] < cd.n[2]) {
-            // the 1D weights of V and W at the fine vertices 2V-1 .. 2V+1 and
-            // 2W-1 .. 2W+1 (the supports of both; 0 outside the lattice)
-            double wv[3][3], ww[3][3];
-            for (int d = 0; d < 3; ++d)
-                for (int m = 0; m < 3; ++m) {
-                    const int fv = 2 * V[d] - 1 + m, fw = 2 * W[d] - 1 + m;
-                    wv[d][m] = (fv >= 0 && fv < f.n[d]) ? w1(fv, V[d], f.n[d], cd.n[d]) : 0.0;
-                    ww[d][m] = (fw >= 0 && fw < f.n[d]) ? w1(fw, W[d], f.n[d], cd.n[d]) : 0.0;
-                }
-            const int sh[3] = { 2 * (V[0] - W[0]), 2 * (V[1] - W[1]), 2 * (V[2] - W[2]) };
-            for (int az = 0; az < 3; ++az) {
-                if (wv[2][az] == 0.0) continue;
-                const int iz = 2 * V[2] - 1 + az;
-                for (int ay = 0; ay < 3; ++ay) {
-                    if (wv[1][ay] == 0.0) continue;
-                    const int iy = 2 * V[1] - 1 + ay;
-                    for (int ax = 0; ax < 3; ++ax) {
-                        if (wv[0][ax] == 0.0) continue;
-                        const int ix = 2 * V[0] - 1 + ax;
-                        const double *a = Af + (ix + (int64_t)f.n[0] * (iy + (int64_t)f.n[1] * iz)) * 27;
-                        double row = 0;
-                        // neighbour j = i + t - 1 per direction sits at index
-                        // b = j - (2W - 1) = a + sh + t - 1 of W's support
-                        for (int tz = 0; tz < 3; ++tz) {
-                            const int bz = az + sh[2] + tz - 1;
-                            if (bz < 0 || bz > 2 || ww[2][bz] == 0.0) continue;
-                            for (int ty = 0; ty < 3; ++ty) {
-                                const int by = ay + sh[1] + ty - 1;
-                                if (by < 0 || by > 2 || ww[1][by] == 0.0) continue;
-                                const double pzy = ww[2][bz] * ww[1][by];
-                                for (int tx = 0; tx < 3; ++tx) {
-                                    const int bx = ax + sh[0] + tx - 1;
-                                    if (bx < 0 || bx > 2) continue;
-                                    row = fma(a[tx + 3 * ty + 9 * tz], pzy * ww[0][bx], row);
-                                }
-                            }
-                        }
-                        acc = fma(wv[2][az] * wv[1][ay] * wv[0][ax], row, acc);
-                    }
-                }
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const int i = 2 * V - 1 + m;
+            const bool ok = i >= 0 && i < nf && wok;
+            const double wv = ok ? w1(i, V, nf, nc) : 0.0;
+            const double *a = row + (ok ? i : 0) * fs * 27;
+            double r = 0;
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                const int j = i + t - 1;
+                r = fma(ok && j >= 0 && j < nf ? w1(j, W, nf, nc) : 0.0, a[t * SD], r);
             }
+            acc = fma(wv, r, acc);
         }
-        Ac[g] = acc;
+        out[g] = acc;
     }
 }
 
@@ -540,49 +526,91 @@ __global__ void k_mg_dense_fill(VDims d, const double *__restrict__ A, double *_
     }
 }
 
-// one pivot step of the in-place Gauss-Jordan inversion without pivoting
-// (X -> Y, pivot c): Y_cc = 1/p, Y_ck = X_ck / p, Y_rc = -X_rc / p, Y_rk =
-// X_rk - X_rc X_ck / p, p = X_cc.  After the steps c = 0..V-1 the matrix is
-// the inverse.  The pivots are the leading Schur complements' diagonals:
-// all positive exactly when the matrix is symmetric positive definite, for
-// which no pivoting is needed; they are recorded for the host to check.
-__device__ __forceinline__ double gj_entry(const double *__restrict__ X, int V, int c, double ip, int r, int k)
+// X -> Y: one block step of the in-place Gauss-Jordan inversion of a V x V matrix,
+// pivot rows and columns C = c .. c + GJ - 1 (the last step has fewer), with
+// P = X[C, C]^-1:
+//   Y[C, C] = P,  Y[C, k] = P X[C, k],  Y[r, C] = -X[r, C] P,
+//   Y[r, k] = X[r, k] - X[r, C] P X[C, k].
+// A launch has to see all of the step before it, so the inversion costs launches:
+// 11 block steps for 343 vertices 190 us, 172 steps of two pivots 690 us.  A workgroup makes
+// a GJ x GJ tile of Y and inverts the pivot block for itself in LDS, two pivots at a
+// time (the chain of a division and an LDS round trip per step is most of a launch:
+// one at a time 25 us).  Its pivots are those of the elimination without pivoting (the matrices are
+// symmetric positive definite); they are recorded for the host to check.
+constexpr int GJ = 32;
+__global__ void __launch_bounds__(256)
+    k_mg_gj_step(int V, int c, const double *__restrict__ X, double *__restrict__ Y, double *__restrict__ piv)
 {
-    if (r == c) return k == c ? ip : X[(int64_t)c * V + k] * ip;
-    if (k == c) return -X[(int64_t)r * V + c] * ip;
-    return X[(int64_t)r * V + k] - X[(int64_t)r * V + c] * X[(int64_t)c * V + k] * ip;
-}
-
-// `steps` (1 or 2) pivot steps c, c + 1 in one launch: the entries of the
-// intermediate matrix that step c + 1 reads (its own, row c + 1, column
-// c + 1) are formed from X by the same operations as in a launch of their
-// own, so the result equals two single steps bit for bit
-__global__ void k_mg_gj_step(int V, int c, int steps, const double *__restrict__ X, double *__restrict__ Y,
-                             double *__restrict__ piv)
-{
-    const int64_t V2 = (int64_t)V * V;
-    const double pc = X[(int64_t)c * V + c];
-    const double ip = 1.0 / pc;
-    const int c1 = c + 1;
-    const double pc1 = steps == 2 ? gj_entry(X, V, c, ip, c1, c1) : 1.0;
-    const double ip1 = 1.0 / pc1;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < V2; i += (int64_t)gridDim.x * blockDim.x) {
-        const int r = (int)(i / V), k = (int)(i - (int64_t)r * V);
-        double y;
-        if (steps == 1) {
-            y = gj_entry(X, V, c, ip, r, k);
-        } else if (r == c1) {
-            y = k == c1 ? ip1 : gj_entry(X, V, c, ip, c1, k) * ip1;
-        } else if (k == c1) {
-            y = -gj_entry(X, V, c, ip, r, c1) * ip1;
-        } else {
-            y = gj_entry(X, V, c, ip, r, k) - gj_entry(X, V, c, ip, r, c1) * gj_entry(X, V, c, ip, c1, k) * ip1;
+    __shared__ double D[2][GJ][GJ + 1], R[GJ][GJ + 1], L[GJ][GJ + 1];
+    const int nb = min(GJ, V - c);
+    const int r0 = blockIdx.y * GJ, k0 = blockIdx.x * GJ;
+    const int ty = threadIdx.x >> 5, tx = threadIdx.x & 31;   // rows ty, ty + 8, ..., column tx
+    constexpr int NR = GJ / 8;
+    // the pivot block (1 on the diagonal past its end), the tile's pivot rows
+    // and pivot columns (0 past the matrix)
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+        const int i = ty + 8 * n;
+        D[0][i][tx] = i < nb && tx < nb ? X[(int64_t)(c + i) * V + c + tx] : (i == tx ? 1.0 : 0.0);
+        R[i][tx] = i < nb && k0 + tx < V ? X[(int64_t)(c + i) * V + k0 + tx] : 0.0;
+        L[i][tx] = r0 + i < V && tx < nb ? X[(int64_t)(r0 + i) * V + c + tx] : 0.0;
+    }
+    __syncthreads();
+    const bool keeper = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
+    int h = 0;
+    for (int p = 0; p < nb; p += 2, h ^= 1) {
+        const double(*A)[GJ + 1] = D[h];
+        double(*B)[GJ + 1] = D[h ^ 1];
+        const double a = A[p][p], b = A[p][p + 1], g = A[p + 1][p], d = A[p + 1][p + 1];
+        const double det = fma(a, d, -b * g), id = 1.0 / det;
+        if (keeper) {
+            piv[c + p] = a;
+            if (p + 1 < nb) piv[c + p + 1] = det / a;
         }
-        if (i == 0) {
-            piv[c] = pc;
-            if (steps == 2) piv[c1] = pc1;
+        // rows p and p + 1 of the next matrix
+        const bool col = (tx >> 1) == (p >> 1), odd = tx & 1;
+        const double u = A[p][tx], v = A[p + 1][tx];
+        const double rp = col ? (odd ? -b : d) * id : fma(d, u, -b * v) * id;
+        const double rq = col ? (odd ? a : -g) * id : fma(a, v, -g * u) * id;
+#pragma unroll
+        for (int n = 0; n < NR; ++n) {
+            const int i = ty + 8 * n;
+            const double y = fma(-A[i][p], rp, fma(-A[i][p + 1], rq, col ? 0.0 : A[i][tx]));
+            B[i][tx] = i == p ? rp : i == p + 1 ? rq : y;
         }
-        Y[i] = y;
+        __syncthreads();
+    }
+    const double(*P)[GJ + 1] = D[h];
+    // T = P X[C, k] for the tile's columns (in the free half of D), then the tile
+    double(*T)[GJ + 1] = D[h ^ 1];
+    const bool pcol = k0 == c, prow = r0 == c;   // tiles and pivot blocks share their edges
+    double t[NR] = {};
+#pragma unroll 8
+    for (int m = 0; m < GJ; ++m) {
+        const double x = R[m][tx];
+#pragma unroll
+        for (int n = 0; n < NR; ++n) t[n] = fma(P[ty + 8 * n][m], x, t[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < NR; ++n) T[ty + 8 * n][tx] = pcol ? P[ty + 8 * n][tx] : t[n];
+    __syncthreads();
+    double y[NR];
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+        const int r = r0 + ty + 8 * n, k = k0 + tx;
+        y[n] = prow ? T[ty + 8 * n][tx] : (!pcol && r < V && k < V) ? X[(int64_t)r * V + k] : 0.0;
+    }
+    if (!prow)
+#pragma unroll 8
+        for (int m = 0; m < GJ; ++m) {
+            const double x = T[m][tx];
+#pragma unroll
+            for (int n = 0; n < NR; ++n) y[n] = fma(-L[ty + 8 * n][m], x, y[n]);
+        }
+#pragma unroll
+    for (int n = 0; n < NR; ++n) {
+        const int r = r0 + ty + 8 * n, k = k0 + tx;
+        if (r < V && k < V) Y[(int64_t)r * V + k] = y[n];
     }
 }
 
@@ -699,7 +727,8 @@ void Multigrid::init(Operator *fine)
         L->x0.alloc(L->V * es);
     }
     d64.alloc(vx[0]->V * 8);
-    As64.alloc(vx[0]->V * 27 * 8);
+    As64.alloc(vx[0]->V * 27 * 8);   // (also the lattice coarsened in x: no larger, coarse1(n) <= n for n >= 2)
+    if (vx.size() > 1) gT.alloc((size_t)vx[1]->nv[0] * vx[1]->nv[1] * vx[0]->nv[2] * 27 * 8);
     const int64_t VC = vx.back()->V;
     gjX.alloc((size_t)VC * VC * 8);
     gjY.alloc((size_t)VC * VC * 8);
@@ -771,8 +800,14 @@ void Multigrid::update()
     for (size_t l = 1; l < vx.size(); ++l) {
         const MGVertexLevel &F = *vx[l - 1], &C = *vx[l];
         VDims df{ { F.nv[0], F.nv[1], F.nv[2] } }, dc{ { C.nv[0], C.nv[1], C.nv[2] } };
-        hipLaunchKernelGGL(k_mg_galerkin, dim3(mg_grid(C.V * 27)), dim3(MGT), 0, s, df, dc, A64[l - 1]->as<double>(),
-                           A64[l]->as<double>());
+        const VDims d1{ { dc.n[0], df.n[1], df.n[2] } }, d2{ { dc.n[0], dc.n[1], df.n[2] } };
+        auto pass = [&](auto kernel, const VDims &f, const VDims &c, const DevBuf &in, DevBuf &out) {
+            hipLaunchKernelGGL(kernel, dim3(mg_grid((int64_t)c.n[0] * c.n[1] * c.n[2] * 27)), dim3(MGT), 0, s, f, c,
+                               in.as<double>(), out.as<double>());
+        };
+        pass(k_mg_galerkin<0>, df, d1, *A64[l - 1], As64);
+        pass(k_mg_galerkin<1>, d1, d2, As64, gT);
+        pass(k_mg_galerkin<2>, d2, dc, gT, *A64[l]);
         FEM_HIP(hipGetLastError());
     }
     // level data in the preconditioner's precision; a reaction-free level
@@ -790,7 +825,7 @@ void Multigrid::update()
         store_as(lp, L.dinv, d64, L.V, ctx);
     }
     // dense inverse of the coarsest level, stored row-major: Gauss-Jordan on
-    // the device (two pivots per launch, no pivoting) for the symmetric
+    // the device (in blocks, no pivoting) for the symmetric
     // positive definite operators of diffusion and non-negative reaction; a
     // non-positive pivot (an indefinite operator) sends the inversion to the
     // host, with partial pivoting
@@ -802,11 +837,12 @@ void Multigrid::update()
         const unsigned G = mg_grid((int64_t)VC * VC);
         hipLaunchKernelGGL(k_mg_dense_fill, dim3(G), dim3(MGT), 0, s, dc, A64.back()->as<double>(), gjX.as<double>());
         int launches = 0;
-        for (int c = 0; c < VC; c += 2, ++launches) {
+        const unsigned T = (unsigned)((VC + GJ - 1) / GJ);
+        for (int c = 0; c < VC; c += GJ, ++launches) {
             const DevBuf &src = (launches & 1) ? gjY : gjX;
             DevBuf &dst = (launches & 1) ? gjX : gjY;
-            hipLaunchKernelGGL(k_mg_gj_step, dim3(G), dim3(MGT), 0, s, VC, c, std::min(2, VC - c), src.as<double>(),
-                               dst.as<double>(), gjp.as<double>());
+            hipLaunchKernelGGL(k_mg_gj_step, dim3(T, T), dim3(256), 0, s, VC, c, src.as<double>(), dst.as<double>(),
+                               gjp.as<double>());
         }
         FEM_HIP(hipGetLastError());
         std::vector<double> piv(VC);

@@ -44,7 +44,7 @@ struct Multigrid {
     // element means of cvol, and scratch for the level data and the
     // coarsest inverse
     std::vector<std::unique_ptr<DevBuf>> A64;
-    DevBuf cmean, cmean32, d64, As64, gjX, gjY, gjp;
+    DevBuf cmean, cmean32, d64, As64, gT, gjX, gjY, gjp;
 
     // builds the hierarchy (levels, operators, buffers), then update()
     void init(Operator *fine);
