@@ -8,6 +8,7 @@ namespace femamd {
 struct CSR {
     Context *ctx = nullptr;
     Operator *op = nullptr;
+    int dg_k = 0, dg_n[3] = {};   // a DG operator's K (else 0) and mesh
     int64_t N = 0, nnz = 0;
     DevBuf rowptr;   // int64 [N + 1]
     DevBuf col;      // int32 [nnz], increasing within a row
