@@ -67,9 +67,15 @@ struct DGShape {
     static constexpr int TS = K * S1;           // one padded K^3 tensor
     // per element: A (u at quadrature points), R (residual at quadrature
     // points), S (neighbour-trace scratch, 4 K^2); the element stride is
-    // padded to an odd multiple of 16 doubles to separate the elements' banks
+    // padded to an odd multiple of 16 doubles to separate the elements' banks.
+    // At K = 2 a 16-lane access group holds four elements, which such a stride
+    // puts on two banks' offsets: unpadded, 36, the modelled conflicts go down
+    // nine times (64^3 pointwise kappa: FP64 45.2 us with 48, 28.2 us with 36,
+    // FP32 26.8 and 18.0, BF16 27.4 and 21.9; 73 % of the LDS cycles were
+    // conflicts)
     static constexpr int SZ0 = 2 * TS + 4 * K2;
-    static constexpr int SZ = ((SZ0 + 15) / 16) * 16 + (((SZ0 + 15) / 16) % 2 == 0 ? 16 : 0);
+    static constexpr int SZ =
+        K == 2 ? SZ0 : ((SZ0 + 15) / 16) * 16 + (((SZ0 + 15) / 16) % 2 == 0 ? 16 : 0);
 };
 
 // Workgroup of the apply: one wavefront of EPB = 64 / K^2 elements, except
@@ -323,9 +329,11 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
     constexpr int SXI = (D35 && K == 3) ? 4 : K;   // face-trace scratch: row stride
     constexpr int SXQ = K * SXI;                   // and quantity stride
     // with pointwise kappa a third tensor KA holds the element's volume kappa
-    // values: loaded once as x-pencils, the y- and z-pencils come from LDS
-    // (K = 4 only: the other orders keep the face-trace scratch there)
-    constexpr bool KLDS = (K == 4) && KQ;
+    // values: loaded once as x-pencils, the y- and z-pencils come from LDS.
+    // K = 4, and FP32 and BF16 at K = 5, where a pencil load touches every line
+    // of the element (32^3: FP32 40.3 us without, 37.5 us with, BF16 42.8 and
+    // 37.9; FP64 63.5 and 63.9); at K = 2 and 3 an element is one to three lines
+    constexpr bool KLDS = (K == 4 || (K == 5 && !std::is_same<T, double>::value)) && KQ;
     // the pointwise/nonlinear reaction is compiled into a variant (RX) of the
     // pointwise-kappa apply: the kernel without it keeps its code and registers
     // (with kappa constant per element the modal kernels have it)
@@ -335,7 +343,8 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
     static_assert(F64MF_ || SZ >= 2 * K * S1 + 4 * SXQ, "tensors and face-trace scratch per element");
     // DGShape layout at K = 4: the third tensor ends at 2 TS + lidx(3,3,3) + 1
     static_assert(F64MF_ || !KLDS || SZ >= 2 * K * S1 + 3 * S1 + 3 * K + 4, "tensors per element");
-    __shared__ T smem[EPB * SZ];
+    constexpr int SZK = SZ + (KLDS && K == 5 ? K3 + 1 : 0);   // (the stride stays odd)
+    __shared__ T smem[EPB * SZK];
     const Tab1D<T> &tb = *a.tab;
     using C = Ctr<K, T, MF>;
     MFRows mr;
@@ -405,10 +414,10 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
     constexpr bool XSH = (K == 4) && std::is_same<T, double>::value && !MF;
     const int xs = (el0 == 0) ? 0 : 1;   // the x side whose neighbour this lane loads
 
-    T *A = smem + el * SZ;
+    T *A = smem + el * SZK;
     T *R = A + K * S1;
-    T *KA = R + K * S1;   // pointwise kappa at the volume points (KLDS only;
-                          // at K = 4 the face-trace scratch Sx is not used)
+    T *KA = R + K * S1 + (K == 4 ? 0 : 4 * SXQ);   // pointwise kappa at the volume points (KLDS only), after
+                                                   // the face-trace scratch Sx, which K = 4 does not use
     auto L = [&](int a_, int b_, int c_) {
         if constexpr (F64MF_ || D35) return a_ * S1 + b_ * SB + c_;
         else return lidx<K>(a_, b_, c_);
@@ -490,8 +499,9 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
 #pragma unroll
         for (int q = 0; q < K; ++q) A[L(i, j, q)] = tmp[q];
     if constexpr (KLDS)
+        if (wr)
 #pragma unroll
-        for (int q = 0; q < K; ++q) KA[L(q, i, j)] = kx[q];
+            for (int q = 0; q < K; ++q) KA[L(q, i, j)] = kx[q];
     lds_sync<WG>();
     // Y layout: thread (i=a, j=qz); each thread rewrites the pencil it read
 #pragma unroll
