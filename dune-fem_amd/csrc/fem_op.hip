@@ -726,46 +726,11 @@ __global__ void k_round32(const double *__restrict__ x, float *__restrict__ y, i
         y[i] = (float)x[i];
 }
 
-// dot (may be null): the workgroup's <p, y> and <p, p>, p the preconditioner's
-// argument (workgroups of RED_THREADS)
-__global__ void __launch_bounds__(RED_THREADS)
-    k_widen64(const float *__restrict__ x, double *__restrict__ y, int64_t n, const int *__restrict__ skip,
-              const double *__restrict__ p, double *__restrict__ dot)
+__global__ void k_widen64(const float *__restrict__ x, double *__restrict__ y, int64_t n, const int *__restrict__ skip)
 {
     if (skip && *skip) return;
-    double a1 = 0, a2 = 0;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    for (; i + 3 * stride < n; i += 4 * stride) {
-        float v[4];
-        double pv[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            v[k] = x[i + k * stride];
-            pv[k] = dot ? p[i + k * stride] : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            y[i + k * stride] = (double)v[k];
-            a1 += pv[k] * (double)v[k];
-            a2 += pv[k] * pv[k];
-        }
-    }
-    for (; i < n; i += stride) {
-        const double v = (double)x[i], pv = dot ? p[i] : 0.0;
-        y[i] = v;
-        a1 += pv * v;
-        a2 += pv * pv;
-    }
-    if (!dot) return;
-    __shared__ double lds[RED_THREADS / 64];
-    const double s1 = block_sum(a1, lds);
-    __syncthreads();
-    const double s2 = block_sum(a2, lds);
-    if (threadIdx.x == 0) {
-        dot[blockIdx.x] = s1;
-        dot[gridDim.x + blockIdx.x] = s2;
-    }
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        y[i] = (double)x[i];
 }
 
 void Precond::init_widening(Operator *o64, const Precond *p32)
@@ -788,25 +753,18 @@ Precond::~Precond()
     delete mg;
 }
 
-// workgroups of k_widen64, about four elements per thread
-static int64_t widen_blocks(int64_t n) { return grid_for(n, 4 * RED_THREADS, 2048); }
-
-int64_t Precond::dot_parts() const
-{
-    return lowp ? widen_blocks(op->N) : dg_bj_blocks(op->k, op->E);
-}
+int64_t Precond::dot_parts() const { return dg_bj_blocks(op->k, op->E); }
 
 void Precond::apply_raw(const void *x, void *y, const int *skip, double *dot) const
 {
     hipStream_t s = op->ctx->stream;
     const int64_t N = op->N;
-    FEM_CHECK(!dot || fused_dot(), FEM_ERR_UNSUPPORTED, "fused dot: block Jacobi, or an FP32 preconditioner of an FP64 solve");
+    FEM_CHECK(!dot || fused_dot(), FEM_ERR_UNSUPPORTED, "fused dot: block Jacobi");
     if (lowp) {
         const unsigned G = grid_for(N, 256, 8192);
         hipLaunchKernelGGL(k_round32, dim3(G), dim3(256), 0, s, (const double *)x, cx.as<float>(), N, skip);
         lowp->apply_raw(cx.p, cy.p, skip);
-        hipLaunchKernelGGL(k_widen64, dim3((unsigned)widen_blocks(N)), dim3(RED_THREADS), 0, s, (const float *)cy.as<float>(),
-                           (double *)y, N, skip, (const double *)x, dot);
+        hipLaunchKernelGGL(k_widen64, dim3(G), dim3(256), 0, s, (const float *)cy.as<float>(), (double *)y, N, skip);
         FEM_HIP(hipGetLastError());
     } else if (kind == FEM_PRE_LEARNED) {
         learned->apply_raw(x, y, skip);

@@ -153,7 +153,7 @@ struct Precond {
     // <x, y> and then of <x, x>, dot_parts() entries each
     void apply_raw(const void *x, void *y, const int *skip, double *dot = nullptr) const;
     bool pointwise() const { return kind == FEM_PRE_JACOBI; }
-    bool fused_dot() const { return kind == FEM_PRE_BLOCK_JACOBI || lowp != nullptr; }
+    bool fused_dot() const { return kind == FEM_PRE_BLOCK_JACOBI; }
     int64_t dot_parts() const;
     ~Precond();
 };

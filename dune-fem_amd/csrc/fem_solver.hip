@@ -155,11 +155,12 @@ __global__ void __launch_bounds__(RED_THREADS) k_cg_check(KState *st, const doub
     cg_end_of_step(st, pp, np, lds, true, beta);
 }
 
-// q = beta q + s, without a preconditioner p = beta p - r
-template <typename T>
+// q = beta q + sg a: a = s, sg = 1 (TA = float: the result of an FP32
+// preconditioner as it is), without a preconditioner a = r, sg = -1
+template <typename T, typename TA>
 __global__ void __launch_bounds__(RED_THREADS)
-    k_cg_dir(T *__restrict__ q, const T *__restrict__ s, const T *__restrict__ r, int64_t n, KState *st,
-             const double *__restrict__ pp, int np, int haspre)
+    k_cg_dir(T *__restrict__ q, const TA *__restrict__ a, double sg, int64_t n, KState *st,
+             const double *__restrict__ pp, int np)
 {
     if (st->done || st->fresh) return;
     __shared__ double lds[2 * (RED_THREADS / 64)];
@@ -167,11 +168,10 @@ __global__ void __launch_bounds__(RED_THREADS)
     if (cg_end_of_step(st, pp, np, lds, blockIdx.x == 0, beta)) return;
     const int64_t stride = (int64_t)gridDim.x * RED_THREADS;
     int64_t i = blockIdx.x * (int64_t)RED_THREADS + threadIdx.x;
-    const T *a = haspre ? s : r;
-    const double sg = haspre ? 1.0 : -1.0;
     // four independent elements in flight per thread
     for (; i + 3 * stride < n; i += 4 * stride) {
-        T vq[4], va[4];
+        T vq[4];
+        TA va[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             vq[k] = q[i + k * stride];
@@ -183,7 +183,8 @@ __global__ void __launch_bounds__(RED_THREADS)
     for (; i < n; i += stride) q[i] = (T)(beta * (double)q[i] + sg * (double)a[i]);
 }
 
-// MODE 0: x += a q, p -= a h (a general preconditioner follows)
+// MODE 0: x += a q, p -= a h (a general preconditioner follows; p32, may be
+//         null: p rounded for an FP32 preconditioner)
 // MODE 1: the same, s = dinv p and the partials of <p, s>, <p, p> (Jacobi)
 // MODE 2: x += a q, r += a h and the partials of <r, r>, twice (no
 //         preconditioner; p is r here)
@@ -191,7 +192,7 @@ template <typename T, int MODE>
 __global__ void __launch_bounds__(RED_THREADS)
     k_cg_update(T *__restrict__ x, T *__restrict__ p, const T *__restrict__ q, const T *__restrict__ h,
                 T *__restrict__ s, const T *__restrict__ dinv, int64_t n, KState *st, const double *__restrict__ qp,
-                int nq, double *__restrict__ pp)
+                int nq, double *__restrict__ pp, float *__restrict__ p32)
 {
     if (st->done) return;
     __shared__ double lds[RED_THREADS / 64];
@@ -210,6 +211,7 @@ __global__ void __launch_bounds__(RED_THREADS)
         x[i] = (T)((double)xv + alpha * (double)qv);
         const T pn = (T)((double)pv + (MODE == 2 ? alpha : -alpha) * (double)hv);
         p[i] = pn;
+        if (MODE == 0 && p32) p32[i] = (float)pn;
         if (MODE == 1) {
             const T sv = dv * pn;
             s[i] = sv;
@@ -246,9 +248,9 @@ __global__ void __launch_bounds__(RED_THREADS)
 }
 
 // partials of <a, b> and (NQ = 2) of <a, a>
-template <typename T, int NQ>
+template <typename T, int NQ, typename TB = T>
 __global__ void __launch_bounds__(RED_THREADS)
-    k_cg_dots(const T *__restrict__ a, const T *__restrict__ b, int64_t n, const KState *__restrict__ st,
+    k_cg_dots(const T *__restrict__ a, const TB *__restrict__ b, int64_t n, const KState *__restrict__ st,
               double *__restrict__ out)
 {
     if (st->done) return;
@@ -257,7 +259,8 @@ __global__ void __launch_bounds__(RED_THREADS)
     const int64_t stride = (int64_t)gridDim.x * RED_THREADS;
     int64_t i = blockIdx.x * (int64_t)RED_THREADS + threadIdx.x;
     for (; i + 3 * stride < n; i += 4 * stride) {
-        T va[4], vb[4];
+        T va[4];
+        TB vb[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             va[k] = a[i + k * stride];
@@ -784,8 +787,6 @@ void Solver::fetch_state()
     FEM_HIP(hipStreamSynchronize(ctx->stream));
 }
 
-static bool pfused_bj(const Precond *p) { return p->kind == FEM_PRE_BLOCK_JACOBI; }
-
 template <typename T>
 static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b, T *x, double eps, int criteria,
                       int maxit, int m, int64_t N, int verbose)
@@ -800,12 +801,19 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
     FEM_HIP(hipMemsetAsync(st, 0, sizeof(KState), s));
     if (method == FEM_SOLVER_CG) {
         T *h = (T *)S.workbuf(0, vb), *r = (T *)S.workbuf(1, vb), *pp = (T *)S.workbuf(2, vb);
-        T *ss = haspre ? (T *)S.workbuf(3, vb) : pp, *q = haspre ? (T *)S.workbuf(4, vb) : pp;
+        // an FP32 preconditioner of an FP64 solve: p rounded (p32) and its
+        // result (s32) pass between it and the CG kernels as they are, in the
+        // place of s: 20 bytes per DoF and step, 40 with passes that round and
+        // widen
+        const Precond *low = haspre && !S.snapshot ? p->lowp : nullptr;
+        const size_t half = (sizeof(float) * N + 255) / 256 * 256;
+        T *ss = haspre ? (T *)S.workbuf(3, std::max(vb, low ? 2 * half : 0)) : pp,
+          *q = haspre ? (T *)S.workbuf(4, vb) : pp;
+        float *s32 = low ? (float *)ss : nullptr, *p32 = low ? (float *)((char *)ss + half) : nullptr;
         o->apply_raw(x, h, nullptr);
         hipLaunchKernelGGL(k_cg_setup<T>, dim3(G), dim3(256), 0, s, b, h, r, pp, N);
         if (haspre) {
-            p->apply_raw(pp, q, nullptr);
-            FEM_HIP(hipMemcpyAsync(ss, q, vb, hipMemcpyDeviceToDevice, s));
+            p->apply_raw(pp, q, nullptr);   // (the first step reads q alone)
         }
         dot_async(*S.ctx, N, pp, q, &st->res, cnt + 1, part);
         dot_async(*S.ctx, N, pp, pp, &st->rr, cnt + 1, part);
@@ -829,7 +837,7 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
         // steps between two looks of the host: a look costs about 20 us, a
         // step past the end one idle launch per kernel, of which a multigrid
         // step has some forty
-        const int most = haspre && !dinv && !pfused_bj(p) ? 4 : 32;
+        const int most = haspre && !dinv && !pfused ? 4 : 32;
         int chunk = S.snapshot ? S.snap_chunk : 4;
         // one CG step as a HIP graph: every kernel of the step reads the
         // device done flag, so replays after convergence do nothing; the step
@@ -846,7 +854,11 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
             }
         } gguard{ graph, gexec };
         auto cg_step = [&]() {
-            hipLaunchKernelGGL(k_cg_dir<T>, dim3(GU), dim3(RED_THREADS), 0, s, q, ss, r, N, st, pparts, np, haspre ? 1 : 0);
+            if (low)
+                hipLaunchKernelGGL((k_cg_dir<T, float>), dim3(GU), dim3(RED_THREADS), 0, s, q, s32, 1.0, N, st, pparts, np);
+            else
+                hipLaunchKernelGGL((k_cg_dir<T, T>), dim3(GU), dim3(RED_THREADS), 0, s, q, haspre ? ss : r,
+                                   haspre ? 1.0 : -1.0, N, st, pparts, np);
             o->apply_raw(q, h, &st->done, qfused ? dq : nullptr);
             if (!qfused)
                 hipLaunchKernelGGL((k_cg_dots<T, 1>), dim3(GU), dim3(RED_THREADS), 0, s, q, h, N, st, dq);
@@ -854,15 +866,18 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
                 hipLaunchKernelGGL(k_cg_fewer, dim3(CG_FEWER), dim3(RED_THREADS), 0, s, dq, nq0, 1, qparts, st);
             if (!haspre) {
                 hipLaunchKernelGGL((k_cg_update<T, 2>), dim3(GU), dim3(RED_THREADS), 0, s, x, r, q, h, (T *)nullptr, dinv,
-                                   N, st, qparts, nq, dp);
+                                   N, st, qparts, nq, dp, (float *)nullptr);
             } else if (dinv) {
                 hipLaunchKernelGGL((k_cg_update<T, 1>), dim3(GU), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, dinv, N, st,
-                                   qparts, nq, dp);
+                                   qparts, nq, dp, (float *)nullptr);
             } else {
-                hipLaunchKernelGGL((k_cg_update<T, 0>), dim3(GU), dim3(RED_THREADS), 0, s, x, pp, q, h, ss, dinv, N, st,
-                                   qparts, nq, dp);
-                p->apply_raw(pp, ss, &st->done, pfused ? dp : nullptr);
-                if (!pfused)
+                hipLaunchKernelGGL((k_cg_update<T, 0>), dim3(GU), dim3(RED_THREADS), 0, s, x, pp, q, h, (T *)nullptr, dinv, N,
+                                   st, qparts, nq, dp, p32);
+                if (low) low->apply_raw(p32, s32, &st->done);
+                else p->apply_raw(pp, ss, &st->done, pfused ? dp : nullptr);
+                if (low)
+                    hipLaunchKernelGGL((k_cg_dots<T, 2, float>), dim3(GU), dim3(RED_THREADS), 0, s, pp, s32, N, st, dp);
+                else if (!pfused)
                     hipLaunchKernelGGL((k_cg_dots<T, 2>), dim3(GU), dim3(RED_THREADS), 0, s, pp, ss, N, st, dp);
             }
             if (np0 > CG_PARTS)
