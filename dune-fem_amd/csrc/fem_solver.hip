@@ -80,7 +80,7 @@ __global__ void k_cg_init(KState *st, double eps, int criteria, int maxit, int c
     st->it = 0;
     st->maxit = maxit;
     st->crit_res = crit_res;
-    st->done = !(r0 > st->tol) || maxit <= 0;
+    st->done = st->end = !(r0 > st->tol) || maxit <= 0;
     st->fresh = 1;
     st->n_res = st->res;
     st->n_rr = st->rr;
@@ -90,9 +90,9 @@ __global__ void k_cg_init(KState *st, double eps, int criteria, int maxit, int c
 // A CG step is: direction (k_cg_dir), apply with the partials of <q, h>,
 // update (k_cg_update), preconditioner with the partials of <p, s> and
 // <p, p>.  The direction kernel sums the latter, forms beta and the stopping
-// test, and leaves the new scalars in n_*; the update kernel sums <q, h>,
-// forms alpha and makes n_* current.  No workgroup of either reads what its
-// first workgroup writes there.
+// test, and its first workgroup keeps the new scalars; the update kernel sums
+// <q, h>, forms alpha and makes them current.  No kernel reads what one of its
+// own workgroups writes (fem_kstate.hpp has the flags).
 
 // two sums at once, of part[0..n) and part[n..2n)
 __device__ __forceinline__ void sum_parts2(const double *__restrict__ part, int n, double *lds, double &s0, double &s1)
@@ -121,38 +121,18 @@ __device__ __forceinline__ void sum_parts2(const double *__restrict__ part, int 
     }
 }
 
-// <p, s> and <p, p> from pp[2][np], and what follows: whether the solve is done
-__device__ __forceinline__ bool cg_end_of_step(KState *st, const double *__restrict__ pp, int np, double *lds,
-                                               bool keeper, double &beta)
-{
-    double r, rr;
-    sum_parts2(pp, np, lds, r, rr);
-    const int it = st->it + 1;
-    beta = r / st->res;
-    const bool done = !((st->crit_res ? rr : r) > st->tol) || it >= st->maxit;
-    __syncthreads();   // every thread has read the scalars
-    if (keeper && threadIdx.x == 0) {
-        st->n_res = r;
-        st->n_rr = rr;
-        st->n_it = it;
-        if (done) {
-            st->res = r;
-            st->rr = rr;
-            st->it = it;
-            st->done = 1;
-        }
-    }
-    return done;
-}
-
-// the same test after the last step of a batch, for the host to read (the
-// next direction kernel repeats it if the solve goes on)
+// the same test after the last step of a batch, for the host to read, by one
+// workgroup (the next direction kernel repeats it if the solve goes on)
 __global__ void __launch_bounds__(RED_THREADS) k_cg_check(KState *st, const double *__restrict__ pp, int np)
 {
-    if (st->done || st->fresh) return;
+    if (cg_skip_dir(*st)) return;
     __shared__ double lds[2 * (RED_THREADS / 64)];
-    double beta;
-    cg_end_of_step(st, pp, np, lds, true, beta);
+    double r, rr;
+    sum_parts2(pp, np, lds, r, rr);   // (its barrier: every wavefront has entered)
+    if (threadIdx.x == 0) {
+        cg_keep(*st, r, rr);
+        if (st->end) cg_pass_on(*st);
+    }
 }
 
 // q = beta q + sg a: a = s, sg = 1 (TA = float: the result of an FP32
@@ -162,10 +142,13 @@ __global__ void __launch_bounds__(RED_THREADS)
     k_cg_dir(T *__restrict__ q, const TA *__restrict__ a, double sg, int64_t n, KState *st,
              const double *__restrict__ pp, int np)
 {
-    if (st->done || st->fresh) return;
+    if (cg_skip_dir(*st)) return;
     __shared__ double lds[2 * (RED_THREADS / 64)];
-    double beta;
-    if (cg_end_of_step(st, pp, np, lds, blockIdx.x == 0, beta)) return;
+    double r, rr;
+    sum_parts2(pp, np, lds, r, rr);
+    if (blockIdx.x == 0 && threadIdx.x == 0) cg_keep(*st, r, rr);
+    if (cg_stops(*st, r, rr)) return;
+    const double beta = r / st->res;
     const int64_t stride = (int64_t)gridDim.x * RED_THREADS;
     int64_t i = blockIdx.x * (int64_t)RED_THREADS + threadIdx.x;
     // four independent elements in flight per thread
@@ -194,17 +177,18 @@ __global__ void __launch_bounds__(RED_THREADS)
                 T *__restrict__ s, const T *__restrict__ dinv, int64_t n, KState *st, const double *__restrict__ qp,
                 int nq, double *__restrict__ pp, float *__restrict__ p32)
 {
-    if (st->done) return;
+    const bool keeper = blockIdx.x == 0 && threadIdx.x == 0;
+    if (cg_skip_step(*st)) {
+        if (keeper) cg_pass_on(*st);
+        return;
+    }
     __shared__ double lds[RED_THREADS / 64];
     const double qh = sum_parts(qp, nq, lds);
     const double alpha = st->n_res / qh;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (keeper) {
         st->qh = qh;
         st->alpha = alpha;
-        st->res = st->n_res;
-        st->rr = st->n_rr;
-        st->it = st->n_it;
-        st->fresh = 0;
+        cg_pass_on(*st);
     }
     double acc = 0, acc2 = 0;
     auto one = [&](int64_t i, T xv, T pv, T qv, T hv, T dv) {
@@ -253,7 +237,7 @@ __global__ void __launch_bounds__(RED_THREADS)
     k_cg_dots(const T *__restrict__ a, const TB *__restrict__ b, int64_t n, const KState *__restrict__ st,
               double *__restrict__ out)
 {
-    if (st->done) return;
+    if (cg_skip_step(*st)) return;
     __shared__ double lds[RED_THREADS / 64];
     double acc = 0, acc2 = 0;
     const int64_t stride = (int64_t)gridDim.x * RED_THREADS;
@@ -290,7 +274,7 @@ __global__ void __launch_bounds__(RED_THREADS)
 __global__ void __launch_bounds__(RED_THREADS)
     k_cg_fewer(const double *__restrict__ in, int64_t n, int nq, double *__restrict__ out, const KState *__restrict__ st)
 {
-    if (st->done) return;
+    if (cg_skip_step(*st)) return;
     __shared__ double lds[RED_THREADS / 64];
     const int64_t lo = n * blockIdx.x / gridDim.x, hi = n * (blockIdx.x + 1) / gridDim.x;
     for (int k = 0; k < nq; ++k) {
@@ -839,8 +823,8 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
         // step has some forty
         const int most = haspre && !dinv && !pfused ? 4 : 32;
         int chunk = S.snapshot ? S.snap_chunk : 4;
-        // one CG step as a HIP graph: every kernel of the step reads the
-        // device done flag, so replays after convergence do nothing; the step
+        // one CG step as a HIP graph: every kernel of the step reads a device
+        // flag of the end, so replays after convergence do nothing; the step
         // holds no memset node.  Captured per solve (the vectors differ).
         hipGraph_t graph = nullptr;
         hipGraphExec_t gexec = nullptr;
@@ -859,7 +843,7 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
             else
                 hipLaunchKernelGGL((k_cg_dir<T, T>), dim3(GU), dim3(RED_THREADS), 0, s, q, haspre ? ss : r,
                                    haspre ? 1.0 : -1.0, N, st, pparts, np);
-            o->apply_raw(q, h, &st->done, qfused ? dq : nullptr);
+            o->apply_raw(q, h, &st->end, qfused ? dq : nullptr);
             if (!qfused)
                 hipLaunchKernelGGL((k_cg_dots<T, 1>), dim3(GU), dim3(RED_THREADS), 0, s, q, h, N, st, dq);
             if (nq0 > CG_PARTS)
@@ -873,8 +857,8 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
             } else {
                 hipLaunchKernelGGL((k_cg_update<T, 0>), dim3(GU), dim3(RED_THREADS), 0, s, x, pp, q, h, (T *)nullptr, dinv, N,
                                    st, qparts, nq, dp, p32);
-                if (low) low->apply_raw(p32, s32, &st->done);
-                else p->apply_raw(pp, ss, &st->done, pfused ? dp : nullptr);
+                if (low) low->apply_raw(p32, s32, &st->end);
+                else p->apply_raw(pp, ss, &st->end, pfused ? dp : nullptr);
                 if (low)
                     hipLaunchKernelGGL((k_cg_dots<T, 2, float>), dim3(GU), dim3(RED_THREADS), 0, s, pp, s32, N, st, dp);
                 else if (!pfused)
