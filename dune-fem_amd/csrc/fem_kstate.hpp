@@ -36,7 +36,8 @@ struct KState {
     double gres;     // the cycle's last residual estimate |g[jlast]|
     int jlast;       // inner steps done in the current cycle
     int converged;   // cycle ended by |g| < tol
-    int cycle_done;  // stop inner loop (converged or maxit)
+    int cycle_end;   // the step just scaled was the cycle's last (converged or maxit)
+    int cycle_done;  // the same, a kernel later
     // BiCGStab
     double nu, omega, bres;
     int fin;         // the iteration just reduced is the last one
@@ -80,5 +81,39 @@ FEM_HD void cg_pass_on(KState &st)
     st.fresh = 0;
     if (st.end) st.done = 1;
 }
+
+// ---- GMRES ----------------------------------------------------------------------
+// A step is: preconditioner, apply, multi-dot, orthogonalisation, scaling.  The
+// scaling kernel finishes column j and finds out whether the cycle ends; the
+// kernels after it enter by `cycle_end`; the orthogonalisation passes it on as
+// `cycle_done`, by which the scaling enters.  At the start of a cycle (j < 0) the
+// scaling always runs.
+FEM_HD bool gm_skip_scale(const KState &st, int j) { return j >= 0 && st.cycle_done; }
+FEM_HD bool gm_skip_step(const KState &st) { return st.cycle_end; }
+
+// by one thread of the scaling at the start of a cycle, nrm = ||r||
+FEM_HD void gm_begin(KState &st, double nrm)
+{
+    st.res = nrm;
+    st.jlast = 0;
+    st.gres = nrm;
+    st.converged = nrm <= st.gtol * (1 + 1e-15);
+    st.cycle_end = st.cycle_done = st.converged || st.it >= st.maxit;
+    if (!st.converged) st.g[0] = -nrm;
+}
+
+// by one thread of the scaling, gl = g[j + 1] after the rotation of column j
+FEM_HD void gm_keep(KState &st, int j, int m, double gl)
+{
+    const double e = gl < 0 ? -gl : gl;
+    st.gres = e;
+    st.it += 1;
+    st.jlast = j + 1;
+    if (e < st.gtol) st.converged = 1;
+    if (st.converged || st.it >= st.maxit || j + 1 == m) st.cycle_end = 1;
+}
+
+// by one thread of the orthogonalisation, where it skips the step
+FEM_HD void gm_pass_on(KState &st) { st.cycle_done = 1; }
 
 }  // namespace femamd

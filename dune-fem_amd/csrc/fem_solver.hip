@@ -307,7 +307,7 @@ __global__ void __launch_bounds__(RED_THREADS)
     k_gm_multidot(const T *__restrict__ V, const T *__restrict__ w, int64_t n, int j, const KState *__restrict__ st,
                   double *__restrict__ mpart)
 {
-    if (st->cycle_done) return;
+    if (gm_skip_step(*st)) return;
     __shared__ double lds[GRP][RED_THREADS / 64];
     const int g0 = blockIdx.y * GRP, cnt = j + 1 - g0 < GRP ? j + 1 - g0 : GRP;
     const int64_t lo = n * blockIdx.x / gridDim.x, hi = n * (blockIdx.x + 1) / gridDim.x;
@@ -368,7 +368,10 @@ __global__ void __launch_bounds__(RED_THREADS)
     k_gm_orth(const T *__restrict__ V, T *__restrict__ w, int64_t n, int j, KState *__restrict__ st,
               const double *__restrict__ mpart, int slices, double *__restrict__ part, int m)
 {
-    if (st->cycle_done) return;
+    if (gm_skip_step(*st)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) gm_pass_on(*st);
+        return;
+    }
     __shared__ double lds[RED_THREADS / 64];
     __shared__ double h[GM_MAX + 1];
     {
@@ -414,9 +417,7 @@ __global__ void __launch_bounds__(RED_THREADS)
     k_gm_scale(T *__restrict__ v, int64_t n, int j, KState *__restrict__ st, const double *__restrict__ part,
                int nparts, int m, const T *__restrict__ dinv, T *__restrict__ z)
 {
-    // (a workgroup that sees the first one's flag of this very step skips the
-    // scaling of a vector that nothing reads any more)
-    if (j >= 0 && st->cycle_done) return;
+    if (gm_skip_scale(*st, j)) return;
     __shared__ double lds[RED_THREADS / 64];
     __shared__ double col[GM_MAX + 1], cs[GM_MAX], sn[GM_MAX];
     const bool keeper = blockIdx.x == 0;
@@ -440,17 +441,7 @@ __global__ void __launch_bounds__(RED_THREADS)
     if (!keeper || threadIdx.x != 0) return;
     if (j < 0) {
         if (j == -1 && st->criteria == FEM_ERRMEASURE_REDUCTION) st->gtol *= nrm;
-        st->res = nrm;
-        st->jlast = 0;
-        st->gres = nrm;
-        if (nrm <= st->gtol * (1 + 1e-15)) {
-            st->converged = 1;
-            st->cycle_done = 1;
-        } else {
-            st->converged = 0;
-            st->cycle_done = st->it >= st->maxit ? 1 : 0;
-            st->g[0] = -nrm;
-        }
+        gm_begin(*st, nrm);
         return;
     }
     double x = col[0];   // H[i][j] while the rotations pass down the column
@@ -472,15 +463,7 @@ __global__ void __launch_bounds__(RED_THREADS)
     rot(gl, gt, c, s);
     st->g[j] = gt;
     st->g[j + 1] = gl;
-    st->gres = fabs(gl);
-    st->it += 1;
-    st->jlast = j + 1;
-    if (fabs(gl) < st->gtol) {
-        st->converged = 1;
-        st->cycle_done = 1;
-    } else if (st->it >= st->maxit || j + 1 == m) {
-        st->cycle_done = 1;
-    }
+    gm_keep(*st, j, m, gl);
 }
 
 // H y = g, back substitution by one wavefront, lane i holding row i
@@ -990,7 +973,7 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
         first = false;
         for (int j = 0; j < m; ++j) {
             T *vj = V + (int64_t)j * N, *w = V + (int64_t)(j + 1) * N;
-            const int *skip = &st->cycle_done;
+            const int *skip = &st->cycle_end;
             if (haspre) {
                 T *zj = flex ? Z + (int64_t)j * N : z;
                 if (!gdinv) p->apply_raw(vj, zj, skip);

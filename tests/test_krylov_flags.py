@@ -16,6 +16,7 @@ COMMON = r"""
 #include "fem_kstate.hpp"
 #include <cstdio>
 #include <cstdlib>
+#include <initializer_list>
 using namespace femamd;
 #define CHECK(c) do { if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); std::exit(1); } } while (0)
 // a kernel: `entry` decides whether a workgroup returns at once, `keeper` is what
@@ -63,6 +64,38 @@ int main()
 }
 """
 
+GMRES = COMMON + r"""
+int main()
+{
+    // restart m, a limit of steps, residuals 16, 8, 4, ... against tolerance 1 or 0
+    for (int m = 1; m < 6; ++m)
+        for (int maxit = 1; maxit < 12; ++maxit)
+            for (double tol : { 1.5, 0.0 }) {
+                KState st{};
+                st.gtol = tol;
+                st.maxit = maxit;
+                int applies = 0, cycles = 0;
+                while (!st.converged && st.it < maxit && cycles < 20) {
+                    ++cycles;
+                    const int before = applies;
+                    kernel(st, [](const KState &s) { return gm_skip_scale(s, -1); },
+                           [&](KState &s, bool) { gm_begin(s, 16.0 / (1 << applies)); });
+                    for (int j = 0; j < m + 2; ++j) {   // (past the end as well)
+                        if (!gm_skip_step(st)) ++applies;
+                        kernel(st, gm_skip_step, [&](KState &s, bool skip) { if (skip) gm_pass_on(s); });
+                        kernel(st, [j](const KState &s) { return gm_skip_scale(s, j); }, [&](KState &s, bool skip) {
+                            if (!skip) gm_keep(s, j, m, -16.0 / (1 << applies));
+                        });
+                    }
+                    CHECK(st.jlast == applies - before && st.jlast <= m);
+                }
+                CHECK(st.it == applies && applies == (maxit < 4 || tol == 0 ? maxit : 4));   // 16 -> 1 takes four
+                CHECK(st.converged == (tol > 0 && maxit >= 4));
+            }
+    return 0;
+}
+"""
+
 
 def run(tmp_path, src):
     (tmp_path / "t.cc").write_text(src)
@@ -73,6 +106,6 @@ def run(tmp_path, src):
     assert p.returncode == 0, p.stdout
 
 
-@pytest.mark.parametrize("solver", ["cg"])
+@pytest.mark.parametrize("solver", ["cg", "gmres"])
 def test_no_kernel_reads_a_flag_that_it_writes(tmp_path, solver):
-    run(tmp_path, {"cg": CG}[solver])
+    run(tmp_path, {"cg": CG, "gmres": GMRES}[solver])
