@@ -867,14 +867,14 @@ static void dispatch_apply(const DGArgs<T> &a, int k, const T *u, T *w, const in
     }
 }
 
-void dg_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
+void dg_apply_f64(const DGPlan<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                   double *dot)
 {
     if (dg_is_modal(a)) dg_modal_apply_f64(a, k, u, w, skip, s, dot);
     else dispatch_apply<double>(a, k, u, w, skip, s, dot);
 }
 
-void dg_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
+void dg_apply_f32(const DGPlan<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                   double *dot)
 {
     if (dg_is_modal(a)) dg_modal_apply_f32(a, k, u, w, skip, s, dot);

@@ -45,6 +45,11 @@ struct ModalRows {
 };
 ModalRows dg_modal_rows(int k, const int *n);
 
+// kernel arguments of the quadrature kernels.  They are copied at every launch
+// and a small apply is little more than its launch, so what only the line
+// kernels read is in ModalArgs and the plans (12 x 10 x 9 elements with pointwise
+// kappa: Q1 FP32 4.95 us with both in one struct, 720 bytes, 4.55 us without; Q3
+// FP64 5.42 us and 5.15 us)
 template <typename T>
 struct DGArgs {
     int n[3];
@@ -80,11 +85,37 @@ struct DGArgs {
     // ty y-rows through all z; `slabs` = 0 selects plain element order
     int slabs, rpb, ty;
     UDiv dv_slab, dv_zrow, dv_rpb;   // by rpb ty nz, rpb ty, rpb
-    // of the modal kernel: 2 |K| / h^2, 2 |F| b, |F| beta / (2 h), |F| / (2 h),
-    // |F| max(b, 0), |F| max(-b, 0) per direction, c |K| and |K|
-    T m_kv[3], m_ad[3], m_pen[3], m_w[3], m_bp[3], m_bm[3], m_c, m_vol;
-    ModalRows mr;
-    ModalTile mt;   // traversal of the modal kernel (fem_dg_modal.hip)
+};
+static_assert(sizeof(DGArgs<double>) <= 416, "what a launch of a quadrature kernel copies");
+
+// kernel arguments of the line kernels (fem_dg_modal.hip): per direction
+// 2 |K| / h^2, 2 |F| b, |F| beta / (2 h), |F| / (2 h), |F| max(b, 0),
+// |F| max(-b, 0), then c |K| and |K|; the coefficients as in DGArgs
+template <typename T>
+struct ModalArgs {
+    int n[3];
+    int terms;   // bits 0..2: b[d] is not 0, bit 3: c is not 0
+    T kv[3], ad[3], pen[3], w[3], bp[3], bm[3], c, vol;
+    T kappa_const;
+    const T *kcell;   // null: kappa_const
+    const T *ccell;
+};
+// the reaction at the volume points, as in DGArgs
+template <typename T>
+struct ModalReaction {
+    const T *cvol = nullptr;
+    T nl_coef = T(0);
+    int nl_pow = 0;
+    const Tab1D<T> *tab = nullptr;
+};
+
+// a DG operator on the host: the arguments of both kernels and the line kernels'
+// traversals
+template <typename T>
+struct DGPlan : DGArgs<T> {
+    ModalArgs<T> modal;   // (kappa and ccell are filled in at the launch)
+    ModalRows rows;
+    ModalTile tile;
 };
 
 // the damped block-Jacobi sweep fused into the apply (multigrid smoothing):
@@ -113,10 +144,10 @@ struct DGResidual {
 // elements per workgroup of the apply for k points per direction
 int dg_apply_epb(int k);
 
-// fills the per-direction constants and the traversal of DGArgs from n, h,
-// ih, beta, b and the number of 1D points k
+// fills the per-direction constants and the traversals of a plan from n, h,
+// ih, beta, b, c and the number of 1D points k
 template <typename T>
-inline void dg_derived(DGArgs<T> &a, int k)
+inline void dg_derived(DGPlan<T> &a, int k)
 {
     const int epb = dg_apply_epb(k);
     a.slabs = 1;
@@ -128,10 +159,12 @@ inline void dg_derived(DGArgs<T> &a, int k)
         a.dv_zrow = make_udiv((unsigned)(a.rpb * a.ty));
         a.dv_rpb = make_udiv((unsigned)a.rpb);
     }
-    a.mt = dg_modal_tile(k, a.n);
-    a.mr = dg_modal_rows(k, a.n);
-    a.m_vol = a.h[0] * a.h[1] * a.h[2];
-    a.m_c = a.c * a.m_vol;
+    a.tile = dg_modal_tile(k, a.n);
+    a.rows = dg_modal_rows(k, a.n);
+    ModalArgs<T> &m = a.modal;
+    m.vol = a.h[0] * a.h[1] * a.h[2];
+    m.c = a.c * m.vol;
+    m.terms = a.c != T(0) ? 8 : 0;
     for (int d = 0; d < 3; ++d) {
         const int t1 = (d == 0) ? 1 : 0, t2 = (d == 2) ? 1 : 2;
         a.pen[d] = a.beta * a.ih[d];
@@ -140,12 +173,14 @@ inline void dg_derived(DGArgs<T> &a, int k)
         a.bh[d] = a.b[d] * a.h[d];
         a.bpos[d] = a.b[d] > T(0) ? a.b[d] : T(0);
         a.bneg[d] = a.b[d] < T(0) ? -a.b[d] : T(0);
-        a.m_kv[d] = T(2) * a.vsc[d];
-        a.m_ad[d] = T(2) * a.farea[d] * a.b[d];
-        a.m_pen[d] = T(0.5) * a.farea[d] * a.pen[d];
-        a.m_w[d] = T(0.5) * a.farea[d] * a.ih[d];
-        a.m_bp[d] = a.farea[d] * a.bpos[d];
-        a.m_bm[d] = a.farea[d] * a.bneg[d];
+        m.n[d] = a.n[d];
+        m.terms |= a.b[d] != T(0) ? 1 << d : 0;
+        m.kv[d] = T(2) * a.vsc[d];
+        m.ad[d] = T(2) * a.farea[d] * a.b[d];
+        m.pen[d] = T(0.5) * a.farea[d] * a.pen[d];
+        m.w[d] = T(0.5) * a.farea[d] * a.ih[d];
+        m.bp[d] = a.farea[d] * a.bpos[d];
+        m.bm[d] = a.farea[d] * a.bneg[d];
     }
 }
 
@@ -154,17 +189,17 @@ inline void dg_derived(DGArgs<T> &a, int k)
 // `dot` as in dg_apply_*, dg_modal_blocks(k, n, reaction) entries (reaction:
 // at the volume points)
 int64_t dg_modal_blocks(int k, const int *n, bool reaction);
-void dg_modal_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
+void dg_modal_apply_f64(const DGPlan<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                         double *dot);
-void dg_modal_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
+void dg_modal_apply_f32(const DGPlan<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                         double *dot);
-void dg_modal_residual_f64(const DGArgs<double> &a, int k, const double *u, const DGResidual<double> &rs,
+void dg_modal_residual_f64(const DGPlan<double> &a, int k, const double *u, const DGResidual<double> &rs,
                            const int *skip, hipStream_t s);
-void dg_modal_residual_f32(const DGArgs<float> &a, int k, const float *u, const DGResidual<float> &rs, const int *skip,
+void dg_modal_residual_f32(const DGPlan<float> &a, int k, const float *u, const DGResidual<float> &rs, const int *skip,
                            hipStream_t s);
-void dg_modal_smooth_f64(const DGArgs<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
+void dg_modal_smooth_f64(const DGPlan<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
                          hipStream_t s);
-void dg_modal_smooth_f32(const DGArgs<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
+void dg_modal_smooth_f32(const DGPlan<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
                          hipStream_t s);
 template <typename T>
 inline bool dg_is_modal(const DGArgs<T> &a)
@@ -176,9 +211,9 @@ inline bool dg_is_modal(const DGArgs<T> &a)
 // does nothing (device-driven solver loops).  `dot` (may be null): each
 // workgroup also writes its FP64 partial of <u, w> to dot[workgroup]
 // (dg_blocks(k, E) entries), for the solver's <q, A q>.
-void dg_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
+void dg_apply_f64(const DGPlan<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                   double *dot = nullptr);
-void dg_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
+void dg_apply_f32(const DGPlan<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                   double *dot = nullptr);
 // BF16 MFMA contraction variant (FP32 data and accumulation)
 void dg_apply_bf16(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s);

@@ -76,7 +76,7 @@ __device__ __forceinline__ void nbr_trace(const T *n, T &nv, T &nd)
 // nv, nd: the neighbours' traces (0 on the boundary); up1, ud1 (may be null):
 // the own traces at xi = 1
 template <int K, int D, typename T>
-__device__ __forceinline__ void line(const DGArgs<T> &a, T k, const T (&ks)[2], T w0, T w1, const T *v,
+__device__ __forceinline__ void line(const ModalArgs<T> &a, T k, const T (&ks)[2], T w0, T w1, const T *v,
                                      const T (&nv)[2], const T (&nd)[2], T *r, T *up1 = nullptr, T *ud1 = nullptr)
 {
     T t[K];
@@ -102,15 +102,15 @@ __device__ __forceinline__ void line(const DGArgs<T> &a, T k, const T (&ks)[2], 
         *ud1 = d1;
     }
     const T j0 = u0 - nv[0], j1 = u1 - nv[1];
-    T c00 = fma(a.m_pen[D] * (k + ks[0]), j0, w0 * fma(k, d0, ks[0] * nd[0]));
-    T c01 = fma(a.m_pen[D] * (k + ks[1]), j1, -w1 * fma(k, d1, ks[1] * nd[1]));
+    T c00 = fma(a.pen[D] * (k + ks[0]), j0, w0 * fma(k, d0, ks[0] * nd[0]));
+    T c01 = fma(a.pen[D] * (k + ks[1]), j1, -w1 * fma(k, d1, ks[1] * nd[1]));
     const T c10 = w0 * k * j0, c11 = -w1 * k * j1;
-    const bool adv = a.b[D] != T(0);
+    const bool adv = a.terms >> D & 1;
     if (adv) {
-        c00 = fma(a.m_bm[D], u0, fma(-a.m_bp[D], nv[0], c00));
-        c01 = fma(a.m_bp[D], u1, fma(-a.m_bm[D], nv[1], c01));
+        c00 = fma(a.bm[D], u0, fma(-a.bp[D], nv[0], c00));
+        c01 = fma(a.bp[D], u1, fma(-a.bm[D], nv[1], c01));
     }
-    const T ce = c01 + c00, co = c01 - c00, de = c11 - c10, dd = c11 + c10, kv = k * a.m_kv[D];
+    const T ce = c01 + c00, co = c01 - c00, de = c11 - c10, dd = c11 + c10, kv = k * a.kv[D];
     // sum_n L_min(m,n) v~_n over n of m's parity: L_m sh for the lowest mode
     // of its parity (m = 1, 2), sl for the highest (m = K - 2, K - 1)
     r[0] = ce;
@@ -126,7 +126,7 @@ __device__ __forceinline__ void line(const DGArgs<T> &a, T k, const T (&ks)[2], 
             T q = t[m - 1];
 #pragma unroll
             for (int n = m - 3; n >= 0; n -= 2) q += t[n];
-            r[m] = fma(-a.m_ad[D], q, r[m]);
+            r[m] = fma(-a.ad[D], q, r[m]);
         }
     }
 #pragma unroll
@@ -166,8 +166,8 @@ __device__ __forceinline__ void modal_dot(double acc, double *__restrict__ dot)
 // apply).  Q3 at 64^3: 131, 93, 80 us; Q2 at 96^3: 287, 183, 144 us.
 template <int K, typename T, bool RES>
 __global__ void __launch_bounds__(MShape<K>::NT)
-    k_dg_modal(const DGArgs<T> a, const T *__restrict__ u, T *__restrict__ w, const int *__restrict__ skip,
-               double *__restrict__ dot, const DGResidual<T> rs)
+    k_dg_modal(const ModalArgs<T> a, const ModalTile mt, const T *__restrict__ u, T *__restrict__ w,
+               const int *__restrict__ skip, double *__restrict__ dot, const DGResidual<T> rs)
 {
     using S = MShape<K>;
     constexpr int K2 = S::K2, K3 = S::K3, EPB = S::EPB, SZ = S::SZ, NT = S::NT;
@@ -176,7 +176,6 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     // the plane's u: the tile's elements, the neighbours behind its edges and
     // a slot of zeros; the y and z parts of the result; the coefficients of
     // each slot along the walk, x0 - 1 .. x1
-    const ModalTile &mt = a.mt;
     const int slots = mt.slots;
     T *const U0 = reinterpret_cast<T *>(modal_lds), *const B0 = U0 + (slots + 1) * SZ, *const K0 = B0 + EPB * SZ;
     const int tid = threadIdx.x;
@@ -216,7 +215,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     const T *ue = u + (size_t)(valid ? e : 0) * K3 + lane;
     const ptrdiff_t uw = reinterpret_cast<const char *>(w) - reinterpret_cast<const char *>(u);
     const int gye = sy ? nx : -nx, gze = sz ? nx * ny : -nx * ny;
-    const bool kcell = a.kappa_mode == FEM_KAPPA_CELL;
+    const bool kcell = a.kcell != nullptr;
 
     // v, vn, vm: the own pencils of this step and the next two; qy, qz: the
     // loaded neighbours' pencils of this step
@@ -267,7 +266,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
         // kept in registers through the walk)
         int in = inner;
         asm volatile("" : "+v"(in));
-        auto wf = [&](int d, int bit) { return (in & bit) ? a.m_w[d] : T(2) * a.m_w[d]; };
+        auto wf = [&](int d, int bit) { return (in & bit) ? a.w[d] : T(2) * a.w[d]; };
         if (valid) {
 #pragma unroll
             for (int m = 0; m < K; ++m) U[L(m, i, j)] = v[m];
@@ -341,14 +340,14 @@ __global__ void __launch_bounds__(MShape<K>::NT)
             const T ks[2] = { KS[-1], KS[1] };
 #pragma unroll
             for (int m = 0; m < K; ++m) v[m] = U[L(m, i, j)];   // (not kept through the other lines)
-            line<K, 0>(a, KS[0], ks, x > 0 ? a.m_w[0] : T(2) * a.m_w[0], up ? a.m_w[0] : T(2) * a.m_w[0], v, nv, nd, rx,
+            line<K, 0>(a, KS[0], ks, x > 0 ? a.w[0] : T(2) * a.w[0], up ? a.w[0] : T(2) * a.w[0], v, nv, nd, rx,
                        &nvl, &ndl);
-            if (a.c != T(0))
+            if (a.terms & 8)
 #pragma unroll
-                for (int m = 0; m < K; ++m) rx[m] = fma(a.m_c, v[m], rx[m]);
+                for (int m = 0; m < K; ++m) rx[m] = fma(a.c, v[m], rx[m]);
             if constexpr (RES)
                 if (a.ccell) {
-                    const T cm = a.m_vol * a.ccell[valid ? e + x - x0 : 0];
+                    const T cm = a.vol * a.ccell[valid ? e + x - x0 : 0];
 #pragma unroll
                     for (int m = 0; m < K; ++m) rx[m] = fma(cm, v[m], rx[m]);
                 }
@@ -433,8 +432,8 @@ __device__ __forceinline__ void from_points(const Tab1D<T> &tb, const T (&v)[K],
 // 8.6 us against 10.4 us, FP32 6.3 us against 7.5 us).
 template <int K, typename T, bool SM, bool RX>
 __global__ void __launch_bounds__(256)
-    k_dg_rows(const DGArgs<T> a, const T *__restrict__ u, T *__restrict__ w, const int *__restrict__ skip,
-              double *__restrict__ dot, const DGSmooth<T> sm, const DGResidual<T> rs)
+    k_dg_rows(const ModalArgs<T> a, const ModalRows mr, const ModalReaction<T> vr, const T *__restrict__ u,
+              T *__restrict__ w, const int *__restrict__ skip, double *__restrict__ dot, const DGSmooth<T> sm, const DGResidual<T> rs)
 {
     using S = MShape<K>;
     constexpr int K2 = S::K2, K3 = S::K3, EPW = S::EPW, R = 4, SZ = S::SZ;
@@ -445,7 +444,6 @@ __global__ void __launch_bounds__(256)
     const bool wr = tid < EPW * K2;
     const int el = wr ? tid / K2 : 0, i = (tid % K2) / K, j = tid % K2 % K, lane = i * K + j;
     const int nx = a.n[0], ny = a.n[1];
-    const ModalRows &mr = a.mr;
     // x-rows in groups of EPW elements, R rows per workgroup, slabs of about
     // 16 rows in y through all z
     const int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
@@ -478,7 +476,7 @@ __global__ void __launch_bounds__(256)
     T v[K], rr[K];   // own x pencil: lane (b, c)
     pencil(0, e, v);
     bool has[3][2];
-    const bool kcell = a.kappa_mode == FEM_KAPPA_CELL;
+    const bool kcell = a.kcell != nullptr;
     const T kin = kcell ? a.kcell[e] : a.kappa_const;
     T ks[3][2], nv[3][2], nd[3][2];
 #pragma unroll
@@ -499,7 +497,7 @@ __global__ void __launch_bounds__(256)
     T cq[K];
     if constexpr (RX)
 #pragma unroll
-        for (int q = 0; q < K; ++q) cq[q] = a.cvol ? a.cvol[(size_t)e * K3 + i + K * j + K2 * q] : T(0);
+        for (int q = 0; q < K; ++q) cq[q] = vr.cvol ? vr.cvol[(size_t)e * K3 + i + K * j + K2 * q] : T(0);
     if constexpr (SM) {
         const T *re = sm.r + (size_t)e * K3, *Qg = sm.Q + (size_t)e * 3 * K2, *lg = sm.lam + (size_t)e * 3 * K;
 #pragma unroll
@@ -513,7 +511,7 @@ __global__ void __launch_bounds__(256)
     if (wr)
 #pragma unroll
         for (int m = 0; m < K; ++m) A[L(m, i, j)] = v[m];
-    auto wf = [&](int d, int s) { return has[d][s] ? a.m_w[d] : T(2) * a.m_w[d]; };
+    auto wf = [&](int d, int s) { return has[d][s] ? a.w[d] : T(2) * a.w[d]; };
     T p[K], q[K], ry[K], rz[K], rx[K];
     wave_lds_sync();
 #pragma unroll
@@ -531,11 +529,11 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
         for (int m = 0; m < K; ++m) A[L(i, j, m)] += rz[m];
     line<K, 0>(a, kin, ks[0], wf(0, 0), wf(0, 1), v, nv[0], nd[0], rx);
-    if (a.c != T(0))
+    if (a.terms & 8)
 #pragma unroll
-        for (int m = 0; m < K; ++m) rx[m] = fma(a.m_c, v[m], rx[m]);
+        for (int m = 0; m < K; ++m) rx[m] = fma(a.c, v[m], rx[m]);
     if (a.ccell) {
-        const T cm = a.m_vol * a.ccell[e];
+        const T cm = a.vol * a.ccell[e];
 #pragma unroll
         for (int m = 0; m < K; ++m) rx[m] = fma(cm, v[m], rx[m]);
     }
@@ -544,7 +542,7 @@ __global__ void __launch_bounds__(256)
     for (int m = 0; m < K; ++m) rx[m] += A[L(m, i, j)];
     if constexpr (RX) {
         // int (cvol + coef u^pw) u v
-        const Tab1D<T> &tb = *a.tab;
+        const Tab1D<T> &tb = *vr.tab;
         T f[K], h[K];
         auto put = [&](int d, const T (&x)[K]) {
             if (wr)
@@ -565,13 +563,13 @@ __global__ void __launch_bounds__(256)
         put(1, h);
         get(2, f);
         to_points<K>(tb, f, h);
-        const T wij = a.m_vol * tb.w[i] * tb.w[j];
+        const T wij = a.vol * tb.w[i] * tb.w[j];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             T c = cq[k];
-            if (a.nl_pow) {
-                T pw = a.nl_coef;
-                for (int n = 0; n < a.nl_pow; ++n) pw *= h[k];
+            if (vr.nl_pow) {
+                T pw = vr.nl_coef;
+                for (int n = 0; n < vr.nl_pow; ++n) pw *= h[k];
                 c += pw;
             }
             f[k] = wij * tb.w[k] * c * h[k];
@@ -700,42 +698,52 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-template <int K, typename T, bool SM, bool RX>
-void launch_rows(const DGArgs<T> &a, const T *u, T *w, const DGSmooth<T> &sm, const DGResidual<T> &rs, const int *skip,
+template <typename T>
+ModalArgs<T> modal_args(const DGPlan<T> &p)
+{
+    ModalArgs<T> a = p.modal;
+    a.kappa_const = p.kappa_const;
+    a.kcell = p.kappa_mode == FEM_KAPPA_CELL ? p.kcell : nullptr;
+    a.ccell = p.ccell;
+    return a;
+}
+
+template <int K, typename T, bool SM>
+void launch_rows(const DGPlan<T> &p, const T *u, T *w, const DGSmooth<T> &sm, const DGResidual<T> &rs, const int *skip,
                  hipStream_t s, double *dot)
 {
-    hipLaunchKernelGGL((k_dg_rows<K, T, SM, RX>), dim3((unsigned)a.mr.blocks), dim3(256), 0, s, a, u, w, skip, dot,
-                       sm, rs);
+    const ModalReaction<T> vr{ p.cvol, p.nl_coef, p.nl_pow, p.tab };
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)p.rows.blocks), dim3(256), 0, s, modal_args(p), p.rows, vr, u, w, skip,
+                           dot, sm, rs);
+    };
+    if (p.cvol || p.nl_pow) go(k_dg_rows<K, T, SM, true>);
+    else if constexpr (SM || K == 2) go(k_dg_rows<K, T, SM, false>);
 }
 
 template <int K, typename T>
-void launch_apply(const DGArgs<T> &a, const T *u, T *w, const DGResidual<T> &rs, const int *skip, hipStream_t s,
+void launch_apply(const DGPlan<T> &p, const T *u, T *w, const DGResidual<T> &rs, const int *skip, hipStream_t s,
                   double *dot)
 {
-    if (a.cvol || a.nl_pow) {
-        launch_rows<K, T, false, true>(a, u, w, DGSmooth<T>{}, rs, skip, s, dot);
-    } else if constexpr (K == 2) {
-        launch_rows<K, T, false, false>(a, u, w, DGSmooth<T>{}, rs, skip, s, dot);
-    } else {
+    if (K == 2 || p.cvol || p.nl_pow) {
+        launch_rows<K, T, false>(p, u, w, DGSmooth<T>{}, rs, skip, s, dot);
+    } else if constexpr (K > 2) {
         using S = MShape<K>;
-        const ModalTile &t = a.mt;
+        const ModalTile &t = p.tile;
         const size_t lds = sizeof(T) * ((size_t)(t.slots + 1 + S::EPB) * S::SZ + (size_t)t.slots * t.ks);
-        if (rs.rc || a.ccell)
-            hipLaunchKernelGGL((k_dg_modal<K, T, true>), dim3((unsigned)t.blocks), dim3(S::NT), lds, s, a, u, w, skip, dot,
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)t.blocks), dim3(S::NT), lds, s, modal_args(p), t, u, w, skip, dot,
                                rs);
-        else
-            hipLaunchKernelGGL((k_dg_modal<K, T, false>), dim3((unsigned)t.blocks), dim3(S::NT), lds, s, a, u, w, skip, dot,
-                               rs);
+        };
+        if (rs.rc || p.ccell) go(k_dg_modal<K, T, true>);
+        else go(k_dg_modal<K, T, false>);
     }
 }
 
 template <int K, typename T>
-void launch_sweep(const DGArgs<T> &a, const T *u, const DGSmooth<T> &sm, const int *skip, hipStream_t s)
+void launch_sweep(const DGPlan<T> &p, const T *u, const DGSmooth<T> &sm, const int *skip, hipStream_t s)
 {
-    const bool rx = a.cvol || a.nl_pow;
-    const DGResidual<T> rs;
-    if (rx) launch_rows<K, T, true, true>(a, u, nullptr, sm, rs, skip, s, nullptr);
-    else launch_rows<K, T, true, false>(a, u, nullptr, sm, rs, skip, s, nullptr);
+    launch_rows<K, T, true>(p, u, nullptr, sm, DGResidual<T>{}, skip, s, nullptr);
 }
 
 #define MODAL_SWITCH(CALL)                                                             \
@@ -749,14 +757,14 @@ void launch_sweep(const DGArgs<T> &a, const T *u, const DGSmooth<T> &sm, const i
     FEM_HIP(hipGetLastError())
 
 template <typename T>
-void modal_check(const DGArgs<T> &a, int k)
+void modal_check(const DGPlan<T> &a, int k)
 {
     FEM_CHECK((int64_t)a.n[0] * a.n[1] * a.n[2] * k * k * k < (int64_t)1 << 31, FEM_ERR_UNSUPPORTED,
               "DG apply: more than 2^31 DoFs");
 }
 
 template <typename T>
-void modal_apply(const DGArgs<T> &a, int k, const T *u, T *w, const DGResidual<T> &rs, const int *skip, hipStream_t s,
+void modal_apply(const DGPlan<T> &a, int k, const T *u, T *w, const DGResidual<T> &rs, const int *skip, hipStream_t s,
                  double *dot)
 {
     modal_check(a, k);
@@ -767,7 +775,7 @@ void modal_apply(const DGArgs<T> &a, int k, const T *u, T *w, const DGResidual<T
 }
 
 template <typename T>
-void modal_smooth(const DGArgs<T> &a, int k, const T *u, const DGSmooth<T> &sm, const int *skip, hipStream_t s)
+void modal_smooth(const DGPlan<T> &a, int k, const T *u, const DGSmooth<T> &sm, const int *skip, hipStream_t s)
 {
     modal_check(a, k);
     FEM_CHECK(dg_is_modal(a), FEM_ERR_UNSUPPORTED, "smoothing sweep: cellwise or constant kappa");
@@ -868,32 +876,32 @@ template void dg_block_apply<double>(int, int64_t, const double *, const double 
 template void dg_block_apply<float>(int, int64_t, const float *, const float *, const float *, const float *, float *,
                                     float, bool, const int *, hipStream_t, double *);
 
-void dg_modal_apply_f64(const DGArgs<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
+void dg_modal_apply_f64(const DGPlan<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                         double *dot)
 {
     modal_apply<double>(a, k, u, w, DGResidual<double>{}, skip, s, dot);
 }
-void dg_modal_apply_f32(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
+void dg_modal_apply_f32(const DGPlan<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                         double *dot)
 {
     modal_apply<float>(a, k, u, w, DGResidual<float>{}, skip, s, dot);
 }
-void dg_modal_residual_f64(const DGArgs<double> &a, int k, const double *u, const DGResidual<double> &rs,
+void dg_modal_residual_f64(const DGPlan<double> &a, int k, const double *u, const DGResidual<double> &rs,
                            const int *skip, hipStream_t s)
 {
     modal_apply<double>(a, k, u, nullptr, rs, skip, s, nullptr);
 }
-void dg_modal_residual_f32(const DGArgs<float> &a, int k, const float *u, const DGResidual<float> &rs, const int *skip,
+void dg_modal_residual_f32(const DGPlan<float> &a, int k, const float *u, const DGResidual<float> &rs, const int *skip,
                            hipStream_t s)
 {
     modal_apply<float>(a, k, u, nullptr, rs, skip, s, nullptr);
 }
-void dg_modal_smooth_f64(const DGArgs<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
+void dg_modal_smooth_f64(const DGPlan<double> &a, int k, const double *u, const DGSmooth<double> &sm, const int *skip,
                          hipStream_t s)
 {
     modal_smooth<double>(a, k, u, sm, skip, s);
 }
-void dg_modal_smooth_f32(const DGArgs<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
+void dg_modal_smooth_f32(const DGPlan<float> &a, int k, const float *u, const DGSmooth<float> &sm, const int *skip,
                          hipStream_t s)
 {
     modal_smooth<float>(a, k, u, sm, skip, s);

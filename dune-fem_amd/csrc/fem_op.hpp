@@ -43,8 +43,8 @@ struct Operator {
     int64_t E = 0, N = 0;
     int vec_prec = FEM_F64;  // precision of the vectors it acts on
     // DG
-    DGArgs<double> a64{};
-    DGArgs<float> a32{};
+    DGPlan<double> a64{};
+    DGPlan<float> a32{};
     DevBuf tab64, tab32;
     DevBuf kvol64, kface64[3], kcell64, kvol32, kface32[3], kcell32;
     // CG
