@@ -88,17 +88,18 @@ struct DGArgs {
 };
 static_assert(sizeof(DGArgs<double>) <= 416, "what a launch of a quadrature kernel copies");
 
-// kernel arguments of the line kernels (fem_dg_modal.hip): per direction
-// 2 |K| / h^2, 2 |F| b, |F| beta / (2 h), |F| / (2 h), |F| max(b, 0),
-// |F| max(-b, 0), then c |K| and |K|; the coefficients as in DGArgs
+// kernel arguments of the line kernels (fem_dg_modal.hip): the coefficients as in
+// DGArgs, then per direction 2 |K| / h^2, 2 |F| b, |F| beta / (2 h), |F| / (2 h),
+// |F| max(b, 0), |F| max(-b, 0), and c |K| and |K|
 template <typename T>
 struct ModalArgs {
     int n[3];
-    int terms;   // bits 0..2: b[d] is not 0, bit 3: c is not 0
-    T kv[3], ad[3], pen[3], w[3], bp[3], bm[3], c, vol;
+    T b[3];
+    T c;
+    int kappa_mode;
     T kappa_const;
-    const T *kcell;   // null: kappa_const
-    const T *ccell;
+    const T *kcell, *ccell;
+    T kv[3], ad[3], pen[3], w[3], bp[3], bm[3], cv, vol;
 };
 // the reaction at the volume points, as in DGArgs
 template <typename T>
@@ -163,8 +164,8 @@ inline void dg_derived(DGPlan<T> &a, int k)
     a.rows = dg_modal_rows(k, a.n);
     ModalArgs<T> &m = a.modal;
     m.vol = a.h[0] * a.h[1] * a.h[2];
-    m.c = a.c * m.vol;
-    m.terms = a.c != T(0) ? 8 : 0;
+    m.c = a.c;
+    m.cv = a.c * m.vol;
     for (int d = 0; d < 3; ++d) {
         const int t1 = (d == 0) ? 1 : 0, t2 = (d == 2) ? 1 : 2;
         a.pen[d] = a.beta * a.ih[d];
@@ -174,7 +175,7 @@ inline void dg_derived(DGPlan<T> &a, int k)
         a.bpos[d] = a.b[d] > T(0) ? a.b[d] : T(0);
         a.bneg[d] = a.b[d] < T(0) ? -a.b[d] : T(0);
         m.n[d] = a.n[d];
-        m.terms |= a.b[d] != T(0) ? 1 << d : 0;
+        m.b[d] = a.b[d];
         m.kv[d] = T(2) * a.vsc[d];
         m.ad[d] = T(2) * a.farea[d] * a.b[d];
         m.pen[d] = T(0.5) * a.farea[d] * a.pen[d];

@@ -105,7 +105,7 @@ __device__ __forceinline__ void line(const ModalArgs<T> &a, T k, const T (&ks)[2
     T c00 = fma(a.pen[D] * (k + ks[0]), j0, w0 * fma(k, d0, ks[0] * nd[0]));
     T c01 = fma(a.pen[D] * (k + ks[1]), j1, -w1 * fma(k, d1, ks[1] * nd[1]));
     const T c10 = w0 * k * j0, c11 = -w1 * k * j1;
-    const bool adv = a.terms >> D & 1;
+    const bool adv = a.b[D] != T(0);
     if (adv) {
         c00 = fma(a.bm[D], u0, fma(-a.bp[D], nv[0], c00));
         c01 = fma(a.bp[D], u1, fma(-a.bm[D], nv[1], c01));
@@ -215,7 +215,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     const T *ue = u + (size_t)(valid ? e : 0) * K3 + lane;
     const ptrdiff_t uw = reinterpret_cast<const char *>(w) - reinterpret_cast<const char *>(u);
     const int gye = sy ? nx : -nx, gze = sz ? nx * ny : -nx * ny;
-    const bool kcell = a.kcell != nullptr;
+    const bool kcell = a.kappa_mode == FEM_KAPPA_CELL;
 
     // v, vn, vm: the own pencils of this step and the next two; qy, qz: the
     // loaded neighbours' pencils of this step
@@ -260,6 +260,11 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     auto L = [&](int a_, int b_, int c_) { return midx<K>(a_, b_, c_); };
     const int inner = (hy0 ? 1 : 0) | (hy1 ? 2 : 0) | (hz0 ? 4 : 0) | (hz1 ? 8 : 0);
     double acc = 0;
+    // the loads above have landed before the walk.  Left to the compiler, a wait
+    // for them can end up inside the loop, behind the loads for the next step
+    // that the step is to hide (64^3 Q4 FP64 165 us, then 171 to 199 us)
+#pragma unroll
+    for (int m = 0; m < K; ++m) asm volatile("" : "+v"(v[m]), "+v"(vn[m]), "+v"(qy[m]), "+v"(qz[m]));
     for (int x = x0; x < x1; ++x) {
         const bool up = x + 1 < nx, more = x + 1 < x1;
         // (opaque: the boundary weights are formed where they are used, not
@@ -342,9 +347,9 @@ __global__ void __launch_bounds__(MShape<K>::NT)
             for (int m = 0; m < K; ++m) v[m] = U[L(m, i, j)];   // (not kept through the other lines)
             line<K, 0>(a, KS[0], ks, x > 0 ? a.w[0] : T(2) * a.w[0], up ? a.w[0] : T(2) * a.w[0], v, nv, nd, rx,
                        &nvl, &ndl);
-            if (a.terms & 8)
+            if (a.c != T(0))
 #pragma unroll
-                for (int m = 0; m < K; ++m) rx[m] = fma(a.c, v[m], rx[m]);
+                for (int m = 0; m < K; ++m) rx[m] = fma(a.cv, v[m], rx[m]);
             if constexpr (RES)
                 if (a.ccell) {
                     const T cm = a.vol * a.ccell[valid ? e + x - x0 : 0];
@@ -476,7 +481,7 @@ __global__ void __launch_bounds__(256)
     T v[K], rr[K];   // own x pencil: lane (b, c)
     pencil(0, e, v);
     bool has[3][2];
-    const bool kcell = a.kcell != nullptr;
+    const bool kcell = a.kappa_mode == FEM_KAPPA_CELL;
     const T kin = kcell ? a.kcell[e] : a.kappa_const;
     T ks[3][2], nv[3][2], nd[3][2];
 #pragma unroll
@@ -529,9 +534,9 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
         for (int m = 0; m < K; ++m) A[L(i, j, m)] += rz[m];
     line<K, 0>(a, kin, ks[0], wf(0, 0), wf(0, 1), v, nv[0], nd[0], rx);
-    if (a.terms & 8)
+    if (a.c != T(0))
 #pragma unroll
-        for (int m = 0; m < K; ++m) rx[m] = fma(a.c, v[m], rx[m]);
+        for (int m = 0; m < K; ++m) rx[m] = fma(a.cv, v[m], rx[m]);
     if (a.ccell) {
         const T cm = a.vol * a.ccell[e];
 #pragma unroll
@@ -702,8 +707,9 @@ template <typename T>
 ModalArgs<T> modal_args(const DGPlan<T> &p)
 {
     ModalArgs<T> a = p.modal;
+    a.kappa_mode = p.kappa_mode;
     a.kappa_const = p.kappa_const;
-    a.kcell = p.kappa_mode == FEM_KAPPA_CELL ? p.kcell : nullptr;
+    a.kcell = p.kcell;
     a.ccell = p.ccell;
     return a;
 }
