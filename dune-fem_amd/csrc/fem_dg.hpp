@@ -36,6 +36,8 @@ struct ModalTile {
     UDiv dv_ty, dv_nty, dv_plane;   // by ty, nty, nty ntz
 };
 ModalTile dg_modal_tile(int k, const int *n);
+// whether the apply on n[0] x n[1] x n[2] elements takes the walk, not the rows
+bool dg_modal_walks(int k, const int *n, const ModalTile &t);
 // traversal by rows: nxg groups of elements per x-row, four rows per
 // workgroup, slabs of ty workgroups in y (about 16 rows), each through all z
 struct ModalRows {
@@ -117,6 +119,7 @@ struct DGPlan : DGArgs<T> {
     ModalArgs<T> modal;   // (kappa and ccell are filled in at the launch)
     ModalRows rows;
     ModalTile tile;
+    bool walks;
 };
 
 // the damped block-Jacobi sweep fused into the apply (multigrid smoothing):
@@ -162,6 +165,7 @@ inline void dg_derived(DGPlan<T> &a, int k)
     }
     a.tile = dg_modal_tile(k, a.n);
     a.rows = dg_modal_rows(k, a.n);
+    a.walks = dg_modal_walks(k, a.n, a.tile);
     ModalArgs<T> &m = a.modal;
     m.vol = a.h[0] * a.h[1] * a.h[2];
     m.c = a.c;

@@ -433,8 +433,9 @@ __device__ __forceinline__ void from_points(const Tab1D<T> &tb, const T (&v)[K],
 //     the Gauss points and back.
 // The sweep needs the registers and the LDS of a walk for the element block
 // (48^3 Q3 FP64: the V-cycle with a walking sweep 458 us, with this one 415 us),
-// and at Q1 a step of a walk is too short for its barriers (48^3: FP64 apply
-// 8.6 us against 10.4 us, FP32 6.3 us against 7.5 us).
+// at Q1 a step of a walk is too short for its barriers (48^3: FP64 apply
+// 8.6 us against 10.4 us, FP32 6.3 us against 7.5 us), and a mesh thin in y and z
+// leaves its lanes idle (dg_modal_walks).
 template <int K, typename T, bool SM, bool RX>
 __global__ void __launch_bounds__(256)
     k_dg_rows(const ModalArgs<T> a, const ModalRows mr, const ModalReaction<T> vr, const T *__restrict__ u,
@@ -724,14 +725,14 @@ void launch_rows(const DGPlan<T> &p, const T *u, T *w, const DGSmooth<T> &sm, co
                            dot, sm, rs);
     };
     if (p.cvol || p.nl_pow) go(k_dg_rows<K, T, SM, true>);
-    else if constexpr (SM || K == 2) go(k_dg_rows<K, T, SM, false>);
+    else go(k_dg_rows<K, T, SM, false>);
 }
 
 template <int K, typename T>
 void launch_apply(const DGPlan<T> &p, const T *u, T *w, const DGResidual<T> &rs, const int *skip, hipStream_t s,
                   double *dot)
 {
-    if (K == 2 || p.cvol || p.nl_pow) {
+    if (!p.walks || p.cvol || p.nl_pow) {
         launch_rows<K, T, false>(p, u, w, DGSmooth<T>{}, rs, skip, s, dot);
     } else if constexpr (K > 2) {
         using S = MShape<K>;
@@ -844,6 +845,21 @@ ModalTile dg_modal_tile(int k, const int *n)
     return t;
 }
 
+// Q1 steps are too short for a walk (see k_dg_rows).  Otherwise the walk, if at
+// least half of a tile's elements exist: on a mesh thin in y and z a workgroup
+// walks along x with few lanes at work, and nothing is left to share through
+// LDS.  Q3 FP64, 20000 x 1 x 1 elements (1/16 of a tile): 46 us walking, 10.6 us by
+// rows; 60000 x 2 x 2 (1/4): 135 and 75 us; 60000 x 3 x 3 (9/16): 190 and 230 us.
+// At Q2 the same meshes have 1/28, 1/7 and 9/28 of a tile: 31.7 and 6.7, 97 and 42, 113
+// and 80 us; Q4 1/8, 1/2 and 9/16: 58 and 20, 221 and 243, 528 and 559 us.  Idle
+// lanes cost nothing while all workgroups run at once (768 do at three per CU):
+// 700 x 6 x 1 Q3 5.0 and 5.2 us, 1600 x 3 x 3 Q2 7.7 and 5.9 us.
+bool dg_modal_walks(int k, const int *n, const ModalTile &t)
+{
+    const int64_t epb = 4 * (64 / (k * k));
+    return k > 2 && (2 * (int64_t)n[1] * n[2] >= (int64_t)t.nty * t.ntz * epb || t.blocks <= 768);
+}
+
 ModalRows dg_modal_rows(int k, const int *n)
 {
     ModalRows r;
@@ -859,7 +875,8 @@ ModalRows dg_modal_rows(int k, const int *n)
 
 int64_t dg_modal_blocks(int k, const int *n, bool reaction)
 {
-    return k == 2 || reaction ? dg_modal_rows(k, n).blocks : dg_modal_tile(k, n).blocks;
+    const ModalTile t = dg_modal_tile(k, n);
+    return reaction || !dg_modal_walks(k, n, t) ? dg_modal_rows(k, n).blocks : t.blocks;
 }
 
 int64_t dg_bj_blocks(int k, int64_t E)
