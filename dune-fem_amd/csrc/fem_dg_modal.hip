@@ -212,8 +212,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     T *const Hy = U0 + sly * SZ, *const Hz = U0 + slz * SZ;
     const int e = x0 + nx * (ey + ny * ez);
     const int lane = i * K + j;
-    const T *ue = u + (size_t)(valid ? e : 0) * K3 + lane;
-    const ptrdiff_t uw = reinterpret_cast<const char *>(w) - reinterpret_cast<const char *>(u);
+    unsigned ou = (unsigned)((valid ? e : 0) * K3 + lane);   // (below 2^31: modal_check)
     const int gye = sy ? nx : -nx, gze = sz ? nx * ny : -nx * ny;
     const bool kcell = a.kappa_mode == FEM_KAPPA_CELL;
 
@@ -226,10 +225,10 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     if (valid) {
         const int xn = x0 + 1 < nx ? 1 : 0;
 #pragma unroll
-        for (int m = 0; m < K; ++m) v[m] = ue[m * K2];
+        for (int m = 0; m < K; ++m) v[m] = u[(size_t)ou + m * K2];
         if (xn)
 #pragma unroll
-            for (int m = 0; m < K; ++m) vn[m] = ue[m * K2 + K3];
+            for (int m = 0; m < K; ++m) vn[m] = u[(size_t)ou + m * K2 + K3];
         for (int t = lane; t < x1 - x0 + 2; t += K2) {
             int x = x0 - 1 + t;
             x = x < 0 ? 0 : x < nx ? x : nx - 1;
@@ -237,14 +236,14 @@ __global__ void __launch_bounds__(MShape<K>::NT)
         }
     }
     if (ldy) {
-        const T *gy = ue + (ptrdiff_t)gye * K3;
+        const T *gy = u + (ou + gye * K3);
 #pragma unroll
         for (int m = 0; m < K; ++m) qy[m] = gy[m * K2];
         for (int t = lane; t < x1 - x0; t += K2)
             K0[sly * mt.ks + 1 + t] = kcell ? a.kcell[e + gye + t] : a.kappa_const;
     }
     if (ldz) {
-        const T *gz = ue + (ptrdiff_t)gze * K3;
+        const T *gz = u + (ou + gze * K3);
 #pragma unroll
         for (int m = 0; m < K; ++m) qz[m] = gz[m * K2];
         for (int t = lane; t < x1 - x0; t += K2)
@@ -254,7 +253,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
     if (valid && x0 > 0) {
         T n[K];
 #pragma unroll
-        for (int m = 0; m < K; ++m) n[m] = ue[m * K2 - K3];
+        for (int m = 0; m < K; ++m) n[m] = u[(size_t)ou + m * K2 - K3];
         nbr_trace<K, false>(n, nvl, ndl);
     }
     auto L = [&](int a_, int b_, int c_) { return midx<K>(a_, b_, c_); };
@@ -285,7 +284,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
             for (int m = 0; m < K; ++m) Hz[L(m, i, j)] = qz[m];
         }
         if (more) {
-            const T *gy = ue + (ptrdiff_t)(gye + 1) * K3, *gz = ue + (ptrdiff_t)(gze + 1) * K3;
+            const T *gy = u + (ou + (gye + 1) * K3), *gz = u + (ou + (gze + 1) * K3);
             if (ldy) {
 #pragma unroll
                 for (int m = 0; m < K; ++m) qy[m] = gy[m * K2];
@@ -295,6 +294,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
                 for (int m = 0; m < K; ++m) qz[m] = gz[m * K2];
             }
             const bool up2 = x + 2 < nx;
+            const T *ue = u + ou;
             if (valid) {
 #pragma unroll
                 for (int m = 0; m < K; ++m) vm[m] = up2 ? ue[m * K2 + 2 * K3] : T(0);
@@ -373,7 +373,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
             }
         } else {
             if (valid) {
-                T *we = reinterpret_cast<T *>(reinterpret_cast<char *>(const_cast<T *>(ue)) + uw);
+                T *we = w + ou;
 #pragma unroll
                 for (int m = 0; m < K; ++m) {
                     we[m * K2] = rx[m];
@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(MShape<K>::NT)
             vn[m] = vm[m];
         }
         ++KS;
-        ue += K3;
+        ou += K3;
         __syncthreads();
     }
     if (dot) modal_dot<NT>(acc, dot);
