@@ -306,7 +306,8 @@ struct Ctr {
 };
 
 // KQ: kappa given at the quadrature points (FEM_KAPPA_QP); otherwise one
-// value per element (FEM_KAPPA_CELL) or one constant (FEM_KAPPA_CONST).
+// value per element (FEM_KAPPA_CELL) or one constant (FEM_KAPPA_CONST), for the
+// BF16 contractions only: FP64 and FP32 then take the line kernels.
 template <int K, typename T, bool MF, bool KQ, bool RX = false>
 __global__ void __launch_bounds__(ApplyShape<K>::WG)
     k_dg_apply(const DGArgs<T> a, const T *__restrict__ u, T *__restrict__ w, const int *__restrict__ skip,
@@ -317,10 +318,11 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
     if (skip && *skip) return;
     // FP64 MFMA path (K = 4, lane 16 i + 4 el + j): a 16-lane LDS access
     // group holds one i of all four elements.  The layout (a, b, c) ->
-    // a * 20 + b * 5 + c with an element stride of 164 doubles puts every
+    // a * 20 + b * 5 + c with an element stride of 244 doubles puts every
     // pencil access pattern of the kernel on 16 distinct 8-byte banks, with
     // compile-time offsets only (searched exhaustively over additive layouts).
     // Otherwise the layout of DGShape (one element per 16-lane group).
+    static_assert(MF ? !RX : KQ, "what the launcher takes");
     constexpr bool F64MF_ = (K == 4) && std::is_same<T, double>::value && !MF;
     // K = 3 and 5 without BF16 MFMA (lane el K^2 + i K + j): unpadded
     // tensors (a, b, c) -> a K^2 + b K + c, face-trace scratch rows of 4 at
@@ -342,8 +344,8 @@ __global__ void __launch_bounds__(ApplyShape<K>::WG)
     // pointwise-kappa apply: the kernel without it keeps its code and registers
     // (with kappa constant per element the modal kernels have it)
     constexpr bool CV = RX;
-    constexpr int SZ = F64MF_ ? (KLDS ? 244 : 164) : D35 ? (K == 3 ? 107 : 361) : S::SZ;
-    static_assert(!F64MF_ || SZ >= (KLDS ? 3 : 2) * K * S1, "tensors per element");
+    constexpr int SZ = F64MF_ ? 244 : D35 ? (K == 3 ? 107 : 361) : S::SZ;
+    static_assert(!F64MF_ || SZ >= 3 * K * S1, "tensors per element");
     static_assert(F64MF_ || SZ >= 2 * K * S1 + 4 * SXQ, "tensors and face-trace scratch per element");
     // DGShape layout at K = 4: the third tensor ends at 2 TS + lidx(3,3,3) + 1
     static_assert(F64MF_ || !KLDS || SZ >= 2 * K * S1 + 3 * S1 + 3 * K + 4, "tensors per element");

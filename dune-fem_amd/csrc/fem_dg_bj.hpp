@@ -5,10 +5,9 @@
 // columns are eigenvectors) and eigenvalues le [3][K].  One element is handled
 // by K*K lanes (i, j).  The phases read and rewrite the pencils of one
 // direction, which partition the tensor, so only the direction changes need a
-// barrier.  The transform synchronises the group of G lanes that holds the
-// element (one wavefront, or the workgroup for G > 64): every lane of it must
-// call it.  Lanes without an element of their own (wr false) shadow another's
-// and write nothing.
+// barrier.  An element lies within one wavefront, every lane of which must call
+// the transform.  Lanes without an element of their own (wr false) shadow
+// another's and write nothing.
 #pragma once
 
 #include "fem_dg_sync.hpp"
@@ -18,7 +17,7 @@ namespace femamd {
 // the transform with the eigen data in LDS (Qs = Qe, le, synchronised), for
 // lanes that pass and receive the x pencil y[0..K)[i][j]; A(a, b, c) gives
 // the address of a tensor entry in the element's LDS scratch
-template <int K, typename T, int G, typename A3>
+template <int K, typename T, typename A3>
 __device__ __forceinline__ void bj_transform_x(A3 A, const T *Qs, int i, int j, bool wr, T (&v)[K])
 {
     constexpr int K2 = K * K;
@@ -38,7 +37,7 @@ __device__ __forceinline__ void bj_transform_x(A3 A, const T *Qs, int i, int j, 
     if (wr)
 #pragma unroll
         for (int r = 0; r < K; ++r) A(r, i, j) = tmp[r];
-    lds_sync<G>();
+    wave_lds_sync();
     // y: lane (i=a', j=c)
 #pragma unroll
     for (int b = 0; b < K; ++b) v[b] = A(i, b, j);
@@ -46,7 +45,7 @@ __device__ __forceinline__ void bj_transform_x(A3 A, const T *Qs, int i, int j, 
     if (wr)
 #pragma unroll
         for (int r = 0; r < K; ++r) A(i, r, j) = tmp[r];
-    lds_sync<G>();
+    wave_lds_sync();
     // z, scale, back: lane (i=a', j=b')
 #pragma unroll
     for (int c = 0; c < K; ++c) v[c] = A(i, j, c);
@@ -58,14 +57,14 @@ __device__ __forceinline__ void bj_transform_x(A3 A, const T *Qs, int i, int j, 
     if (wr)
 #pragma unroll
         for (int r = 0; r < K; ++r) A(i, j, r) = tmp[r];
-    lds_sync<G>();
+    wave_lds_sync();
 #pragma unroll
     for (int b = 0; b < K; ++b) v[b] = A(i, b, j);
     mul(1, false);
     if (wr)
 #pragma unroll
         for (int r = 0; r < K; ++r) A(i, r, j) = tmp[r];
-    lds_sync<G>();
+    wave_lds_sync();
 #pragma unroll
     for (int a = 0; a < K; ++a) v[a] = A(a, i, j);
     mul(0, false);

@@ -443,7 +443,6 @@ __global__ void __launch_bounds__(256)
 {
     using S = MShape<K>;
     constexpr int K2 = S::K2, K3 = S::K3, EPW = S::EPW, R = 4, SZ = S::SZ;
-    constexpr int KC = (K + 1) / 2;   // modes of the next DG level: order (K - 1) / 2
     if (skip && *skip) return;
     __shared__ T smem[R * EPW * (SZ + (SM ? S::SQ : 0))];
     const int g = threadIdx.x >> 6, tid = threadIdx.x & 63;
@@ -640,7 +639,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int m = 0; m < K; ++m) rx[m] = rr[m] - rx[m];
     wave_lds_sync();
-    bj_transform_x<K, T, 64>([&](int a_, int b_, int c_) -> T & { return A[L(a_, b_, c_)]; }, Q, i, j, wr, rx);
+    bj_transform_x<K, T>([&](int a_, int b_, int c_) -> T & { return A[L(a_, b_, c_)]; }, Q, i, j, wr, rx);
     if (active) {
         T *xe = sm.xout + (size_t)e * K3 + lane;
 #pragma unroll
@@ -685,7 +684,7 @@ __global__ void __launch_bounds__(256)
         for (int k = lane; k < 3 * K; k += K2) Q[3 * K2 + k] = le[k];
     }
     wave_lds_sync();
-    bj_transform_x<K, T, 64>([&](int a_, int b_, int c_) -> T & { return A[midx<K>(a_, b_, c_)]; }, Q, i, j, wr, v);
+    bj_transform_x<K, T>([&](int a_, int b_, int c_) -> T & { return A[midx<K>(a_, b_, c_)]; }, Q, i, j, wr, v);
     double a1 = 0, a2 = 0;
     if (active) {
         T *ye = y + e * K3 + lane;
