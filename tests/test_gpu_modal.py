@@ -217,3 +217,57 @@ def test_direction_of_a_thin_mesh_does_not_matter_for_time(ctx):
         t.append(best)
     print("thin", [round(1e4 * v, 1) for v in t], flush=True)
     assert t[0] < 2.5 * t[1]
+
+
+# meshes whose walks take three steps (the last two) and sixteen (the last
+# fifteen), with a remainder of the tile in y and in z
+WALKS = [((11, 103, 107), 2), ((11, 81, 85), 3), ((11, 57, 59), 4),
+         ((47, 135, 137), 2), ((47, 101, 105), 3), ((47, 71, 75), 4)]
+
+
+@pytest.mark.parametrize("prec,tol", [(fa.F64, 1e-12), (fa.F32, 2e-5)])
+@pytest.mark.parametrize("n,p", WALKS)
+def test_long_walks_equal_rows(ctx, n, p, prec, tol):
+    """A pointwise reaction of zeros sends the same operator by rows, without a walk:
+    the same lines, added in another order."""
+    rng = np.random.default_rng(p)
+    E = n[0] * n[1] * n[2]
+    op = operator(ctx, n, p, (1, -.5, .25), 0.3, np.exp(rng.normal(size=E)), prec)
+    u = rng.standard_normal(op.N, dtype=np.float64 if prec == fa.F64 else np.float32)
+    U, W = op.vector(u), op.vector()
+    W.fill(np.nan)
+    op(U, W)
+    walk = W.download()
+    op.set_reaction_qp(np.zeros((E, (p + 1) ** 3)))
+    W.fill(np.nan)
+    op(U, W)
+    err = rel(walk, W.download())
+    print("walk", n, p, prec, err, flush=True)
+    assert err < tol
+
+
+@pytest.mark.parametrize("n,p", WALKS[:3])
+def test_residual_of_a_long_walk_equals_rows(ctx, n, p):
+    """V-cycles of the same operator, its reaction once as the constant c (the
+    residual by a walk on every level above Q1) and once as values at the points
+    (the finest residual by rows, the coarser ones by a walk with a reaction per
+    element).  Bars as in test_gpu_multigrid.py."""
+    rng = np.random.default_rng(p)
+    E = n[0] * n[1] * n[2]
+    kappa, c = np.exp(rng.normal(size=E)), 7.0
+    r = rng.normal(size=E * (p + 1) ** 3)
+    for prec in (fa.F64, fa.F32):
+        z = []
+        for points in (False, True):
+            op = operator(ctx, n, p, (0, 0, 0), 0.0 if points else c, kappa, prec)
+            if points:
+                op.set_reaction_qp(np.full((E, (p + 1) ** 3), c))
+            R, Z = op.vector(r), op.vector()
+            Z.fill(np.nan)
+            fa.Preconditioner(op, fa.PRE_MULTIGRID)(R, Z)
+            z.append(Z.download())
+        print("residual", n, p, prec, rel(*z), flush=True)
+        if prec == fa.F64:
+            assert rel(*z) < 1e-12
+        else:
+            assert np.linalg.norm(z[0] - z[1]) < 1e-4 * np.linalg.norm(z[1])

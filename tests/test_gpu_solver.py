@@ -418,3 +418,42 @@ def test_cg_steps_match_the_recurrence(ctx, case, graph):
         err = np.linalg.norm(X.download() - x) / np.linalg.norm(x)
         print("cg", case, k, err, flush=True)
         assert err < (1e-8 if prec == fa.F64 else 1e-2)
+
+
+@pytest.mark.parametrize("prec", [fa.F64, fa.F32])
+def test_cg_steps_with_many_block_jacobi_partials(ctx, prec):
+    # 64 x 65 x 65 Q1 elements: 4420 workgroups of the apply and 4225 of block
+    # Jacobi, so both of its lists and that of <q, A q> are first brought down to
+    # fewer.  Bars as in test_cg_steps_match_the_recurrence
+    n, rng = (64, 65, 65), np.random.default_rng(5)
+    op = fa.GalerkinOperator(ctx, fa.OP_DG_SIPG_3D, n, 1, 10.0, (0, 0, 0), 0.0, fa.KAPPA_CELL, precision=prec)
+    op.set_kappa_cell(rng.uniform(0.5, 2.0, size=n[0] * n[1] * n[2]))
+    pre = fa.Preconditioner(op, fa.PRE_BLOCK_JACOBI)
+    U, W = op.vector(), op.vector()
+
+    def on_device(call, v):
+        U.upload(v)
+        call(U, W)
+        return W.download().astype(np.float64)
+
+    b = rng.normal(size=op.N)
+    for k in (1, 2, 6):
+        x, r = np.zeros(op.N), b
+        q = s = on_device(pre, r)
+        res = np.dot(r, s)
+        for it in range(k):
+            q = s + beta * q if it else s
+            h = on_device(op, q)
+            alpha = res / np.dot(q, h)
+            x, r = x + alpha * q, r - alpha * h
+            s = on_device(pre, r)
+            new = np.dot(r, s)
+            beta, res = new / res, new
+        inv = fa.InverseOperator(ctx, method=fa.CG, tolerance=1e-30, errormeasure=fa.RELATIVE, maxiterations=k)
+        inv.bind(op, pre)
+        X = op.vector(np.zeros(op.N))
+        inv(op.vector(b), X)
+        assert inv.iterations() == -k
+        err = np.linalg.norm(X.download() - x) / np.linalg.norm(x)
+        print("cg many", k, err, flush=True)
+        assert err < (1e-8 if prec == fa.F64 else 1e-2)
