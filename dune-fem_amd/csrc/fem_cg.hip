@@ -32,9 +32,10 @@ CGTab make_cg_tab()
 // w = A u (APPLY), the diagonal, the load vector.  The apply moves 9 coefficients per
 // element and two vectors, and on a few hundred thousand elements it is a single set of
 // workgroups, so what counts is the chain of one of them: 517 x 386 FP64 with pointwise
-// kappa 7.1 us (27 MB; 12.8 us with FP64 tables converted at each use, four coloured
-// additions into LDS with a barrier each, and neighbouring tiles on different XCDs; of
-// that last 1.8 us), 1024^2 26 us (49.6 us).  tile_inst names the instance of a
+// kappa 7.1 us back to back on vectors that the caches keep (27 MB; 12.2 us with FP64 tables
+// converted at each use, four coloured additions into LDS with a barrier each, and
+// neighbouring tiles on different XCDs, of that last 1.8 us), 8.7 us (13.5 us) where the
+// vectors change from call to call; 1024^2 26 us (49.6 us).  tile_inst names the instance of a
 // workgroup, one load where a search over the instances' first tiles was a chain of five
 // to eight; a single instance comes with the arguments.
 template <int TX, int TY, typename T, bool APPLY, bool RX>

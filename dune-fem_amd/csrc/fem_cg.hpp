@@ -23,8 +23,10 @@ struct CGInst {
 // tile shapes available to the autotuner (owned elements per tile)
 constexpr int CG_NSHAPES = 5;
 constexpr int CG_SHAPES[CG_NSHAPES][2] = { { 15, 15 }, { 7, 7 }, { 15, 7 }, { 31, 7 }, { 7, 31 } };
-// the shape of a single instance's operator: FP64, pointwise kappa, 517 x 386 elements
-// 7.1 us (7 x 7: 8.3, 15 x 7: 7.4, 31 x 7: 7.4), 1024^2 27.7 us (32.4, 27.7, 26.5)
+// the shape of a single instance's operator: FP64, pointwise kappa, back to back on the
+// same vectors, 517 x 386 elements 7.1 us (7 x 7: 8.3, 15 x 7: 7.4, 31 x 7: 7.4), 1024^2
+// 27.7 us (32.4, 27.7, 26.5): 31 x 7 is ahead by 4 % where the chip is full many times
+// over, behind by as much at a single set of workgroups
 constexpr int CG_SINGLE = 0;
 
 // an instance of nx x ny elements in tiles of the given shape

@@ -178,7 +178,8 @@ __global__ void k_csr_q2_extract(Q2Dims d, const T *__restrict__ y, const int64_
 // row's additions is that of a wavefront per row).  Q2, 18 x 16 x 20 elements, FP64
 // (28.0M nonzeros, 224 MB): 40.9 us, with the column indices and a wavefront per row
 // 88 us.
-constexpr int csr_rows(int nb) { return nb <= 27 ? 8 : 4; }   // rows of a wavefront: 24 to 56 loads in flight per lane
+// rows of a wavefront: a lane has 8, 24, 28 and 56 values in flight at Q1 to Q4
+constexpr int csr_rows(int nb) { return nb <= 27 ? 8 : 4; }
 
 template <int NB, typename TX>
 __global__ void __launch_bounds__(256)

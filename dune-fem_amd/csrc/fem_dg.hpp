@@ -215,15 +215,16 @@ inline bool dg_is_modal(const DGArgs<T> &a)
 // w = A u.  `skip` (device flag, may be null): when *skip != 0 the launch
 // does nothing (device-driven solver loops).  `dot` (may be null): each
 // workgroup also writes its FP64 partial of <u, w> to dot[workgroup]
-// (dg_blocks(k, E) entries), for the solver's <q, A q>.
+// (Operator::dot_blocks() entries: dg_modal_blocks with kappa constant per
+// element, else dg_blocks), for the solver's <q, A q>.
 void dg_apply_f64(const DGPlan<double> &a, int k, const double *u, double *w, const int *skip, hipStream_t s,
                   double *dot = nullptr);
 void dg_apply_f32(const DGPlan<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s,
                   double *dot = nullptr);
 // BF16 MFMA contraction variant (FP32 data and accumulation)
 void dg_apply_bf16(const DGArgs<float> &a, int k, const float *u, float *w, const int *skip, hipStream_t s);
-// workgroups of the DG apply launch for order k-1 on n[0] x n[1] x n[2]
-// elements (its per-workgroup dot partials), and of the block-Jacobi launch
+// workgroups of the pointwise-kappa apply for order k-1 on n[0] x n[1] x n[2]
+// elements, and of block Jacobi on E elements (their dot partials)
 int64_t dg_blocks(int k, const int *n);
 int64_t dg_bj_blocks(int k, int64_t E);
 // operator diagonal

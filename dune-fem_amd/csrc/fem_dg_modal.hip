@@ -74,7 +74,10 @@ __device__ __forceinline__ void nbr_trace(const T *n, T &nv, T &nd)
 // r = line operator on the pencil v; k: kappa here, ks: behind the two faces
 // (k where there is no element), w0, w1: |F| / (2 h), on the boundary |F| / h,
 // nv, nd: the neighbours' traces (0 on the boundary); up1, ud1 (may be null):
-// the own traces at xi = 1
+// the own traces at xi = 1.  The order of the additions is one of several as
+// good (errors of 1e-15 and 1e-7), but not free: BiCGStab's step counts are chaotic
+// in rounding, and test_gpu_solver.py bounds one of them (207 with this order, 234
+// with another; 205 to 231 under changes of 1e-15 of the load)
 template <int K, int D, typename T>
 __device__ __forceinline__ void line(const ModalArgs<T> &a, T k, const T (&ks)[2], T w0, T w1, const T *v,
                                      const T (&nv)[2], const T (&nd)[2], T *r, T *up1 = nullptr, T *ud1 = nullptr)
@@ -162,8 +165,8 @@ __device__ __forceinline__ void modal_dot(double acc, double *__restrict__ dot)
 //   * the coefficients of the walk are read once, before it.
 // FP64 Q4 at 96^3: 1155 us by quadrature, 870 us with every lane loading its
 // six neighbour pencils from memory (7 loads of a vector through the vector
-// caches), 565 us so (3.1 TB/s of vectors read and written; 2.2 GB moved per
-// apply).  Q3 at 64^3: 131, 93, 80 us; Q2 at 96^3: 287, 183, 144 us.
+// caches), 550 us so (3.2 TB/s of vectors read and written; 2.2 GB moved per
+// apply).  Q3 at 64^3: 115, 79, 67 us; Q2 at 96^3: 287, 183, 144 us.
 template <int K, typename T, bool RES>
 __global__ void __launch_bounds__(MShape<K>::NT)
     k_dg_modal(const ModalArgs<T> a, const ModalTile mt, const T *__restrict__ u, T *__restrict__ w,

@@ -12,11 +12,12 @@
 //          dune/fem/solver/istlinverseoperators.hh:176-178).
 //
 // All scalars (alpha, beta, Hessenberg matrix, rotations) live in device
-// memory and are updated by the last block of each reduction kernel, so a
-// Krylov step needs no host round trip.  Every kernel reads a device `done`
-// flag and returns at once when the solve has finished; the host launches
-// steps in batches and reads the state back once per batch (CG) or once per
-// restart cycle (GMRES).
+// memory, so a Krylov step needs no host round trip.  CG and GMRES leave a
+// reduction's partials to the kernel that needs the sum, whose first workgroup
+// keeps the scalars; BiCGStab has the last block of a reduction update them.
+// Every kernel reads a device flag of the end and returns at once when the
+// solve has finished; the host launches steps in batches and reads the state
+// back once per batch (CG, BiCGStab) or once per restart cycle (GMRES).
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -951,7 +952,11 @@ static int run_krylov(Solver &S, int method, Operator *o, Precond *p, const T *b
     }
     // slices of the multi-dot and workgroups of the other square sums: about
     // 1024 and 256 elements each while vectors are short (a step at 69 k DoFs:
-    // 33.4 us with slices of 2048, 29.6 with 1024, 31.1 with 512).  Workgroups
+    // 33.4 us with slices of 2048, 29.6 with 1024, 31.1 with 512), and from
+    // 262 k DoFs on 256 slices, a workgroup per CU and group of vectors.
+    // GMRES(30) + Jacobi, FP64, a step at 69 k, 0.88 M, 4.1 M and 16.8 M DoFs: 28,
+    // 74, 321 and 1249 us (67, 117, 363 and 1283 us with 512 workgroups and a
+    // finish by the last one).  Workgroups
     // go to the 8 XCDs in turn, so a multiple of 8 slices puts a slice of all
     // basis vectors into one XCD's L2, for the multi-dot and the
     // orthogonalisation alike (8.8 and 8.4 us without, 7.6 and 7.4 us with)

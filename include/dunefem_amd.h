@@ -572,8 +572,8 @@ int fem_batch_apply(fem_batch *b, const fem_vec *u, fem_vec *w);
 int fem_batch_assemble_rhs(fem_batch *b, const double *fq, fem_vec *F);
 /* time every tile shape on the batch and keep the fastest; returns its shape */
 int fem_batch_autotune(fem_batch *b, int *tile_x, int *tile_y, float *ms_per_shape /* 5 entries or NULL */);
-/* x: initial guess in, solution out (FP64).  use_graph: replay one captured
- * inner step as a HIP graph */
+/* x: initial guess in, solution out (FP64).  use_graph: replay captured inner
+ * steps as a HIP graph */
 int fem_batch_solve(fem_batch *b, const fem_vec *rhs, fem_vec *x, double tol, double inner_tol, int inner_maxit,
                     int max_outer, int use_graph, fem_batch_info *info);
 /* per-instance results of the last solve: inner iterations and FP64 relative residual */
