@@ -654,7 +654,7 @@ __global__ void __launch_bounds__(256)
 // EPW elements each.  dot (may be null): the workgroup's <x, y> and <x, x>.
 // Reads and writes the vectors once and the eigen data (3 K^2 + 3 K values per
 // element) once, which is what bounds it.
-template <int K, typename T, bool ADD>
+template <int K, typename T, bool ADD, bool DOT>
 __global__ void __launch_bounds__(256)
     k_dg_block(int64_t E, const T *__restrict__ Qg, const T *__restrict__ lg, const T *__restrict__ x,
                const T *__restrict__ t, T *__restrict__ y, T omega, const int *__restrict__ skip,
@@ -675,7 +675,7 @@ __global__ void __launch_bounds__(256)
     T v[K], xv[K];
 #pragma unroll
     for (int m = 0; m < K; ++m) xv[m] = v[m] = xe[m * K2];
-    if (t) {
+    if constexpr (ADD) {
         const T *te = t + e * K3 + lane;
 #pragma unroll
         for (int m = 0; m < K; ++m) v[m] -= te[m * K2];
@@ -695,11 +695,13 @@ __global__ void __launch_bounds__(256)
         for (int m = 0; m < K; ++m) {
             const T r = ADD ? fma(omega, v[m], ye[m * K2]) : omega * v[m];
             ye[m * K2] = r;
-            a1 += (double)xv[m] * (double)r;
-            a2 += (double)xv[m] * (double)xv[m];
+            if constexpr (DOT) {
+                a1 += (double)xv[m] * (double)r;
+                a2 += (double)xv[m] * (double)xv[m];
+            }
         }
     }
-    if (dot) {
+    if constexpr (DOT) {
         modal_dot<256>(a1, dot);
         __syncthreads();
         modal_dot<256>(a2, dot + gridDim.x);
@@ -800,10 +802,12 @@ void launch_block(int64_t E, const T *Q, const T *lam, const T *x, const T *t, T
                   const int *skip, hipStream_t s, double *dot)
 {
     const unsigned nb = (unsigned)dg_bj_blocks(K, E);
-    if (add)
-        hipLaunchKernelGGL((k_dg_block<K, T, true>), dim3(nb), dim3(256), 0, s, E, Q, lam, x, t, y, omega, skip, dot);
-    else
-        hipLaunchKernelGGL((k_dg_block<K, T, false>), dim3(nb), dim3(256), 0, s, E, Q, lam, x, t, y, omega, skip, dot);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, s, E, Q, lam, x, t, y, omega, skip, dot);
+    };
+    if (add) go(k_dg_block<K, T, true, false>);
+    else if (dot) go(k_dg_block<K, T, false, true>);
+    else go(k_dg_block<K, T, false, false>);
 }
 
 }  // namespace
