@@ -180,6 +180,12 @@ __global__ void k_csr_q2_extract(Q2Dims d, const T *__restrict__ y, const int64_
 // 88 us.
 // rows of a wavefront: a lane has 8, 24, 28 and 56 values in flight at Q1 to Q4
 constexpr int csr_rows(int nb) { return nb <= 27 ? 8 : 4; }
+// Small matrices are bound by the chain of loads of one wavefront and by the
+// wavefronts in flight, not by the bytes: there a wavefront per row is faster.  Q1
+// 12^3 (0.72 M nonzeros) 3.95 us by rows and 4.25 us so, 20^3 (3.4 M) 15.6 and 10.5; Q2
+// 6 x 6 x 5 (0.78 M) 3.4 and 4.1, 8^3 (2.3 M) 7.1 and 5.3; Q3 2^3 (0.13 M) 3.1 and 3.7,
+// 4 x 4 x 5 (1.8 M) 5.5 and 4.5; Q4 2^3 (0.5 M) 3.4 and 4.8, 3^3 (2.1 M) 7.6 and 5.2.
+constexpr int64_t CSR_DG_NNZ = 1000000;
 
 template <int NB, typename TX>
 __global__ void __launch_bounds__(256)
@@ -367,7 +373,7 @@ void CSR::apply(const Vec &x, Vec &y) const
         using TX = decltype(t);
         const TX *xp = (const TX *)x.data;
         TX *yp = (TX *)y.data;
-        if (dg_k) {
+        if (dg_k && nnz >= CSR_DG_NNZ) {
             const int nb = dg_k * dg_k * dg_k, sr = csr_rows(nb);
             const DGDims d{ { dg_n[0], dg_n[1], dg_n[2] }, nb };
             auto go = [&](auto kernel) {

@@ -1,5 +1,6 @@
-"""The SpMV of a DG matrix reads no column indices: against the downloaded CSR
-arrays, on meshes whose elements have from none to all six neighbours.
+"""The SpMV of a DG matrix, by rows below a million nonzeros and by elements without
+column indices above: against the downloaded CSR arrays, on meshes whose elements
+have from none to all six neighbours.
 
 Bar: a row sums at most 875 products, so both sides differ by at most 2 * 875 eps =
 4e-13 of sum |a| |x|; FP32 vectors add the rounding of the result, 6e-8 of |y|."""
@@ -30,3 +31,14 @@ def test_dg_spmv_matches_its_arrays(ctx, n, p):
         err = np.abs(Y.download() - ref)
         print("csr", n, p, prec, (err / bar).max(), flush=True)
         assert (err <= bar).all()
+
+
+@pytest.mark.parametrize("p,n", [
+    # a million nonzeros and more, from where on the element kernel is taken: rows of
+    # elements with one, two, three and up to six neighbours
+    (1, (1, 1, 5500)), (1, (70, 60, 1)), (1, (13, 15, 16)),
+    (2, (480, 1, 1)), (2, (2, 3, 70)), (2, (7, 6, 8)),
+    (3, (1, 90, 1)), (3, (4, 3, 5)), (4, (1, 1, 24)), (4, (3, 3, 2)),
+])
+def test_large_dg_spmv_matches_its_arrays(ctx, p, n):
+    test_dg_spmv_matches_its_arrays(ctx, n, p)
